@@ -1737,7 +1737,7 @@ __global__ __launch_bounds__(kFinWaves * kWave) void gqa_bounds_kernel(
   __syncthreads();
   if (wave == 0) {
     WaveList B;
-    block_merge<kFinWaves>(s_lists, k, B);
+    block_merge(s_lists, kFinWaves, k, B);
     if (lane < k) block_out[(static_cast<size_t>(qb) * nsblk + sblk) * k + lane] = wl_entry(B);
   }
 }
@@ -1844,7 +1844,7 @@ __global__ __launch_bounds__(kFinWaves * kWave) void gqa_bounds_wide_kernel(
   __syncthreads();
   if (wave == 0) {
     WaveList B;
-    block_merge<kFinWaves>(s_lists, k, B);
+    block_merge(s_lists, kFinWaves, k, B);
     if (lane < k) block_out[(static_cast<size_t>(qb) * nsblk + sblk) * k + lane] = wl_entry(B);
   }
 }
@@ -2052,7 +2052,7 @@ __global__ __launch_bounds__(kCandWaves * kWave) void gqa_cands_kernel(
   __syncthreads();
   if (wave == 0) {
     WaveList B;
-    block_merge<kCandWaves>(s_lists, k, B);
+    block_merge(s_lists, kCandWaves, k, B);
     const float t = lane_f32(B.s, k - 1);
     if (lane == 0) s_tau = isfinite(t) ? t : -INFINITY;
   }

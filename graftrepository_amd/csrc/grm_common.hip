@@ -121,6 +121,9 @@ int wait_flags(const MappedBuf& buf, unsigned seq, size_t n, hipEvent_t ev) {
 int wait_tagged(const Cand* entries, size_t n, unsigned seq, hipEvent_t ev) {
   const volatile uint32_t* tags = reinterpret_cast<const volatile uint32_t*>(entries);
   const uint32_t tag = route_tag(seq);
+  // The device wrote every line, so each read misses the host's caches:
+  // ask for the lines ahead of the reads.
+  for (size_t i = 0; i < n; i += 4) __builtin_prefetch(entries + i);
   // the slot field is the second word of each 16-byte entry
   for (size_t i = 0; i < n; ++i) {
     for (uint64_t spin = 1; tags[4 * i + 1] != tag; ++spin) {
@@ -244,7 +247,7 @@ __global__ __launch_bounds__(kMergeWaves * kWave) void topk_merge_kernel(
   __syncthreads();
   if (wave == 0) {
     WaveList B;
-    block_merge<kMergeWaves>(s_lists, k, B);
+    block_merge(s_lists, kMergeWaves, k, B);
     if (lane < k) out[static_cast<size_t>(blockIdx.x) * k + lane] = wl_entry(B);
     if (lane == 0 && flags) flags[blockIdx.x] = 0u;
   }

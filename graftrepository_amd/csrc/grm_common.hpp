@@ -198,16 +198,16 @@ __device__ inline Cand wl_entry(const WaveList& L) {
   return c;
 }
 
-// Merge the per-wave lists of a block (written to `lists[wave][0..k)`) into
-// wave 0's list.  Caller synchronises the block before and reads the result
-// from wave 0 after.
-template <int NW, int CAP>
-__device__ inline void block_merge(Cand (*lists)[CAP], int k, WaveList& out) {
+// Merge the per-wave lists of a block of nw waves (written to
+// `lists[wave][0..k)`) into wave 0's list.  Caller synchronises the block
+// before and reads the result from wave 0 after.
+template <int CAP>
+__device__ inline void block_merge(Cand (*lists)[CAP], int nw, int k, WaveList& out) {
   const int lane = __lane_id();
   wl_init(out);
-  for (int base = 0; base < NW * k; base += kWave) {
+  for (int base = 0; base < nw * k; base += kWave) {
     const int i = base + lane;
-    const bool v = i < NW * k;
+    const bool v = i < nw * k;
     Cand c;
     c.score = -INFINITY;
     c.slot = kNoSlot;
@@ -273,26 +273,27 @@ __device__ inline void store_entry(Cand* __restrict__ dst, Cand c, uint32_t tag)
   *reinterpret_cast<u32x4_t*>(dst) = v;
 }
 
-// Block epilogue shared by the route kernels: merge the block's wave lists
-// in LDS and write the block's k best entries to block_out[blockIdx.x*k ..)
-// (tagged with `tag` unless it is kNoSlot, store_entry).  Must be reached
-// by every thread of the block.  Device-side lists are merged by
-// topk_merge_kernel, launched next on the same stream; the kernel boundary
-// orders the writes, so no device-scope fence (an L2 write-back on gfx950)
-// is paid per block.
-template <int NW, int CAP>
-__device__ inline void block_topk_write(WaveList& L, int k,
+// Block epilogue of a route kernel of nw waves: merge the block's wave
+// lists in LDS (a single wave's list needs no merge) and write the block's
+// k best entries to block_out[blockIdx.x*k ..) (tagged with `tag` unless it
+// is kNoSlot, store_entry).  Must be reached by every thread of the block.
+// Device-side lists are merged by topk_merge_kernel, launched next on the
+// same stream; the kernel boundary orders the writes, so no device-scope
+// fence (an L2 write-back on gfx950) is paid per block.
+template <int CAP>
+__device__ inline void block_topk_write(WaveList& L, int k, int nw,
                                         Cand (*s_lists)[CAP],
                                         Cand* __restrict__ block_out,
                                         uint32_t tag = kNoSlot) {
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
-  if (lane < CAP) s_lists[wave][lane] = wl_entry(L);
-  __syncthreads();
-  if (wave == 0) {
-    WaveList B;
-    block_merge<NW>(s_lists, k, B);
-    if (lane < k) store_entry(block_out + static_cast<size_t>(blockIdx.x) * k + lane, wl_entry(B), tag);
+  if (nw > 1) {
+    if (lane < CAP) s_lists[wave][lane] = wl_entry(L);
+    __syncthreads();
+    if (wave == 0) block_merge(s_lists, nw, k, L);
+  }
+  if (wave == 0 && lane < k) {
+    store_entry(block_out + static_cast<size_t>(blockIdx.x) * k + lane, wl_entry(L), tag);
   }
 }
 

@@ -47,8 +47,8 @@ namespace mla {
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kMaxDim = 4096;
-constexpr int kRouteWaves = 4;           // waves per block, plain kernel
-constexpr int kPipeWaves = 16;           // waves per block, pipelined kernel
+constexpr int kRouteWaves = 16;          // most waves per block of the single-query kernel
+constexpr int kDeepWaves = 8;            // most waves per block of its deep form
 constexpr uint32_t kStageRows = 1u << 16;  // rows per attach staging batch
 
 // ------------------------------------------------------------------ kernels
@@ -75,209 +75,196 @@ __device__ inline double chunk_dot(u32x4 v, const double* __restrict__ q,
   return acc;
 }
 
-// Dot product of this lane's row with the query, d ascending.
+// Stage the query as doubles in LDS (zero beyond dim).  Up to 8 loads per
+// thread are in flight at once, unconditional ones: a block may be a single
+// wave, which would otherwise wait for memory once per load.
+template <typename T>
+__device__ inline void stage_values(double* qd, const T* __restrict__ query, uint32_t dim,
+                                    uint32_t dim_pad) {
+  constexpr int kAhead = 8;
+  for (uint32_t d0 = threadIdx.x; d0 < dim_pad; d0 += kAhead * blockDim.x) {
+    T v[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) v[j] = query[min(d0 + j * blockDim.x, dim - 1)];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const uint32_t d = d0 + j * blockDim.x;
+      float f;
+      if constexpr (sizeof(T) == 2) {
+        f = bf16_to_f32(v[j]);
+      } else {
+        f = v[j];
+      }
+      if (d < dim_pad) qd[d] = d < dim ? static_cast<double>(f) : 0.0;
+    }
+  }
+}
+__device__ inline void stage_query(double* qd, const void* __restrict__ query,
+                                   int query_dtype, uint32_t dim,
+                                   uint32_t dim_pad) {
+  if (query_dtype == kBF16) {
+    stage_values(qd, static_cast<const uint16_t*>(query), dim, dim_pad);
+  } else {
+    stage_values(qd, static_cast<const float*>(query), dim, dim_pad);
+  }
+}
+
+// q[0, N) in order through `use(value, index)`, read from LDS kAhead values
+// ahead of their use: a lone wave on its SIMD would otherwise wait for LDS
+// (over 100 cycles) at every chunk of its serial fp64 chain.
+template <int N, int kAhead, typename F>
+__device__ __forceinline__ void stream_lds(const double* __restrict__ q, F use) {
+  static_assert(N % kAhead == 0, "whole stages");
+  double cur[kAhead], nxt[kAhead];
+#pragma unroll
+  for (int e = 0; e < kAhead; ++e) cur[e] = q[e];
+#pragma unroll
+  for (int s = 0; s < N / kAhead; ++s) {
+    if (s + 1 < N / kAhead) {
+#pragma unroll
+      for (int e = 0; e < kAhead; ++e) nxt[e] = q[(s + 1) * kAhead + e];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int e = 0; e < kAhead; ++e) use(cur[e], s * kAhead + e);
+#pragma unroll
+    for (int e = 0; e < kAhead; ++e) cur[e] = nxt[e];
+  }
+}
+
+// Value i of a chunk (fp32 or bf16) as a double.
 template <int DT>
-__device__ inline double tile_dot(const u32x4* __restrict__ p, uint32_t chunks,
-                                  size_t plane, const double* __restrict__ qd) {
-  constexpr int EPC = DT == kF32 ? 4 : 8;
-  constexpr uint32_t kBatch = 8;
+__device__ __forceinline__ double chunk_value(u32x4 v, int i) {
+  const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
+  if constexpr (DT == kF32) {
+    return static_cast<double>(__uint_as_float(w4[i]));
+  } else {
+    const uint32_t w = w4[i >> 1];
+    return static_cast<double>(__uint_as_float((i & 1) ? (w & 0xffff0000u) : (w << 16)));
+  }
+}
+
+// The law's query norm from the staged query (zeros past dim add nothing):
+// one serial fp64 chain over d (cpp/grm_runtime.cpp:4310-4314).  n is a
+// multiple of 4.
+__device__ inline double staged_norm(const double* __restrict__ qd, uint32_t n) {
   double acc = 0.0;
-  uint32_t c = 0;
-  for (; c + kBatch <= chunks; c += kBatch) {
-    u32x4 v[kBatch];
-#pragma unroll
-    for (uint32_t j = 0; j < kBatch; ++j) {
-      v[j] = __builtin_nontemporal_load(p + static_cast<size_t>(c + j) * plane);
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < kBatch; ++j) {
-      acc = chunk_dot<DT>(v[j], qd + (c + j) * EPC, acc);
-    }
-  }
-  for (; c < chunks; ++c) {
-    acc = chunk_dot<DT>(__builtin_nontemporal_load(p + static_cast<size_t>(c) * plane),
-                        qd + c * EPC, acc);
-  }
-  return acc;
+  uint32_t d = 0;
+  for (; d + 64 <= n; d += 64) stream_lds<64, 16>(qd + d, [&](double q, int) { acc = fma(q, q, acc); });
+  for (; d < n; d += 4) stream_lds<4, 4>(qd + d, [&](double q, int) { acc = fma(q, q, acc); });
+  return sqrt(acc);
 }
 
 // One query against every slot; each block writes its k best entries to
 // block_out[blockIdx.x*k ..), then (with done) seq to done[blockIdx.x];
 // with stamps a timed route's start and end ticks (RouteStamps).
-template <int DT, int NW>
-__global__ __launch_bounds__(NW * kWave) void mla_route_kernel(
+//
+// Waves walk 64-slot tiles, a lane per slot, d ascending (the law's order),
+// as a software pipeline: while a batch of B chunks is folded into the fp64
+// dot product the next batch (of the same tile or the wave's next tile) is
+// in flight, and the row norm of the next tile is fetched ahead of its
+// data.  A row whose chunks are no whole number of batches reads its last
+// chunk again in place of the missing ones; the staged query is zero there,
+// so they add exact zeros (a stored row is finite).  Wave w of block b
+// starts at tile b * waves + w, or with `spread` at w * blocks + b
+// (single_geom), and steps by blocks * waves.
+//
+// The query's norm (a serial sum over d) is formed by one wave while every
+// wave's first batch is on its way from memory.
+//
+// Two forms, chosen by the bank's size (single_geom):
+//  * kMaxNW = 16, B = 6..9: four waves per SIMD, 9 KiB in flight per wave --
+//    bound by HBM (1M x 288 fp32: 170 us = 6.8 TB/s).
+//  * kMaxNW = 8, B = 12..18 (deep): banks of at most 8 tiles per CU, a wave
+//    per tile on every CU.  Bound by latency: one round trip to memory and
+//    the fp64 chain of one row.  10k x 288 fp32 on the device: 8.3 us,
+//    against 24.6 us for 16-wave blocks on 10 CUs; with two, four or eight
+//    waves per block at that size 9.9, 11.4 and 15.5 us.  100k x 288: 20.9
+//    against 31.6 us.
+template <int DT, int B, int kMaxNW>
+__global__ __launch_bounds__(kMaxNW * kWave) void mla_route_kernel(
     const u32x4* __restrict__ tiles, const float* __restrict__ norms,
     const uint64_t* __restrict__ ids, uint32_t num_tiles, uint32_t chunks,
-    size_t plane, uint32_t dim, uint32_t dim_pad,
-    const void* __restrict__ query, int query_dtype, int k,
-    Cand* __restrict__ block_out, unsigned* __restrict__ done, unsigned seq, RouteStamps stamps) {
+    size_t plane, uint32_t dim, const void* __restrict__ query, int query_dtype, int k,
+    Cand* __restrict__ block_out, unsigned* __restrict__ done, unsigned seq, RouteStamps stamps,
+    int spread) {
   route_start_stamp(stamps, seq);
-  extern __shared__ double qd[];
+  constexpr uint32_t EPC = DT == kF32 ? 4 : 8;
+  extern __shared__ double qd[];  // nb * B * EPC values
   __shared__ double s_qnorm;
-  __shared__ Cand s_lists[NW][kMaxTopK];
-  const int tid = threadIdx.x;
-  const int lane = tid & (kWave - 1);
-  const int wave = tid / kWave;
-
-  for (uint32_t d = tid; d < dim_pad; d += NW * kWave) {
-    double v = 0.0;
-    if (d < dim) {
-      v = query_dtype == kBF16
-              ? static_cast<double>(bf16_to_f32(static_cast<const uint16_t*>(query)[d]))
-              : static_cast<double>(static_cast<const float*>(query)[d]);
-    }
-    qd[d] = v;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    double acc = 0.0;  // cpp/grm_runtime.cpp:4310-4314, sequential
-    for (uint32_t d = 0; d < dim; ++d) acc = fma(qd[d], qd[d], acc);
-    s_qnorm = sqrt(acc);
-  }
-  __syncthreads();
-  const double qnorm = s_qnorm;
-
-  WaveList L;
-  wl_init(L);
-  for (uint32_t t = blockIdx.x * NW + wave; t < num_tiles; t += gridDim.x * NW) {
-    const double dot = tile_dot<DT>(
-        tiles + static_cast<size_t>(t) * kWave + lane, chunks, plane, qd);
-    const uint32_t slot = t * kWave + lane;
-    const float nrm = norms[slot];  // NaN marks an empty or evicted slot
-    const double den = qnorm * static_cast<double>(nrm) + 1.0e-8;
-    const float s = static_cast<float>(dot / den);
-    const bool need = isfinite(s) && s >= L.th_s;
-    uint64_t id = kNoId;
-    if (need) id = ids[slot];
-    wl_consume(L, k, s, id, slot, need);
-  }
-
-  block_topk_write<NW>(L, k, s_lists, block_out, done ? route_tag(seq) : kNoSlot);
-  block_done_flag(done, seq, stamps.end);
-}
-
-// Stage the query as doubles in LDS (zero beyond dim).
-__device__ inline void stage_query(double* qd, const void* __restrict__ query,
-                                   int query_dtype, uint32_t dim,
-                                   uint32_t dim_pad) {
-  for (uint32_t d = threadIdx.x; d < dim_pad; d += blockDim.x) {
-    double v = 0.0;
-    if (d < dim) {
-      v = query_dtype == kBF16
-              ? static_cast<double>(bf16_to_f32(static_cast<const uint16_t*>(query)[d]))
-              : static_cast<double>(static_cast<const float*>(query)[d]);
-    }
-    qd[d] = v;
-  }
-}
-
-template <int DT, int B>
-__device__ inline double batch_dot(const u32x4 (&v)[B],
-                                   const double* __restrict__ q, double acc) {
-  constexpr int EPC = DT == kF32 ? 4 : 8;
+  __shared__ Cand s_lists[kMaxNW][kMaxTopK];
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t nw = blockDim.x / kWave;
+  const uint32_t stride = gridDim.x * nw;
+  const uint32_t nb = (chunks + B - 1) / B;
+  // Beyond-the-end prefetches read tile 0 (never folded).
+  auto load = [&](u32x4 (&v)[B], uint32_t t, uint32_t b) {
+    const u32x4* base = tiles + (t < num_tiles ? static_cast<size_t>(t) * kWave : 0);
 #pragma unroll
-  for (int j = 0; j < B; ++j) acc = chunk_dot<DT>(v[j], q + j * EPC, acc);
-  return acc;
-}
-
-// Software-pipelined variant for rows of a whole number of B-chunk batches:
-// while a batch is folded into the fp64 dot product the next batch (of the
-// same tile or the wave's next tile) is already in flight, and the row norm
-// of the next tile is fetched ahead of its data.  Arithmetic and order are
-// those of mla_route_kernel.
-template <int DT, int NW, int B>
-__global__ __launch_bounds__(NW * kWave) void mla_route_pipe_kernel(
-    const u32x4* __restrict__ tiles, const float* __restrict__ norms,
-    const uint64_t* __restrict__ ids, uint32_t num_tiles, uint32_t chunks,
-    size_t plane, uint32_t dim, uint32_t dim_pad,
-    const void* __restrict__ query, int query_dtype, int k,
-    Cand* __restrict__ block_out, unsigned* __restrict__ done, unsigned seq, RouteStamps stamps) {
-  route_start_stamp(stamps, seq);
-  constexpr int EPC = DT == kF32 ? 4 : 8;
-  extern __shared__ double qd[];
-  __shared__ double s_qnorm;
-  __shared__ Cand s_lists[NW][kMaxTopK];
-  const int tid = threadIdx.x;
-  const int lane = tid & (kWave - 1);
-  const int wave = tid / kWave;
-  const uint32_t stride = gridDim.x * NW;
-  const uint32_t nb = chunks / B;
-  // Beyond-the-end prefetches read tile 0's first batch (cache resident).
-  auto batch_ptr = [&](uint32_t t, uint32_t b) {
-    return t < num_tiles
-               ? tiles + static_cast<size_t>(b) * B * plane + static_cast<size_t>(t) * kWave + lane
-               : tiles + lane;
-  };
-  auto load = [&](u32x4 (&v)[B], const u32x4* p) {
-#pragma unroll
-    for (int j = 0; j < B; ++j) v[j] = __builtin_nontemporal_load(p + j * plane);
+    for (uint32_t j = 0; j < B; ++j) {
+      const uint32_t c = min(b * B + j, chunks - 1);
+      v[j] = __builtin_nontemporal_load(base + static_cast<size_t>(c) * plane + lane);
+    }
   };
 
-  uint32_t t = blockIdx.x * NW + wave;
+  stage_query(qd, query, query_dtype, dim, nb * B * EPC);
+  constexpr bool kDeep = kMaxNW <= kDeepWaves;
+  uint32_t t = spread ? wave * gridDim.x + blockIdx.x : blockIdx.x * nw + wave;
   uint32_t b = 0;
   u32x4 bufA[B], bufB[B];
   float nrm_cur = norms[(t < num_tiles ? t : 0) * kWave + lane];
-  load(bufA, batch_ptr(t, 0));
-
-  stage_query(qd, query, query_dtype, dim, dim_pad);
+  load(bufA, t, 0);
   __syncthreads();
-  if (tid == 0) {
-    double acc = 0.0;  // cpp/grm_runtime.cpp:4310-4314, sequential
-    for (uint32_t d = 0; d < dim; ++d) acc = fma(qd[d], qd[d], acc);
-    s_qnorm = sqrt(acc);
-  }
+  if (threadIdx.x == 0) s_qnorm = staged_norm(qd, nb * B * EPC);
   __syncthreads();
   const double qnorm = s_qnorm;
 
   WaveList L;
   wl_init(L);
-  auto finish = [&](uint32_t tt, double dot, float nrm) {
-    const uint32_t slot = tt * kWave + lane;
-    const double den = qnorm * static_cast<double>(nrm) + 1.0e-8;
-    const float s = static_cast<float>(dot / den);
-    const bool need = isfinite(s) && s >= L.th_s;
-    uint64_t id = kNoId;
-    if (need) id = ids[slot];
-    wl_consume(L, k, s, id, slot, need);
-  };
   double acc = 0.0;
   float nrm_next = 0.0f;
-  while (t < num_tiles) {
+  // Fold `now` while the next batch loads into `later`; false at the end of
+  // the wave's tiles.
+  auto step = [&](u32x4 (&now)[B], u32x4 (&later)[B]) -> bool {
     uint32_t tn = t, bn = b + 1;
     if (bn == nb) {
       tn = t + stride;
       bn = 0;
       nrm_next = norms[(tn < num_tiles ? tn : 0) * kWave + lane];
     }
-    load(bufB, batch_ptr(tn, bn));
-    acc = batch_dot<DT, B>(bufA, qd + b * B * EPC, acc);
+    load(later, tn, bn);
+    const double* q = qd + b * B * EPC;
+    if constexpr (kDeep) {
+      // fma(r, q, acc) is exact as in chunk_dot
+      stream_lds<B * EPC, (B * EPC) % 16 == 0 ? 16 : 12>(q, [&](double qv, int i) {
+        acc = fma(chunk_value<DT>(now[i / EPC], i % EPC), qv, acc);
+      });
+    } else {
+#pragma unroll
+      for (uint32_t j = 0; j < B; ++j) acc = chunk_dot<DT>(now[j], q + j * EPC, acc);
+    }
     if (bn == 0) {
-      finish(t, acc, nrm_cur);
+      const uint32_t slot = t * kWave + lane;
+      // NaN norm marks an empty or evicted slot
+      const double den = qnorm * static_cast<double>(nrm_cur) + 1.0e-8;
+      const float s = static_cast<float>(acc / den);
+      const bool need = isfinite(s) && s >= L.th_s;
+      uint64_t id = kNoId;
+      if (need) id = ids[slot];
+      wl_consume(L, k, s, id, slot, need);
       acc = 0.0;
       nrm_cur = nrm_next;
     }
     t = tn;
     b = bn;
-    if (t >= num_tiles) break;
-
-    tn = t;
-    bn = b + 1;
-    if (bn == nb) {
-      tn = t + stride;
-      bn = 0;
-      nrm_next = norms[(tn < num_tiles ? tn : 0) * kWave + lane];
+    return t < num_tiles;
+  };
+  if (t < num_tiles) {
+    while (step(bufA, bufB) && step(bufB, bufA)) {
     }
-    load(bufA, batch_ptr(tn, bn));
-    acc = batch_dot<DT, B>(bufB, qd + b * B * EPC, acc);
-    if (bn == 0) {
-      finish(t, acc, nrm_cur);
-      acc = 0.0;
-      nrm_cur = nrm_next;
-    }
-    t = tn;
-    b = bn;
   }
-  block_topk_write<NW>(L, k, s_lists, block_out, done ? route_tag(seq) : kNoSlot);
+  block_topk_write(L, k, static_cast<int>(nw), s_lists, block_out, done ? route_tag(seq) : kNoSlot);
   block_done_flag(done, seq, stamps.end);
 }
 
@@ -450,9 +437,8 @@ struct MlaDeviceArena {
   uint64_t single_queries = 0;   // queries through the single-query kernel
   std::vector<hipEvent_t> screen_ev;  // begin/end pairs around timed screens
   float screen_ms = 0.0f;        // screen-kernel time of the last batched route
-  bool pipeline = true;     // software-pipelined kernel when rows allow it
   uint32_t cus = 256;       // compute units of the device
-  uint32_t max_blocks = 0;  // plain-kernel grid cap (4 blocks per CU)
+  uint32_t max_blocks = 0;  // single-query grid cap (GRM_HIP_MLA_BLOCKS; a block per CU)
 };
 
 // Per-block top-k lists of the allocation-free route (see route_noalloc).
@@ -599,13 +585,12 @@ int create_arena(const void* rows, int dtype, uint64_t nodes, int dim,
       cus = 256;
     }
     a->cus = static_cast<uint32_t>(cus);
-    a->max_blocks = static_cast<uint32_t>(cus) * 4;
+    a->max_blocks = static_cast<uint32_t>(cus);
   }
   if (const char* env = getenv("GRM_HIP_MLA_BLOCKS")) {
     const long v = strtol(env, nullptr, 10);
     if (v >= 1 && v <= 65536) a->max_blocks = static_cast<uint32_t>(v);
   }
-  if (const char* env = getenv("GRM_HIP_MLA_PIPELINE")) a->pipeline = env[0] != '0';
   if (const char* env = getenv("GRM_HIP_BATCH_RING")) a->ring = env[0] != '0';
   if (const char* env = getenv("GRM_HIP_QUERY_COPY")) a->query_dma = strcmp(env, "dma") == 0;
   a->ticks_per_ms = grm::wall_ticks_per_ms(a->device);
@@ -702,26 +687,36 @@ int create_arena(const void* rows, int dtype, uint64_t nodes, int dim,
 // Launch geometry of the single-query route kernel.
 struct SingleGeom {
   uint32_t num_tiles = 0, blocks = 0, nw = 0;
-  int batch = 0;  // chunks per pipelined load batch (0: plain kernel)
+  int batch = 0;      // chunks per pipelined load batch
+  bool deep = false;  // the deep form (mla_route_kernel)
+  int spread = 0;     // tiles dealt out block by block rather than in runs per block
 };
 
 SingleGeom single_geom(const MlaDeviceArena* a) {
   SingleGeom g;
   g.num_tiles = static_cast<uint32_t>((a->high_water + grm::kWave - 1) / grm::kWave);
-  // The pipelined kernel runs one 16-wave block per CU (4 waves per SIMD);
-  // the plain kernel (rows that do not split into whole batches) 4-wave
-  // blocks, 4 per CU.
-  if (a->pipeline) {
-    for (int b : {9, 8, 6}) {
-      if (a->chunks % b == 0) {
-        g.batch = b;
-        break;
-      }
+  const uint32_t cap = std::min(a->cus, a->max_blocks);
+  // As many waves per block as spread the tiles over every CU, so banks of
+  // few tiles run one wave on each of many CUs.
+  const uint32_t per_cu = std::max<uint32_t>(1, (g.num_tiles + cap - 1) / cap);
+  g.deep = per_cu <= static_cast<uint32_t>(grm::mla::kDeepWaves);
+  g.nw = std::min<uint32_t>(per_cu, g.deep ? grm::mla::kDeepWaves : grm::mla::kRouteWaves);
+  g.blocks = std::max<uint32_t>(1, std::min((g.num_tiles + g.nw - 1) / g.nw, cap));
+  // Tiles per wave below 4 (or one): dealt out one per block in turn, since a
+  // last round taken by whole blocks would leave CUs with nothing to do
+  // (300k x 288 fp32: 55.7 us against 75.2).  From 4 rounds on a block's
+  // waves take neighbouring tiles, which streams better (1M x 288: 170 us
+  // against 173).
+  g.spread = static_cast<uint64_t>(g.num_tiles) <= 3ull * g.blocks * g.nw ? 1 : 0;
+  // the batch that pads the row's chunks least, the longest of those
+  uint32_t best = ~0u;
+  for (int b : {g.deep ? 18 : 9, g.deep ? 16 : 8, g.deep ? 12 : 6}) {
+    const uint32_t padded = (a->chunks + b - 1) / b * b;
+    if (padded < best) {
+      best = padded;
+      g.batch = b;
     }
   }
-  g.nw = g.batch ? grm::mla::kPipeWaves : grm::mla::kRouteWaves;
-  const uint32_t cap = g.batch ? std::min(a->cus, a->max_blocks) : a->max_blocks;
-  g.blocks = std::max<uint32_t>(1, std::min((g.num_tiles + g.nw - 1) / g.nw, cap));
   return g;
 }
 
@@ -731,30 +726,30 @@ SingleGeom single_geom(const MlaDeviceArena* a) {
 int launch_single(MlaDeviceArena* a, const SingleGeom& g, const void* q, int q_dtype, int topk,
                   Cand* bout, unsigned* done = nullptr,
                   const grm::RouteStamps& st = grm::RouteStamps{nullptr, nullptr}) {
-  const size_t lds = static_cast<size_t>(a->dim_pad) * sizeof(double);
+  const size_t padded = (a->chunks + g.batch - 1) / g.batch * g.batch;
+  const size_t lds = padded * a->epc * sizeof(double);
   const dim3 grid(g.blocks), block(g.nw * grm::kWave);
   const float* nrm = a->route_norms ? a->route_norms : a->d_norms;
-#define GRM_MLA_ARGS                                                                  \
-  a->d_tiles, nrm, a->d_ids, g.num_tiles, a->chunks, a->capacity, a->dim, a->dim_pad, q, \
-      q_dtype, topk, bout, done, a->route_seq, st
-  constexpr int PW = grm::mla::kPipeWaves;
-  constexpr int RW = grm::mla::kRouteWaves;
-  if (a->dtype == kF32) {
-    switch (g.batch) {
-      case 9: grm::mla::mla_route_pipe_kernel<kF32, PW, 9><<<grid, block, lds, a->stream>>>(GRM_MLA_ARGS); break;
-      case 8: grm::mla::mla_route_pipe_kernel<kF32, PW, 8><<<grid, block, lds, a->stream>>>(GRM_MLA_ARGS); break;
-      case 6: grm::mla::mla_route_pipe_kernel<kF32, PW, 6><<<grid, block, lds, a->stream>>>(GRM_MLA_ARGS); break;
-      default: grm::mla::mla_route_kernel<kF32, RW><<<grid, block, lds, a->stream>>>(GRM_MLA_ARGS); break;
-    }
-  } else {
-    switch (g.batch) {
-      case 9: grm::mla::mla_route_pipe_kernel<kBF16, PW, 9><<<grid, block, lds, a->stream>>>(GRM_MLA_ARGS); break;
-      case 8: grm::mla::mla_route_pipe_kernel<kBF16, PW, 8><<<grid, block, lds, a->stream>>>(GRM_MLA_ARGS); break;
-      case 6: grm::mla::mla_route_pipe_kernel<kBF16, PW, 6><<<grid, block, lds, a->stream>>>(GRM_MLA_ARGS); break;
-      default: grm::mla::mla_route_kernel<kBF16, RW><<<grid, block, lds, a->stream>>>(GRM_MLA_ARGS); break;
-    }
+#define GRM_MLA_ROUTE(DT, B, NW)                                                               \
+  grm::mla::mla_route_kernel<DT, B, NW><<<grid, block, lds, a->stream>>>(                      \
+      a->d_tiles, nrm, a->d_ids, g.num_tiles, a->chunks, a->capacity, a->dim, q, q_dtype, topk, \
+      bout, done, a->route_seq, st, g.spread)
+#define GRM_MLA_BATCH(DT)                                              \
+  switch (g.batch) {                                                   \
+    case 18: GRM_MLA_ROUTE(DT, 18, grm::mla::kDeepWaves); break;       \
+    case 16: GRM_MLA_ROUTE(DT, 16, grm::mla::kDeepWaves); break;       \
+    case 12: GRM_MLA_ROUTE(DT, 12, grm::mla::kDeepWaves); break;       \
+    case 9: GRM_MLA_ROUTE(DT, 9, grm::mla::kRouteWaves); break;        \
+    case 8: GRM_MLA_ROUTE(DT, 8, grm::mla::kRouteWaves); break;        \
+    default: GRM_MLA_ROUTE(DT, 6, grm::mla::kRouteWaves); break;       \
   }
-#undef GRM_MLA_ARGS
+  if (a->dtype == kF32) {
+    GRM_MLA_BATCH(kF32);
+  } else {
+    GRM_MLA_BATCH(kBF16);
+  }
+#undef GRM_MLA_BATCH
+#undef GRM_MLA_ROUTE
   GRM_HIP_CHECK(hipGetLastError());
   return 0;
 }
@@ -1355,7 +1350,7 @@ __global__ __launch_bounds__(grm::kMergeWaves * grm::kWave) void mla_merge_out_k
   __syncthreads();
   if (wave == 0) {
     grm::WaveList B;
-    grm::block_merge<grm::kMergeWaves>(s_lists, k, B);
+    grm::block_merge(s_lists, grm::kMergeWaves, k, B);
     if (lane < k) {
       const bool ok = isfinite(B.s) && B.id != kNoId;
       out_ids[lane] = ok ? B.id : kNoId;
