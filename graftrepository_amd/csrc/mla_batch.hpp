@@ -1,15 +1,17 @@
 // mla_batch.hpp -- batched MLA route on the matrix cores (included by
 // mla_route.hip only).
 //
-// Q queries against a bf16 bank, law as the single-query route
+// Q queries against a bank, law as the single-query route
 // (cpp/grm_runtime.cpp:3518-3545):
 //   score = float( dot / (qnorm * (double)norm_f + 1e-8) ),  dot in fp64, d ascending.
 // The scores of all Q x N pairs form a dense contraction.  It runs as bf16
 // MFMA 32x32x16 with fp32 accumulation, reduced on the fly: the score
-// matrix never leaves registers.
+// matrix never leaves registers.  fp32 rows enter as the sum of two bf16
+// values, as do their queries (three products).
 //
 //  * screen  -- every node tile (32 slots) against every query of a pass
-//               (up to 256, staged in LDS).  The screened score
+//               (up to 128 staged in LDS, mla_batch_stream_kernel, or 256 in
+//               registers, mla_batch_ring_kernel).  The screened score
 //               s~ = u * (1/qnorm), u = acc * (1/norm_f) with the slot's
 //               index written into the low `ibits` mantissa bits of u,
 //               obeys |s~ - score| <= B, B a per-query constant (see
@@ -56,8 +58,8 @@ __device__ __forceinline__ uint32_t and_or_b32(uint32_t a, uint32_t b, uint32_t 
   return r;
 }
 
-constexpr int kBatchWaves = 8;       // wavefronts per screen block (one block per CU)
-constexpr int kBatchMaxCols = 256;   // queries per screen pass
+constexpr int kBatchWaves = 8;       // wavefronts per stream-screen block (one block per CU)
+constexpr int kStreamMaxCols = 128;  // queries per stream-screen pass
 constexpr int kEntryPlanes = 3;      // u1, u2, nk
 
 // Screen results, one row of n_sub values per (plane, query): plane p of
@@ -66,219 +68,293 @@ constexpr int kEntryPlanes = 3;      // u1, u2, nk
 //   the low ibits bits), nk the largest u it did not keep.
 //
 // Slot code of a value: (half << (ibits - 1)) | ((t - t_begin) << 4) | r
-// for result register r of lane half `half` in tile t of a wavefront
+// for result register r of lane half `half` in tile t of a sub-stream
 // whose tiles start at t_begin; ibits - 5 bits hold the tile offset, so
-// the host picks ibits from the longest run of tiles a wavefront walks.
+// the host picks ibits from the longest run of tiles a sub-stream walks.
 // Writing the code moves u by less than 2^(ibits-23) |u| (2^(ibits-149)
 // near zero), which the merge adds to B.
-// Screen; grid = one block of kBatchWaves wavefronts per CU, LDS holds the
-// pass's queries: qpad[QP][stride] bf16 (row d of query j at j*stride + d,
-// stride = 16*KS + 8 so the 16-byte reads of 32 rows hit distinct
-// banks).  Wavefront w walks 32-slot tiles [w*T/W, (w+1)*T/W).  For K-step
-// ks the A fragment of lane l is chunk 2*ks + l/32 (8 values) of slot
-// tile*32 + l%32 -- two 512-byte runs per load -- and the B fragment is
-// query ct*32 + l%32 at dims 16*ks + 8*(l/32) .. +8; result register r of
-// lane l is slot tile*32 + 8*(r/4) + 4*(l/32) + r%4 against that query.
+
+// bf16 pattern of f, to nearest even.
+__device__ __forceinline__ uint32_t bf16_bits_rne(float f) {
+  const uint32_t u = __float_as_uint(f);
+  return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+}
+
+// ---------------------------------------------------------- stream screen
+//
+// Passes of up to 32*CT queries against a bank of either type and any row
+// length whose query rows fit LDS.  Grid = one block of kBatchWaves
+// wavefronts per CU.  Sub-stream i walks 32-slot tiles
+// [i*T/n_sub, (i+1)*T/n_sub); with fewer tiles than wavefronts each tile
+// is a sub-stream of its own and they are dealt out block by block, so
+// every CU takes part.
+//
+// LDS holds the pass's queries: s_qb[QP][stride] bf16 (stride =
+// 16*steps + 8, an odd number of 16-byte pieces, so the reads of 32 rows
+// hit distinct banks; zero past dim), for an fp32 bank followed by the
+// same array of the remainders q - bf16(q), rounded to bf16.  For K-step
+// ks the A fragment of lane l is dims 16*ks + 8*(l/32) .. +8 of slot
+// tile*32 + l%32 (one 16-byte chunk of a bf16 bank, two of an fp32 bank)
+// and the B fragment the same dims of query ct*32 + l%32; result register
+// r of lane l is slot tile*32 + 8*(r/4) + 4*(l/32) + r%4 against that
+// query.  An fp32 fragment x is split in registers, xh = bf16(x),
+// xl = bf16(x - xh), and takes three products: xh qh + xl qh + xh ql.
+//
+// The wavefront's fragments form a ring of P K-steps: a step's registers
+// are loaded again, for the step P further on (in this tile or the next),
+// as soon as it is consumed, so P KiB (bf16) or 2 P KiB (fp32) per
+// wavefront are always in flight.  A row of ks_need K-steps runs
+// nb * P >= ks_need steps; the steps past its end, and the chunks past its
+// end in its last step, read the row's last chunk again, against zeros
+// (stored rows are finite).
+//
+// What bounds it: HBM.  Per tile of 288 fp32 values a wavefront issues 18
+// steps of 24 conversions and 3 CT MFMAs -- 54 MFMAs of 32 cycles at CT = 1
+// against 36 KiB to stream, 15 % of the matrix cores' rate.
 //
 // kProbe (tests of the screen bound only): every coded u goes to
 // planes[q*cap + slot] instead of the lists, and nothing else is written.
-template <int KS, int CT, bool kProbe = false>
-__global__ __launch_bounds__(kBatchWaves * kWave) void mla_batch_screen_kernel(
+template <int DT, int P, int CT, bool kProbe = false>
+__global__ __launch_bounds__(kBatchWaves * kWave) void mla_batch_stream_kernel(
     const u32x4* __restrict__ tiles, const float* __restrict__ norms, uint64_t cap,
-    uint32_t chunks, uint32_t n_tiles32, const uint16_t* __restrict__ qpad, int stride_arg,
-    int ibits, uint32_t* __restrict__ planes) {
+    uint32_t chunks, uint32_t n_tiles32, uint32_t n_sub, uint32_t nb, uint32_t ks_need,
+    const void* __restrict__ query, int q_dtype, int qc, uint32_t dim, float* __restrict__ inv_qn,
+    int ibits, uint32_t* __restrict__ planes, RouteStamps stamps, unsigned seq,
+    unsigned long long* __restrict__ screen_tick) {
+  route_start_stamp(stamps, seq);
+  if (screen_tick && blockIdx.x == 0 && threadIdx.x == 0) *screen_tick = wall_clock64();
+  constexpr bool kSplit = DT == kF32;
+  constexpr int V = kSplit ? 2 : 1;  // 16-byte pieces of a fragment
   constexpr int QP = 32 * CT;
-  constexpr int stride = 16 * KS + 8;  // the host's row stride (stride_arg)
-  (void)stride_arg;
-  extern __shared__ uint16_t s_qb[];  // [QP][stride]
-  {
-    const u32x4* src = reinterpret_cast<const u32x4*>(qpad);
-    u32x4* dst = reinterpret_cast<u32x4*>(s_qb);
-    const int n16 = QP * stride / 8;
-    for (int i = threadIdx.x; i < n16; i += blockDim.x) dst[i] = src[i];
-  }
-  __syncthreads();
+  const uint32_t steps = nb * P;
+  const uint32_t stride = 16 * steps + 8;
+  extern __shared__ uint16_t s_qb[];
+  uint16_t* s_ql = s_qb + QP * stride;  // remainders (fp32 banks)
   const int lane = threadIdx.x & (kWave - 1);
   const int half = lane >> 5;
   const int col = lane & 31;
-  const uint32_t W = gridDim.x * kBatchWaves;
-  const uint32_t w = blockIdx.x * kBatchWaves + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const uint32_t t_begin = static_cast<uint32_t>(static_cast<uint64_t>(w) * n_tiles32 / W);
-  const uint32_t t_end = static_cast<uint32_t>(static_cast<uint64_t>(w + 1) * n_tiles32 / W);
+  const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const uint32_t sub = n_sub == gridDim.x * kBatchWaves ? blockIdx.x * kBatchWaves + wv
+                                                        : wv * gridDim.x + blockIdx.x;
+  uint32_t t_begin = 0, t_end = 0;
+  if (sub < n_sub) {
+    t_begin = static_cast<uint32_t>(static_cast<uint64_t>(sub) * n_tiles32 / n_sub);
+    t_end = static_cast<uint32_t>(static_cast<uint64_t>(sub + 1) * n_tiles32 / n_sub);
+  }
+  auto load_frag = [&](u32x4 (&a)[V], uint32_t t, uint32_t ks) {
+    const uint32_t c0 = V * (2 * min(ks, ks_need - 1) + half);
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const uint32_t c = min(c0 + v, chunks - 1);
+      a[v] = __builtin_nontemporal_load(tiles + static_cast<uint64_t>(c) * cap +
+                                        static_cast<uint64_t>(t) * 32 + col);
+    }
+  };
+  // Row norms of a tile are wave-uniform loads, fetched one tile ahead.
+  float ns[32];
+  auto load_norms = [&](uint32_t t) {
+#pragma unroll
+    for (int j = 0; j < 32; ++j) ns[j] = norms[static_cast<size_t>(t) * 32 + j];
+  };
+  u32x4 a[P][V];
+  if (t_begin < t_end) {
+    load_norms(t_begin);
+#pragma unroll
+    for (int j = 0; j < P; ++j) load_frag(a[j], t_begin, j);
+  }
+  // Stage the queries while the first fragments are on their way: a
+  // wavefront per query row, a pair of values per lane and iteration.
+  // Block j also forms 1/||q_j|| (fp32; NaN for columns past qc).
+  auto value = [&](uint32_t q, uint32_t d) -> float {
+    const size_t i = static_cast<size_t>(q) * dim + min(d, dim - 1);
+    const float f = q_dtype == kBF16 ? bf16_to_f32(static_cast<const uint16_t*>(query)[i])
+                                     : static_cast<const float*>(query)[i];
+    return d < dim ? f : 0.0f;
+  };
+  constexpr int kStage = 4;
+  for (uint32_t q = wv; q < QP; q += kBatchWaves) {
+    uint32_t* hi = reinterpret_cast<uint32_t*>(s_qb + q * stride);
+    uint32_t* lo = reinterpret_cast<uint32_t*>(s_ql + q * stride);
+    const uint32_t qs = min(q, static_cast<uint32_t>(qc - 1));
+    for (uint32_t p0 = lane; p0 < 8 * steps; p0 += kStage * kWave) {
+      float f[kStage][2];
+#pragma unroll
+      for (int j = 0; j < kStage; ++j) {
+        f[j][0] = value(qs, 2 * (p0 + j * kWave));
+        f[j][1] = value(qs, 2 * (p0 + j * kWave) + 1);
+      }
+#pragma unroll
+      for (int j = 0; j < kStage; ++j) {
+        const uint32_t p = p0 + j * kWave;
+        if (p >= 8 * steps) continue;
+        const bool on = q < static_cast<uint32_t>(qc);
+        const uint32_t h0 = on ? bf16_bits_rne(f[j][0]) : 0u, h1 = on ? bf16_bits_rne(f[j][1]) : 0u;
+        hi[p] = h0 | (h1 << 16);
+        if constexpr (kSplit) {
+          const uint32_t l0 = on ? bf16_bits_rne(f[j][0] - bf16_to_f32(h0)) : 0u;
+          const uint32_t l1 = on ? bf16_bits_rne(f[j][1] - bf16_to_f32(h1)) : 0u;
+          lo[p] = l0 | (l1 << 16);
+        }
+      }
+    }
+  }
+  if (wv == kBatchWaves - 1) {
+    for (uint32_t q = blockIdx.x; q < QP; q += gridDim.x) {
+      double ss = 0.0;
+      if (q < static_cast<uint32_t>(qc)) {
+        for (uint32_t d = lane; d < dim; d += kWave) {
+          const double f = value(q, d);
+          ss = fma(f, f, ss);
+        }
+      }
+#pragma unroll
+      for (int off = 1; off < kWave; off <<= 1) ss += __shfl_xor(ss, off);
+      if (lane == 0) {
+        inv_qn[q] = q < static_cast<uint32_t>(qc) ? static_cast<float>(1.0 / sqrt(ss)) : __builtin_nanf("");
+      }
+    }
+  }
+  __syncthreads();
+
   // per column tile: the three largest coded u as signed-integer bits
   // (b1 >= b2 >= b3)
   int b1[CT], b2[CT], b3[CT];
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) b1[ct] = b2[ct] = b3[ct] = INT32_MIN;
   const uint32_t keep_mask = ~((1u << ibits) - 1u);
-  // A fragment ks of tile t: chunk 2*ks + half of slot t*32 + col (the
-  // bank holds 2*KS planes, zero past its chunks)
-  const u32x4* lane_base = tiles + static_cast<uint64_t>(half) * cap + col;
-  auto load_frag = [&](u32x4 (&a)[KS], uint32_t t, int ks) {
-    a[ks] = __builtin_nontemporal_load(lane_base + static_cast<uint64_t>(2 * ks) * cap +
-                                       static_cast<uint64_t>(t) * 32);
-  };
   const uint16_t* qrow = s_qb + col * stride + 8 * half;
   // Lanes track u = acc * (1/norm_f); s~ = u * (1/qnorm) is formed by the
   // merge (rounding is monotone, so the largest u give the largest s~).
   // A slot that never ranks (tombstone, unused slot, non-finite row: the
   // bank stores its row as zeros) has 1/norm_f = -0, so u is a zero and
   // never outranks a positive value.  The accumulation cannot overflow
-  // where the merge certifies (it checks ||q|| * max norm_f), so a u that
-  // is not finite comes from a non-finite query, which the merge never
-  // certifies.  u's low bits take the slot code, and the three largest
-  // move by two medians and a maximum of the integer bits:
-  // b3 = med3(b2, b3, v), b2 = med3(b1, b2, v), b1 = max(b1, v) keep
-  // b1 >= b2 >= b3 the three largest values seen.
-  auto update = [&](float accv, float w, int ct, uint32_t code) {
-    const int v = static_cast<int>(and_or_b32(__float_as_uint(accv * w), keep_mask, code));
+  // where the merge certifies (it checks the norms), so a u that is not
+  // finite comes from a query that the merge never certifies.  u's low
+  // bits take the slot code, and the three largest move by two medians and
+  // a maximum of the integer bits: b3 = med3(b2, b3, v),
+  // b2 = med3(b1, b2, v), b1 = max(b1, v) keep b1 >= b2 >= b3 the three
+  // largest values seen.
+  auto offer = [&](int v, int ct) {
     med3_i32_into(b2[ct], b3[ct], v);
     med3_i32_into(b1[ct], b2[ct], v);
     b1[ct] = max(b1[ct], v);
   };
-  // Matrix-core chains: the column tiles advance in groups of kG
-  // independent accumulation chains -- step ks issues the kG MFMAs of a[ks]
-  // with the group's kG query fragments -- and the group's 16*kG results
-  // are reduced once its chains end.  With two wavefronts per SIMD, two
-  // chains keep the matrix core as busy as four (the other wavefront
-  // fills the gaps) and halve the stretch of MFMAs between reductions,
-  // which the other wavefront's reductions then overlap more evenly: 1M x
-  // 288 x 256 queries screened in 152 us with kG = 2 against 161 us with
-  // kG = 4.  Query fragments stream from LDS kPre fragments ahead, across
-  // step and group boundaries.  In the tile's last
-  // group each a[ks] is reloaded with the next tile's fragment as soon as
-  // its last MFMA has issued, so the next tile's loads are in flight
-  // during the rest of the group and the reductions (no second tile
-  // buffer is needed).  The reload is unconditional: after a wavefront's
-  // last tile it reads that tile again (cached, and never folded).
-  constexpr int kG = CT < 2 ? CT : 2;
-  constexpr int kGroups = CT / kG;
-  constexpr int kPre = 4;
-  constexpr int kSteps = CT * KS;  // fragment stream: (group, ks, chain)
-  auto bfrag = [&](int step) -> u32x4 {
-    const int g = step / (KS * kG);
-    const int ks = (step / kG) % KS;
-    const int ct = g * kG + step % kG;
-    return *reinterpret_cast<const u32x4*>(qrow + ct * 32 * stride + 16 * ks);
-  };
-  auto fold = [&](u32x4 (&a)[KS], const float (&wr)[16], uint32_t t, uint32_t t_next) {
-    // code of result register r (slot t*32 + 8*(r/4) + 4*half + r%4): tcode | r
-    const uint32_t tcode = (static_cast<uint32_t>(half) << (ibits - 1)) | ((t - t_begin) << 4);
-    u32x4 bw[kPre];
-#pragma unroll
-    for (int j = 0; j < kPre; ++j) bw[j] = bfrag(j);
-#pragma unroll
-    for (int g = 0; g < kGroups; ++g) {
-      f32x16 acc[kG];
-#pragma unroll
-      for (int c = 0; c < kG; ++c) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[c][r] = 0.0f;
-      }
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-        for (int c = 0; c < kG; ++c) {
-          const int step = (g * KS + ks) * kG + c;
-          const u32x4 b = bw[step % kPre];
-          if (step + kPre < kSteps) bw[step % kPre] = bfrag(step + kPre);
-          acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[ks]),
-                                                           __builtin_bit_cast(bf16x8, b), acc[c],
-                                                           0, 0, 0);
-        }
-        if (g == kGroups - 1) load_frag(a, t_next, ks);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int c = 0; c < kG; ++c) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          if constexpr (kProbe) {
-            const uint32_t slot = t * 32u + 8u * (r / 4) + 4u * half + (r % 4);
-            const uint32_t q = (g * kG + c) * 32u + col;
-            planes[static_cast<size_t>(q) * cap + slot] =
-                and_or_b32(__float_as_uint(acc[c][r] * wr[r]), keep_mask, tcode | static_cast<uint32_t>(r));
-          } else {
-            update(acc[c][r], wr[r], g * kG + c, tcode | static_cast<uint32_t>(r));
-          }
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-  // Row norms of a tile are wave-uniform loads, fetched one tile ahead.
-  // 1/norm_f: -0 for a slot that never ranks (norm NaN: tombstone, unused
-  // slot, non-finite row) and for a norm that overflowed (its law score is
-  // a zero), 0 for an all-zero row (score 0, exact).
-  float ns[32];
-  auto load_norms = [&](uint32_t t) {
-#pragma unroll
-    for (int j = 0; j < 32; ++j) ns[j] = norms[static_cast<size_t>(t) * 32 + j];
-  };
-  // One tile buffer per wavefront, refilled for the next tile during the
-  // current tile's last group (see fold).
-  u32x4 a[KS];
-  if (t_begin < t_end) {
-    load_norms(t_begin);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) load_frag(a, t_begin, ks);
-  }
   for (uint32_t t = t_begin; t < t_end; ++t) {
+    // 1/norm_f: -0 for a slot that never ranks (norm NaN) and for a norm
+    // that overflowed (its law score is a zero), 0 for an all-zero row
+    // (score 0, exact).
     float wr[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int j = 8 * (r / 4) + (r % 4);
-      const float n0 = ns[j];
-      const float n1 = ns[j + 4];
-      const float nf = __builtin_bit_cast(float, half ? __float_as_uint(n1) : __float_as_uint(n0));
+      const float nf = __uint_as_float(half ? __float_as_uint(ns[j + 4]) : __float_as_uint(ns[j]));
       wr[r] = nf == 0.0f ? 0.0f : (nf < INFINITY ? __builtin_amdgcn_rcpf(nf) : -0.0f);
     }
-    if (t + 1 < t_end) load_norms(t + 1);
-    fold(a, wr, t, t + 1 < t_end ? t + 1 : t);
+    const uint32_t t_next = t + 1 < t_end ? t + 1 : t;  // the last reload is never folded
+    load_norms(t_next);
+    f32x16 acc[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) acc[ct] = f32x16{};
+    for (uint32_t kb = 0; kb < nb; ++kb) {
+      const bool last = kb + 1 == nb;
+      const uint32_t t_load = last ? t_next : t;
+      const uint32_t k_load = last ? 0 : (kb + 1) * P;
+#pragma unroll
+      for (int j = 0; j < P; ++j) {
+        const uint16_t* qk = qrow + 16 * (kb * P + j);
+        u32x4 bh[CT];
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+          bh[ct] = *reinterpret_cast<const u32x4*>(qk + ct * 32 * stride);
+        }
+        if constexpr (kSplit) {
+          u32x4 bl[CT];
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) {
+            bl[ct] = *reinterpret_cast<const u32x4*>(qk + (QP + ct * 32) * stride);
+          }
+          const u32x4 w0 = a[j][0], w1 = a[j][V - 1];
+          const uint32_t w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+          bf16x8 xh, xl;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float x = __uint_as_float(w[e]);
+            xh[e] = static_cast<__bf16>(x);
+            xl[e] = static_cast<__bf16>(x - static_cast<float>(xh[e]));
+          }
+          load_frag(a[j], t_load, k_load + j);
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) {
+            acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xh, __builtin_bit_cast(bf16x8, bh[ct]),
+                                                              acc[ct], 0, 0, 0);
+          }
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) {
+            acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xl, __builtin_bit_cast(bf16x8, bh[ct]),
+                                                              acc[ct], 0, 0, 0);
+          }
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) {
+            acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xh, __builtin_bit_cast(bf16x8, bl[ct]),
+                                                              acc[ct], 0, 0, 0);
+          }
+        } else {
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct) {
+            acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[j][0]),
+                                                              __builtin_bit_cast(bf16x8, bh[ct]),
+                                                              acc[ct], 0, 0, 0);
+          }
+          load_frag(a[j], t_load, k_load + j);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    const uint32_t tcode = (static_cast<uint32_t>(half) << (ibits - 1)) | ((t - t_begin) << 4);
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const uint32_t u = and_or_b32(__float_as_uint(acc[ct][r] * wr[r]), keep_mask,
+                                      tcode | static_cast<uint32_t>(r));
+        if constexpr (kProbe) {
+          const uint32_t slot = t * 32u + 8u * (r / 4) + 4u * half + (r % 4);
+          planes[static_cast<size_t>(ct * 32u + col) * cap + slot] = u;
+        } else {
+          offer(static_cast<int>(u), ct);
+        }
+      }
+    }
   }
   if constexpr (kProbe) return;
+  if (sub >= n_sub) return;
   // The two lane halves of a column hold disjoint slots: merge their lists
-  // (each half's three values go through the same update as a score), then
-  // the block's 8 sub-streams per query go out through LDS so that every
-  // (plane, query) row receives one 32-byte run.
-  __syncthreads();  // every wavefront is done with the staged queries
-  uint32_t* s_out = reinterpret_cast<uint32_t*>(s_qb);  // [kEntryPlanes][QP][kBatchWaves]
-  const int wv = threadIdx.x / kWave;
+  // (each half's three values go through the same update as a score).
 #pragma unroll
   for (int ct = 0; ct < CT; ++ct) {
     const int o1 = __shfl_xor(b1[ct], 32);
     const int o2 = __shfl_xor(b2[ct], 32);
     const int o3 = __shfl_xor(b3[ct], 32);
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const int v = j == 0 ? o1 : (j == 1 ? o2 : o3);
-      med3_i32_into(b2[ct], b3[ct], v);
-      med3_i32_into(b1[ct], b2[ct], v);
-      b1[ct] = max(b1[ct], v);
-    }
+    offer(o1, ct);
+    offer(o2, ct);
+    offer(o3, ct);
     if (half == 0) {
-      const int q = ct * 32 + col;
-      s_out[(0 * QP + q) * kBatchWaves + wv] = static_cast<uint32_t>(b1[ct]);
-      s_out[(1 * QP + q) * kBatchWaves + wv] = static_cast<uint32_t>(b2[ct]);
-      s_out[(2 * QP + q) * kBatchWaves + wv] = static_cast<uint32_t>(b3[ct]);
+      const size_t q = static_cast<size_t>(ct * 32 + col);
+      planes[(0 * QP + q) * n_sub + sub] = static_cast<uint32_t>(b1[ct]);
+      planes[(1 * QP + q) * n_sub + sub] = static_cast<uint32_t>(b2[ct]);
+      planes[(2 * QP + q) * n_sub + sub] = static_cast<uint32_t>(b3[ct]);
     }
-  }
-  __syncthreads();
-  const size_t n_sub = static_cast<size_t>(gridDim.x) * kBatchWaves;
-  for (int x = threadIdx.x; x < kEntryPlanes * QP * 2; x += blockDim.x) {
-    const int pq = x >> 1;
-    const u32x4 v = reinterpret_cast<const u32x4*>(s_out)[x];
-    *reinterpret_cast<u32x4*>(planes + pq * n_sub + blockIdx.x * kBatchWaves + (x & 1) * 4) = v;
   }
 }
 
 // ------------------------------------------------------------ ring screen
 //
-// The same screen for a full pass of 256 queries, with the roles of LDS
-// and registers swapped: each wavefront holds 64 queries' B fragments in
-// registers for the whole bank, and the bank's 32-slot tiles stream into
-// LDS, so every A fragment read from LDS feeds two MFMAs (the query
-// fragments of mla_batch_screen_kernel cost one 1 KiB LDS read per MFMA).
+// The same screen for a full pass of 256 queries on a bf16 bank, with the
+// roles of LDS and registers swapped: each wavefront holds 64 queries' B
+// fragments in registers for the whole bank, and the bank's 32-slot tiles
+// stream into LDS, so every A fragment read from LDS feeds two MFMAs (the
+// query fragments of mla_batch_stream_kernel cost one 1 KiB LDS read per
+// MFMA).
 //
 //  * One block of four wavefronts per CU; wavefront w holds queries
 //    [64 w, 64 w + 64) and has SIMD w to itself, so its 512 registers hold
@@ -290,7 +366,7 @@ __global__ __launch_bounds__(kBatchWaves * kWave) void mla_batch_screen_kernel(
 //  * Block b is sub-stream b of W = blocks and walks tiles
 //    [b * n_tiles32 / W, (b + 1) * n_tiles32 / W), one per step, so the
 //    merge decodes its slot codes as for the wavefront sub-streams of
-//    mla_batch_screen_kernel.
+//    mla_batch_stream_kernel.
 //  * A ring of kRing tiles in LDS (2 KS chunk planes of 512 bytes each,
 //    chunk c of the tile at c * 512) with their 32 slot weights.  Direct
 //    loads (global_load_lds_dwordx4) fill it without registers.  A step is
@@ -307,7 +383,7 @@ __global__ __launch_bounds__(kBatchWaves * kWave) void mla_batch_screen_kernel(
 //    past the block's last tile re-read that tile (never screened), so
 //    every step has the same load count.
 //  * The slot weights 1/norm_f come from mla_batch_weights_kernel, the
-//    values mla_batch_screen_kernel forms per tile (same reciprocal).
+//    values mla_batch_stream_kernel forms per tile (same reciprocal).
 template <int KS>
 struct RingShape {
   static constexpr int kRing = 8;                         // tiles in LDS
@@ -344,7 +420,9 @@ __global__ void mla_batch_weights_kernel(const float* __restrict__ norms, uint64
 template <int KS, bool kProbe = false>
 __global__ __launch_bounds__(kRingWaves * kWave, 1) void mla_batch_ring_kernel(
     const u32x4* __restrict__ tiles, const float* __restrict__ winv, uint64_t cap,
-    uint32_t n_tiles32, const uint16_t* __restrict__ qpad, int ibits, uint32_t* __restrict__ planes) {
+    uint32_t n_tiles32, const uint16_t* __restrict__ qpad, int ibits, uint32_t* __restrict__ planes,
+    unsigned long long* __restrict__ screen_tick) {
+  if (screen_tick && blockIdx.x == 0 && threadIdx.x == 0) *screen_tick = wall_clock64();
   using RS = RingShape<KS>;
   constexpr int stride = 16 * KS + 8;  // qpad row stride (bf16 elements)
   constexpr int QP = kRingQueries;
@@ -545,13 +623,14 @@ __global__ __launch_bounds__(kRingWaves * kWave, 1) void mla_batch_ring_kernel(
   }
 }
 
-// Query rows of one pass for the screen: qpad[j][0, stride) = query j's
+// Query rows of one ring pass: qpad[j][0, stride) = query j's
 // values rounded to bf16 (nearest even; bf16 queries are copied), zero past
 // dim; inv_qn[j] = 1 / ||q_j|| rounded to fp32.  Rows j >= qc are zero with
 // inv_qn NaN (nothing is kept for them).  grid = QP blocks.
 __global__ __launch_bounds__(kWave) void mla_batch_qprep_kernel(
     const void* __restrict__ query, int q_dtype, int qc, uint32_t dim, int stride,
-    uint16_t* __restrict__ qpad, float* __restrict__ inv_qn) {
+    uint16_t* __restrict__ qpad, float* __restrict__ inv_qn, RouteStamps stamps, unsigned seq) {
+  route_start_stamp(stamps, seq);
   const int j = blockIdx.x;
   const int lane = threadIdx.x;
   double ss = 0.0;
@@ -565,8 +644,7 @@ __global__ __launch_bounds__(kWave) void mla_batch_qprep_kernel(
         f = bf16_to_f32(bits);
       } else {
         f = static_cast<const float*>(query)[idx];
-        const uint32_t u = __float_as_uint(f);
-        bits = static_cast<uint16_t>((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+        bits = static_cast<uint16_t>(bf16_bits_rne(f));
       }
       ss = fma(static_cast<double>(f), static_cast<double>(f), ss);
     }
@@ -603,13 +681,18 @@ __device__ inline float wave_sort_desc(float v) {
 // the code in u's low ibits bits.  The screen bound for the query
 // (|s~ - score|):
 //   B0 = (gamma + delta) * (1 + 2^-20) + 8 * 2^-24
-//        + 1.01e-8 / (qn * nmin) + sqrt(dim) * 2^-125 * (1/qn + 1/nmin)
-//        + dim * 2^-125 / (qn * nmin),
+//        + 1.01e-8 / (qn * nmin) + m * sqrt(dim) * 2^-125 * (1/qn + 1/nmin)
+//        + m * dim * 2^-125 / (qn * nmin),
 //   B  = B0 + 2^(ibits-23) * (1 + B0) * (1 + 2^-20) + 2^(ibits-148) / qn,
-// gamma bounding the fp32 accumulation, delta the rounding of an fp32
-// query to bf16, 8 * 2^-24 the reciprocals and products of the screened
+// gamma bounding the fp32 accumulation, delta what the bf16 operands leave
+// out (of a bf16 bank ||q - bf16(q)|| / ||q||, Cauchy-Schwarz, about a
+// third of 2^-8 for an fp32 query and 0 for a bf16 one; of an fp32 bank, with
+// x = xh + xl + ex and q = qh + ql + eq, |xl| <= 2^-9 |x| and
+// |ex| <= 2^-18 |x| per value: ex q, x eq and xl ql, below 4 * 2^-18
+// together), 8 * 2^-24 the reciprocals and products of the screened
 // score and the score's own rounding, the 1e-8 term the law's
-// denominator, the next terms bf16 values or products flushed near zero;
+// denominator, the next terms bf16 values or products flushed near zero
+// (m = 1, or 4 for the fp32 bank's two parts a value and three products);
 // the last two the slot code written into u (relative to |u|, with
 // |score| <= 1, and absolute near zero).  qn is the law's query norm and
 // nmin the smallest positive row norm.
@@ -626,48 +709,81 @@ __device__ inline float wave_sort_desc(float v) {
 // prefix of the ranking -- form the law's dot products of their rows and
 // are ranked by law score (score desc, node id asc).  Rescoring entries
 // below t as well changes nothing: they are real nodes with law scores.
-// Writes out[qi*k ..) (the law's top-k, host mapped) and status[qi] = 1
-// when certified (0: route qi again on the exact path).
-constexpr uint32_t kBatchMaxDim = 288;
+// Writes out[qi*k ..) (host mapped): the law's top-k where certified, else
+// k entries without a node (kNoId: route qi again on the exact path).  With
+// `done` the entries carry the route's tag and done[qi] takes its number
+// (store_entry, block_done_flag).
+//
+// Dynamic LDS: the query as doubles, zero past dim up to whole batches of
+// kMergeChunks row chunks (merge_query_len).
+constexpr int kMergeChunks = 36;  // row chunks a rescoring thread has in flight
 
-// The law's query norm (d ascending, fp64): one wavefront stages query qi
-// (`dim` values, F32 or BF16, qstride elements apart) as doubles in
-// s_q[kBatchMaxDim], zero past dim; its lane 0 sums the squares and
-// returns the norm (other lanes return 0).
+__host__ __device__ inline uint32_t merge_query_len(uint32_t chunks, uint32_t epc) {
+  return (chunks + kMergeChunks - 1) / kMergeChunks * kMergeChunks * epc;
+}
+
+// One wavefront stages query qi (`dim` values, F32 or BF16, qstride elements
+// apart) as doubles in s_q[0, len), zero past dim; its lane 0 returns the
+// law's norm (staged_norm; other lanes 0).  rest takes
+// ||q - bf16(q)||, every lane.
 __device__ inline double stage_query_norm(double* __restrict__ s_q, const void* __restrict__ query,
                                           int q_dtype, size_t qstride, int qi, uint32_t dim,
-                                          int lane) {
+                                          uint32_t len, int lane, double& rest) {
   const unsigned char* qbase = static_cast<const unsigned char*>(query) +
                                static_cast<size_t>(qi) * qstride * (q_dtype == kBF16 ? 2 : 4);
-  for (uint32_t d = lane; d < kBatchMaxDim; d += kWave) {
-    double x = 0.0;
-    if (d < dim) {
-      x = q_dtype == kBF16
-              ? static_cast<double>(bf16_to_f32(reinterpret_cast<const uint16_t*>(qbase)[d]))
-              : static_cast<double>(reinterpret_cast<const float*>(qbase)[d]);
+  constexpr int kAhead = 8;
+  double rr = 0.0;
+  for (uint32_t d0 = lane; d0 < len; d0 += kAhead * kWave) {
+    float f[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const uint32_t d = min(d0 + j * kWave, dim - 1);
+      f[j] = q_dtype == kBF16 ? bf16_to_f32(reinterpret_cast<const uint16_t*>(qbase)[d])
+                              : reinterpret_cast<const float*>(qbase)[d];
     }
-    s_q[d] = x;
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+      const uint32_t d = d0 + j * kWave;
+      if (d < len) s_q[d] = d < dim ? static_cast<double>(f[j]) : 0.0;
+      const double r = f[j] - bf16_to_f32(bf16_bits_rne(f[j]));  // exact
+      if (d < dim) rr = fma(r, r, rr);
+    }
   }
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) rr += __shfl_xor(rr, off);
+  rest = sqrt(rr);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  double acc = 0.0;
-  if (lane == 0) {
-#pragma unroll
-    for (uint32_t d = 0; d < kBatchMaxDim; ++d) acc = fma(s_q[d], s_q[d], acc);
-  }
-  return sqrt(acc);
+  return lane == 0 ? staged_norm(s_q, (dim + 3) / 4 * 4) : 0.0;
 }
 
+// What the screen bound of a pass rests on besides the norms.
+struct ScreenBound {
+  double gamma;  // fp32 accumulation
+  double delta;  // operands' rounding to bf16; negative: that of the query alone
+  double absm;   // m: the terms near zero
+  uint32_t dim;
+  int ibits;     // slot code width
+};
+
 // The screen bound B of a query (|s~ - score|, see mla_batch_merge_kernel)
-// from the law's query norm qn and the smallest positive row norm nmin;
-// it holds where qn * nmax < 2^125 (nmax the largest row norm).
-__device__ inline double batch_screen_bound(double gamma, double delta, double qn, double nmin,
-                                            uint32_t dim, int ibits) {
-  const double bound0 = (gamma + delta) * (1.0 + 0x1p-20) + 8.0 * 0x1p-24 + 1.01e-8 / (qn * nmin) +
-                        sqrt(static_cast<double>(dim)) * 0x1p-125 * (1.0 / qn + 1.0 / nmin) +
-                        dim * 0x1p-125 / (qn * nmin);
-  return bound0 + ldexp(1.0 + bound0, ibits - 23) * (1.0 + 0x1p-20) + ldexp(1.0, ibits - 148) / qn;
+// from the law's query norm qn, rest = ||q - bf16(q)|| and the smallest
+// positive row norm nmin;
+// it holds where screen_in_range(qn, nmax).
+__device__ inline double batch_screen_bound(const ScreenBound& b, double qn, double rest, double nmin) {
+  const double dim = static_cast<double>(b.dim);
+  const double delta = b.delta < 0.0 ? rest / qn : b.delta;
+  const double bound0 = (b.gamma + delta) * (1.0 + 0x1p-20) + 8.0 * 0x1p-24 + 1.01e-8 / (qn * nmin) +
+                        b.absm * sqrt(dim) * 0x1p-125 * (1.0 / qn + 1.0 / nmin) +
+                        b.absm * dim * 0x1p-125 / (qn * nmin);
+  return bound0 + ldexp(1.0 + bound0, b.ibits - 23) * (1.0 + 0x1p-20) + ldexp(1.0, b.ibits - 148) / qn;
+}
+// No product or partial sum of the screen can reach the fp32 overflow
+// threshold (Cauchy-Schwarz, with the operands' and the accumulation's
+// rounding), and no value its rounding to bf16; nmax the largest row norm.
+__device__ inline bool screen_in_range(double qn, double nmax) {
+  return qn * nmax < 0x1p125 && qn < 0x1p126 && nmax < 0x1p126;
 }
 
 constexpr int kMergeThreads = 512;
@@ -676,14 +792,18 @@ constexpr int kMergeLoaders = kMergeThreads - kWave;  // threads of the entry-lo
 constexpr int kMergePer = 8;       // sub-streams per loading thread: n_sub <= 3584
 constexpr int kSurvMax = kMergeThreads;
 
+template <int DT>
 __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
-    const uint32_t* __restrict__ planes, uint32_t n_sub, int QP, uint32_t n_tiles32, int ibits,
+    const uint32_t* __restrict__ planes, uint32_t n_sub, int QP, uint32_t n_tiles32,
     const float* __restrict__ inv_qn, const u32x4* __restrict__ tiles,
     const float* __restrict__ norms, const uint64_t* __restrict__ ids, uint64_t cap,
-    uint32_t dim, const void* __restrict__ query, int q_dtype, size_t qstride, double gamma,
-    double delta, const unsigned* __restrict__ norm_range, int k, Cand* __restrict__ out,
-    unsigned* __restrict__ status) {
-  __shared__ double s_q[kBatchMaxDim];      // the query, zero past dim
+    uint32_t chunks, const void* __restrict__ query, int q_dtype, size_t qstride, ScreenBound sb,
+    const unsigned* __restrict__ norm_range, int k, Cand* __restrict__ out,
+    unsigned* __restrict__ done, unsigned seq, unsigned long long* __restrict__ end_tick,
+    unsigned long long* __restrict__ screen_tick) {
+  if (screen_tick && blockIdx.x == 0 && threadIdx.x == 0) *screen_tick = wall_clock64();
+  constexpr uint32_t EPC = DT == kF32 ? 4 : 8;
+  extern __shared__ double s_q[];           // the query, zero past dim
   __shared__ float s_lw[kMergeWavesB];      // per wavefront: k-th largest lane maximum
   __shared__ float s_nk[kMergeWavesB];      // per wavefront: largest dropped s~
   __shared__ __align__(16) float s_sv[kSurvMax];       // survivors: s~
@@ -692,8 +812,8 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
   __shared__ uint16_t s_byrank[kSurvMax];   // survivor holding each s~ rank
   __shared__ float s_es[kSurvMax];          // law scores of the ranked prefix (NaN: not finite)
   __shared__ uint64_t s_eid[kSurvMax];
-  __shared__ uint32_t s_eslot[kSurvMax];
-  __shared__ double s_qn;
+  __shared__ Cand s_top[kMaxTopK];
+  __shared__ double s_qn, s_rest;
   __shared__ float s_ek;
   __shared__ unsigned s_count;
   const int tid = threadIdx.x;
@@ -706,6 +826,7 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
   const float* p_u2 = p_u1 + plane;
   const float* p_nk = p_u2 + plane;
   const float iq = inv_qn[qi];
+  const int ibits = sb.ibits;
   const uint32_t cmask = (1u << ibits) - 1u;
   // slot of coded value u kept by sub-stream i (see the screen's slot code)
   auto slot_of = [&](float u, uint32_t i) -> uint32_t {
@@ -738,8 +859,13 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
   }
   if (wave == kMergeWavesB - 1) {
     // the last wavefront stages the query and forms the law's qnorm
-    const double qn = stage_query_norm(s_q, query, q_dtype, qstride, qi, dim, lane);
-    if (lane == 0) s_qn = qn;
+    double rest;
+    const double qn = stage_query_norm(s_q, query, q_dtype, qstride, qi, sb.dim,
+                                       merge_query_len(chunks, EPC), lane, rest);
+    if (lane == 0) {
+      s_qn = qn;
+      s_rest = rest;
+    }
   }
   if (tid == 0) s_count = 0u;
   // largest finite kept s~ of the thread; a +inf s~ voids the certificate
@@ -761,7 +887,7 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
   const double qn = s_qn;
   const double nmin = static_cast<double>(__uint_as_float(norm_range[0]));
   const double nmax = static_cast<double>(__uint_as_float(norm_range[1]));
-  const double bound = batch_screen_bound(gamma, delta, qn, nmin, dim, ibits);
+  const double bound = batch_screen_bound(sb, qn, s_rest, nmin);
   float L = -INFINITY, nk_all = -INFINITY;
 #pragma unroll
   for (int w = 0; w < kMergeWavesB - 1; ++w) {
@@ -820,25 +946,19 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
     if (sup) {
       // the law's dot product of the row, d ascending (rows and the
       // staged query are zero past dim: exact zeros)
-      constexpr int kC = kBatchMaxDim / 8;
       slot = s_slot[tid];
-      const uint32_t chunks = (dim + 7) / 8;
-      u32x4 rv[kC];
-#pragma unroll
-      for (int j = 0; j < kC; ++j) {
-        const u32x4 zero = {0u, 0u, 0u, 0u};
-        rv[j] = static_cast<uint32_t>(j) < chunks ? tiles[static_cast<size_t>(j) * cap + slot] : zero;
-      }
       nf = norms[slot];
       eid = ids[slot];
+      for (uint32_t c0 = 0; c0 < chunks; c0 += kMergeChunks) {
+        u32x4 rv[kMergeChunks];
 #pragma unroll
-      for (int j = 0; j < kC; ++j) {
-        const uint32_t w4[4] = {rv[j].x, rv[j].y, rv[j].z, rv[j].w};
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float f = bf16_to_f32((w4[e >> 1] >> (16 * (e & 1))) & 0xffffu);
-          dot = fma(static_cast<double>(f), s_q[j * 8 + e], dot);
+        for (uint32_t j = 0; j < kMergeChunks; ++j) {
+          const u32x4 zero = {0u, 0u, 0u, 0u};
+          rv[j] = c0 + j < chunks ? tiles[static_cast<size_t>(c0 + j) * cap + slot] : zero;
         }
+        const double* q = s_q + c0 * EPC;
+#pragma unroll
+        for (uint32_t j = 0; j < kMergeChunks; ++j) dot = chunk_dot<DT>(rv[j], q + j * EPC, dot);
       }
     }
   }
@@ -846,19 +966,15 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
   const float vk = n >= k ? s_sv[s_byrank[k - 1]] : -INFINITY;
   const double t = static_cast<double>(vk) - 2.0 * bound - 0x1p-40;
   // t > 0: the screen kept its values by their integer bits, the float
-  // order only from +0 up.  qn * nmax < 2^125: no product or partial sum
-  // of the bf16 query (norm at most qn * (1 + 2^-8)) and a row can reach
-  // the fp32 overflow threshold (Cauchy-Schwarz, with the accumulation's
-  // rounding), so the bound B holds for every screened value.
+  // order only from +0 up.
   const bool pre = any_pinf == 0 && count <= static_cast<unsigned>(kSurvMax) && n >= k &&
-                   static_cast<double>(nk_all) < t && t > 0.0 && qn * nmax < 0x1p125;
+                   static_cast<double>(nk_all) < t && t > 0.0 && screen_in_range(qn, nmax);
   // the rescored prefix: ranks [0, n_el)
   if (sup) {
     const float sc = static_cast<float>(dot / (qn * static_cast<double>(nf) + 1e-8));
     const bool fin = isfinite(sc);
     s_es[my_rank] = fin ? sc : __builtin_nanf("");
     s_eid[my_rank] = fin ? eid : kNoId;
-    s_eslot[my_rank] = slot;
   }
   __syncthreads();
   // rank the prefix by (law score desc, node id asc)
@@ -871,40 +987,47 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
     if (rank < k) {
       Cand c;
       c.score = es;
-      c.slot = s_eslot[tid];
+      c.slot = kNoSlot;
       c.id = id;
-      out[static_cast<size_t>(qi) * k + rank] = c;
+      s_top[rank] = c;
     }
     if (rank == k - 1) s_ek = es;
   }
   const int n_fin = __syncthreads_count(fin ? 1 : 0);
-  if (tid == 0) {
+  if (tid < k) {
     // every node outside the prefix scores below v_k - B
     const bool ok = pre && n_fin >= k &&
                     static_cast<double>(s_ek) >= static_cast<double>(vk) - bound;
-    status[qi] = ok ? 1u : 0u;
+    Cand c;
+    c.score = __builtin_nanf("");
+    c.slot = kNoSlot;
+    c.id = kNoId;
+    if (ok) c = s_top[tid];
+    store_entry(out + static_cast<size_t>(qi) * k + tid, c, done ? route_tag(seq) : kNoSlot);
   }
+  block_done_flag(done, seq, end_tick);
 }
 
 // Tests of the screen bound: the screened scores s~ = u * (1/||q||) of a
 // probe screen (planes[q*cap + slot], coded u bits) for slots [0, n),
 // out_values[qi*n + slot], and the query's bound B, out_bounds[qi] (+inf
-// where qn * nmax >= 2^125: B is not established there).  grid = queries
+// where it is not established, screen_in_range).  grid = queries
 // of the pass, one wavefront each.
 __global__ __launch_bounds__(kWave) void mla_batch_probe_finish_kernel(
     const uint32_t* __restrict__ planes, uint64_t cap, uint32_t n, const float* __restrict__ inv_qn,
-    const void* __restrict__ query, int q_dtype, size_t qstride, uint32_t dim, double gamma,
-    double delta, const unsigned* __restrict__ norm_range, int ibits, float* __restrict__ out_values,
+    const void* __restrict__ query, int q_dtype, size_t qstride, uint32_t len, ScreenBound sb,
+    const unsigned* __restrict__ norm_range, float* __restrict__ out_values,
     double* __restrict__ out_bounds) {
-  __shared__ double s_q[kBatchMaxDim];
+  extern __shared__ double s_q[];  // len values
   const int qi = blockIdx.x;
   const int lane = threadIdx.x;
-  const double qn = stage_query_norm(s_q, query, q_dtype, qstride, qi, dim, lane);
+  double rest;
+  const double qn = stage_query_norm(s_q, query, q_dtype, qstride, qi, sb.dim, len, lane, rest);
   if (lane == 0) {
     const double nmin = static_cast<double>(__uint_as_float(norm_range[0]));
     const double nmax = static_cast<double>(__uint_as_float(norm_range[1]));
-    out_bounds[qi] = qn * nmax < 0x1p125 ? batch_screen_bound(gamma, delta, qn, nmin, dim, ibits)
-                                         : static_cast<double>(INFINITY);
+    out_bounds[qi] = screen_in_range(qn, nmax) ? batch_screen_bound(sb, qn, rest, nmin)
+                                               : static_cast<double>(INFINITY);
   }
   const float iq = inv_qn[qi];
   for (uint32_t s = lane; s < n; s += kWave) {

@@ -23,9 +23,9 @@
 // mapped host memory, where the host merges the per-block lists after the
 // kernel's completion event -- the score vector never leaves registers.
 //
-// Batched queries on a bf16 bank take the matrix-core path (mla_batch.hpp):
-// an MFMA screen of 32 slots x up to 256 queries per wave keeps a per-lane
-// shortlist, a merge kernel certifies each query's top-k against a proven
+// Batched queries take the matrix-core path (mla_batch.hpp): an MFMA screen
+// of 32 slots x up to 256 queries per wave keeps a per-lane shortlist, a
+// merge kernel certifies each query's top-k against a proven
 // bound on the screen's rounding error and rescores the shortlist with the
 // exact law; queries without a certificate are routed again here.
 #include "grm_common.hpp"
@@ -35,6 +35,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <limits>
 #include <mutex>
 #include <set>
@@ -373,7 +374,7 @@ struct MlaDeviceArena {
   uint32_t dim_pad = 0;
   uint32_t epc = 4;
   uint32_t chunks = 0;
-  uint32_t planes = 0;      // chunk planes allocated: chunks, or (bf16) the batched screen's 2*KS
+  uint32_t planes = 0;      // chunk planes allocated: chunks, or (bf16) the ring screen's 2*KS
   uint64_t capacity = 0;    // slots, multiple of 64
   uint64_t high_water = 0;  // slots [0, high_water) may hold live rows
   uint64_t live = 0;
@@ -412,7 +413,7 @@ struct MlaDeviceArena {
   hipEvent_t ev_mut = nullptr;
   bool mut_pending = false;
   unsigned* d_min_norm = nullptr;  // [smallest positive, largest finite] row norm placed (float bits)
-  // batched route (bf16 banks): pass buffers and per-query results
+  // batched route: pass buffers and per-query results
   uint16_t* d_qpad = nullptr;
   size_t d_qpad_count = 0;
   float* d_inv_qn = nullptr;
@@ -420,7 +421,7 @@ struct MlaDeviceArena {
   uint32_t* d_entries = nullptr;   // screen result planes
   size_t d_entries_count = 0;
   grm::MappedCands batch_out;
-  grm::MappedBuf batch_status;
+  grm::MappedBuf screen_ticks;  // device clock at the start of each pass's screen and merge
   // host queries staged for fetch_async (GRM_HIP_QUERY_COPY=dma: the copy
   // engine instead)
   grm::MappedBuf q_map;
@@ -468,7 +469,7 @@ void destroy_arena(MlaDeviceArena* a) {
   if (a->d_entries) (void)hipFree(a->d_entries);
   if (a->d_winv) (void)hipFree(a->d_winv);
   grm::release_mapped(&a->batch_out);
-  grm::release_mapped_bytes(&a->batch_status);
+  grm::release_mapped_bytes(&a->screen_ticks);
   grm::release_mapped_bytes(&a->q_map);
   grm::release_mapped(&a->blocks_out);
   grm::release_mapped_bytes(&a->done_flags);
@@ -566,7 +567,7 @@ int create_arena(const void* rows, int dtype, uint64_t nodes, int dim,
   a->epc = dtype == kF32 ? 4 : 8;
   a->dim_pad = (a->dim + a->epc - 1) / a->epc * a->epc;
   a->chunks = a->dim_pad / a->epc;
-  // bf16 banks get zero planes up to the batched screen's 16-dimension
+  // bf16 banks get zero planes up to the ring screen's 16-dimension
   // K-steps (16, 32 or 36 planes), which it then reads unconditionally
   a->planes = a->chunks;
   if (dtype == kBF16) {
@@ -762,66 +763,86 @@ void write_cands(const Cand* c, int topk, uint64_t* out_ids, float* out_scores) 
   }
 }
 
-// Batched-route plan: K-steps of 16 dims (template), LDS row stride.
+// Batched-route plan.
 struct BatchPlan {
-  int ks = 0;        // 8, 16 or 18
-  int stride = 0;    // bf16 elements per staged query row
-  int qp_max = 0;    // queries per pass (multiple of 32, <= 256)
-  int ibits = 0;     // width of the slot code the screen writes into its values
-  bool ring = false;   // full passes run mla_batch_ring_kernel
+  int ks = 0;          // K-steps of 16 dims that cover a row
+  int p = 0;           // K-steps in flight per wavefront of the stream screen
+  int nb = 0;          // batches of p steps: nb * p >= ks
+  int qp_max = 0;      // queries per pass (32, 64, 128, or 256 on the ring)
+  int qp_stream = 0;   // queries per stream-screen pass
+  uint32_t subs = 0;   // sub-streams of a stream-screen pass
+  int ibits = 0;       // width of the slot code the stream screen writes into its values
+  bool ring = false;   // full passes of a bf16 bank run mla_batch_ring_kernel
+  int ks_ring = 0;     // its K-steps (8, 16 or 18)
   int ibits_ring = 0;  // its slot code width (one sub-stream per block)
 };
 
 // Slot code width of the batched screen: 4 bits of result register, the
-// lane half, and enough bits for the longest run of tiles one screen
-// wavefront walks.  The code costs the screen bound 2^(ibits-23) relative,
-// so banks whose runs would need more than 16 bits route on the
-// single-query path instead.
+// lane half, and enough bits for the longest run of tiles one sub-stream
+// walks.  The code costs the screen bound 2^(ibits-23) relative, so banks
+// whose runs would need more than 16 bits route on the single-query path
+// instead.
 constexpr int kMaxSlotCodeBits = 16;
 
+// LDS of a stream-screen pass of qp queries (of an fp32 bank their bf16
+// parts and remainders).
+size_t stream_lds(const MlaDeviceArena* a, const BatchPlan& p, int qp) {
+  return static_cast<size_t>(qp) * (16 * p.nb * p.p + 8) * (a->dtype == kF32 ? 4 : 2);
+}
+
 bool batch_plan(const MlaDeviceArena* a, int q_timed, BatchPlan* p) {
-  if (a->dtype != kBF16 || q_timed < a->batch_min) return false;
-  const uint32_t ks_need = (a->chunks + 1) / 2;
-  p->ks = ks_need <= 8 ? 8 : (ks_need <= 16 ? 16 : (ks_need <= 18 ? 18 : 0));
-  if (p->ks == 0 || a->planes < 2u * p->ks) return false;
-  // 16*ks >= dim_pad always (ks covers the row's chunks); the screen
-  // kernel takes this stride as a compile-time constant of its KS
-  p->stride = 16 * p->ks + 8;
-  const size_t row = std::max(static_cast<size_t>(p->stride) * 2,
-                              static_cast<size_t>(grm::mla::kEntryPlanes) * grm::mla::kBatchWaves * 4);
-  int qp = grm::mla::kBatchMaxCols;
-  while (qp >= 32 && static_cast<size_t>(qp) * row > a->lds_max) qp /= 2;
-  if (qp < 32) return false;
-  // the merge holds kMergePer sub-streams (screen wavefronts) per thread
-  if (static_cast<size_t>(a->cus) * grm::mla::kBatchWaves >
-      static_cast<size_t>(grm::mla::kMergeLoaders) * grm::mla::kMergePer) {
-    return false;
+  if (q_timed < a->batch_min) return false;
+  const uint32_t per_step = a->dtype == kF32 ? 4 : 2;  // chunks
+  p->ks = static_cast<int>((a->chunks + per_step - 1) / per_step);
+  // the steps in flight that pad the row least, the most of those
+  int best = 0;
+  for (int c : {18, 16, 12, 9, 8, 6, 4}) {
+    if (a->dtype == kF32 ? c > 9 : (c == 9 || c == 6)) continue;
+    const int padded = (p->ks + c - 1) / c * c;
+    if (best == 0 || padded < best) {
+      best = padded;
+      p->p = c;
+    }
   }
-  if (a->dim > grm::mla::kBatchMaxDim) return false;
+  p->nb = best / p->p;
+  int qp = grm::mla::kStreamMaxCols;
+  while (qp >= 32 && stream_lds(a, *p, qp) > a->lds_max) qp /= 2;
+  if (qp < 32) return false;
+  p->qp_stream = qp;
+  // the merge holds kMergePer sub-streams (screen wavefronts) per thread
+  const uint32_t waves = a->cus * grm::mla::kBatchWaves;
+  if (waves > static_cast<uint32_t>(grm::mla::kMergeLoaders) * grm::mla::kMergePer) return false;
   const uint32_t n_tiles32 = static_cast<uint32_t>((a->high_water + 31) / 32);
+  if (n_tiles32 == 0) return false;
   auto code_bits = [&](uint32_t n_sub) {
     const uint32_t max_run = (n_tiles32 + n_sub - 1) / n_sub;
     int ibits = 5;
     while ((1u << (ibits - 5)) < max_run) ++ibits;
     return ibits;
   };
-  const int ibits = code_bits(static_cast<uint32_t>(a->cus) * grm::mla::kBatchWaves);
-  if (ibits > kMaxSlotCodeBits) return false;
-  p->ibits = ibits;
-  p->qp_max = qp;
-  p->ibits_ring = code_bits(static_cast<uint32_t>(a->cus));
-  p->ring = a->ring && qp == grm::mla::kRingQueries && p->ibits_ring <= kMaxSlotCodeBits &&
-            grm::mla::RingShape<18>::kLds <= a->lds_max;
+  p->subs = std::min(waves, n_tiles32);
+  p->ibits = code_bits(p->subs);
+  if (p->ibits > kMaxSlotCodeBits) return false;
+  p->ks_ring = p->ks <= 8 ? 8 : (p->ks <= 16 ? 16 : (p->ks <= 18 ? 18 : 0));
+  p->ibits_ring = code_bits(a->cus);
+  p->ring = a->ring && a->dtype == kBF16 && qp == grm::mla::kStreamMaxCols && p->ks_ring != 0 && a->planes >= 2u * p->ks_ring &&
+            p->ibits_ring <= kMaxSlotCodeBits && grm::mla::RingShape<18>::kLds <= a->lds_max;
+  p->qp_max = p->ring ? grm::mla::kRingQueries : qp;
   return true;
 }
 
-// A pass of ct column tiles runs on the ring screen when the plan allows
-// it and the pass is full (more than 128 queries, padded to 256).
-bool ring_pass(const BatchPlan& p, int ct) { return p.ring && ct == 8; }
-uint32_t pass_subs(const MlaDeviceArena* a, const BatchPlan& p, int ct) {
-  return static_cast<uint32_t>(a->cus) * (ring_pass(p, ct) ? 1u : static_cast<uint32_t>(grm::mla::kBatchWaves));
+// One pass of qc queries: on the ring screen when the plan has it and the
+// pass holds more than 128 queries (padded to 256).
+struct PassShape {
+  bool ring;
+  int qp;          // columns
+  uint32_t subs;   // sub-streams
+  int ibits;
+};
+PassShape pass_shape(const MlaDeviceArena* a, const BatchPlan& p, int qc) {
+  if (qc > grm::mla::kStreamMaxCols) return {true, grm::mla::kRingQueries, a->cus, p.ibits_ring};
+  return {false, qc <= 32 ? 32 : (qc <= 64 ? 64 : 128), p.subs, p.ibits};
 }
-int pass_ibits(const BatchPlan& p, int ct) { return ring_pass(p, ct) ? p.ibits_ring : p.ibits; }
 
 // The ring screen's slot weights, formed again when the bank changed.
 int ensure_weights(MlaDeviceArena* a) {
@@ -837,7 +858,8 @@ int ensure_weights(MlaDeviceArena* a) {
 }
 
 template <int KS, bool kProbe = false>
-int launch_ring(MlaDeviceArena* a, uint32_t n_tiles32, int ibits, uint32_t* planes) {
+int launch_ring(MlaDeviceArena* a, uint32_t n_tiles32, int ibits, uint32_t* planes,
+                unsigned long long* tick) {
   using RS = grm::mla::RingShape<KS>;
   auto kern = grm::mla::mla_batch_ring_kernel<KS, kProbe>;
   GRM_CHECK_RC(ensure_weights(a));
@@ -845,90 +867,137 @@ int launch_ring(MlaDeviceArena* a, uint32_t n_tiles32, int ibits, uint32_t* plan
                                     hipFuncAttributeMaxDynamicSharedMemorySize,
                                     static_cast<int>(RS::kLds)));
   kern<<<a->cus, grm::mla::kRingWaves * grm::kWave, RS::kLds, a->stream>>>(
-      a->d_tiles, a->d_winv, a->capacity, n_tiles32, a->d_qpad, ibits, planes);
+      a->d_tiles, a->d_winv, a->capacity, n_tiles32, a->d_qpad, ibits, planes, tick);
   GRM_HIP_CHECK(hipGetLastError());
   return 0;
 }
 
-template <int KS, int CT, bool kProbe = false>
-int launch_screen(MlaDeviceArena* a, uint32_t n_tiles32, int stride, int ibits, size_t lds,
-                  uint32_t* planes) {
-  auto kern = grm::mla::mla_batch_screen_kernel<KS, CT, kProbe>;
+// A pass's queries (device) and what its kernels report on the way.
+struct PassQueries {
+  const void* q;
+  int dtype;
+  int count;
+};
+struct PassMarks {
+  grm::RouteStamps start{nullptr, nullptr};    // the route's first timed kernel
+  unsigned long long* screen_tick = nullptr;   // [screen start, merge start]
+  hipEvent_t* ev = nullptr;                    // events around the screen kernel
+};
+
+template <int DT, int P, int CT, bool kProbe>
+int launch_stream(MlaDeviceArena* a, const BatchPlan& p, const PassQueries& q, uint32_t* planes,
+                  const PassMarks& m) {
+  auto kern = grm::mla::mla_batch_stream_kernel<DT, P, CT, kProbe>;
+  const size_t lds = stream_lds(a, p, 32 * CT);
   if (lds > 65536) {
     GRM_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                       hipFuncAttributeMaxDynamicSharedMemorySize,
                                       static_cast<int>(lds)));
   }
+  const uint32_t n_tiles32 = static_cast<uint32_t>((a->high_water + 31) / 32);
   kern<<<a->cus, grm::mla::kBatchWaves * grm::kWave, lds, a->stream>>>(
-      a->d_tiles, a->d_norms, a->capacity, a->chunks, n_tiles32, a->d_qpad, stride, ibits, planes);
+      a->d_tiles, a->d_norms, a->capacity, a->chunks, n_tiles32, p.subs,
+      static_cast<uint32_t>(p.nb), static_cast<uint32_t>(p.ks), q.q, q.dtype, q.count, a->dim,
+      a->d_inv_qn, p.ibits, planes, m.start, a->route_seq, m.screen_tick);
   GRM_HIP_CHECK(hipGetLastError());
   return 0;
 }
 
+template <int DT, int P, bool kProbe>
+int launch_stream_ct(MlaDeviceArena* a, const BatchPlan& p, int qp, const PassQueries& q,
+                     uint32_t* planes, const PassMarks& m) {
+  if (qp == 32) return launch_stream<DT, P, 1, kProbe>(a, p, q, planes, m);
+  if (qp == 64) return launch_stream<DT, P, 2, kProbe>(a, p, q, planes, m);
+  return launch_stream<DT, P, 4, kProbe>(a, p, q, planes, m);
+}
+
+// The screen of one pass, its queries prepared first where the screen does
+// not do so itself.
 template <bool kProbe>
-int dispatch_screen(MlaDeviceArena* a, const BatchPlan& p, int ct, uint32_t n_tiles32, size_t lds,
-                    uint32_t* planes) {
-  if (ring_pass(p, ct)) {
-    switch (p.ks) {
-      case 8: return launch_ring<8, kProbe>(a, n_tiles32, p.ibits_ring, planes);
-      case 16: return launch_ring<16, kProbe>(a, n_tiles32, p.ibits_ring, planes);
-      default: return launch_ring<18, kProbe>(a, n_tiles32, p.ibits_ring, planes);
+int launch_screen(MlaDeviceArena* a, const BatchPlan& p, const PassShape& s, const PassQueries& q,
+                  uint32_t* planes, const PassMarks& m) {
+  if (s.ring) {
+    grm::mla::mla_batch_qprep_kernel<<<s.qp, grm::kWave, 0, a->stream>>>(
+        q.q, q.dtype, q.count, a->dim, 16 * p.ks_ring + 8, a->d_qpad, a->d_inv_qn, m.start,
+        a->route_seq);
+    GRM_HIP_CHECK(hipGetLastError());
+  }
+  if (m.ev) GRM_HIP_CHECK(hipEventRecord(m.ev[0], a->stream));
+  int rc = 0;
+  if (s.ring) {
+    const uint32_t n_tiles32 = static_cast<uint32_t>((a->high_water + 31) / 32);
+    switch (p.ks_ring) {
+      case 8: rc = launch_ring<8, kProbe>(a, n_tiles32, s.ibits, planes, m.screen_tick); break;
+      case 16: rc = launch_ring<16, kProbe>(a, n_tiles32, s.ibits, planes, m.screen_tick); break;
+      default: rc = launch_ring<18, kProbe>(a, n_tiles32, s.ibits, planes, m.screen_tick); break;
+    }
+  } else if (a->dtype == kF32) {
+    switch (p.p) {
+      case 9: rc = launch_stream_ct<kF32, 9, kProbe>(a, p, s.qp, q, planes, m); break;
+      case 8: rc = launch_stream_ct<kF32, 8, kProbe>(a, p, s.qp, q, planes, m); break;
+      case 6: rc = launch_stream_ct<kF32, 6, kProbe>(a, p, s.qp, q, planes, m); break;
+      default: rc = launch_stream_ct<kF32, 4, kProbe>(a, p, s.qp, q, planes, m); break;
+    }
+  } else {
+    switch (p.p) {
+      case 18: rc = launch_stream_ct<kBF16, 18, kProbe>(a, p, s.qp, q, planes, m); break;
+      case 16: rc = launch_stream_ct<kBF16, 16, kProbe>(a, p, s.qp, q, planes, m); break;
+      case 12: rc = launch_stream_ct<kBF16, 12, kProbe>(a, p, s.qp, q, planes, m); break;
+      case 8: rc = launch_stream_ct<kBF16, 8, kProbe>(a, p, s.qp, q, planes, m); break;
+      default: rc = launch_stream_ct<kBF16, 4, kProbe>(a, p, s.qp, q, planes, m); break;
     }
   }
-  const int ibits = p.ibits;
-#define GRM_SCREEN_CT(KS)                                                                        \
-  switch (ct) {                                                                                  \
-    case 1: return launch_screen<KS, 1, kProbe>(a, n_tiles32, p.stride, ibits, lds, planes);     \
-    case 2: return launch_screen<KS, 2, kProbe>(a, n_tiles32, p.stride, ibits, lds, planes);     \
-    case 4: return launch_screen<KS, 4, kProbe>(a, n_tiles32, p.stride, ibits, lds, planes);     \
-    default: return launch_screen<KS, 8, kProbe>(a, n_tiles32, p.stride, ibits, lds, planes);    \
-  }
-  switch (p.ks) {
-    case 8: GRM_SCREEN_CT(8);
-    case 16: GRM_SCREEN_CT(16);
-    default: GRM_SCREEN_CT(18);
-  }
-#undef GRM_SCREEN_CT
+  GRM_CHECK_RC(rc);
+  if (m.ev) GRM_HIP_CHECK(hipEventRecord(m.ev[1], a->stream));
+  return 0;
 }
 
-// Screen-bound constants: gamma bounds the fp32 accumulation of 16*ks
-// products in 32x32x16 steps (with the MFMA's internal order unknown),
-// delta the rounding of an fp32 query to bf16.
-double batch_gamma(const BatchPlan& p) { return 2.0 * (16.0 * p.ks + 2.0 * p.ks) * ldexp(1.0, -24); }
-double batch_delta(int q_dtype) { return q_dtype == kF32 ? ldexp(1.0, -8) : 0.0; }
-
-// LDS of a screen pass of qp queries: the staged queries, later the
-// block's result rows.
-size_t batch_lds(const BatchPlan& p, int qp) {
-  return std::max(static_cast<size_t>(qp) * p.stride * 2,
-                  static_cast<size_t>(grm::mla::kEntryPlanes) * qp * grm::mla::kBatchWaves * 4);
+// What the screen's bound rests on: gamma bounds the fp32 accumulation of
+// 16*ks products per product term in 32x32x16 steps (with the MFMA's
+// internal order unknown), delta what the bf16 operands leave out.
+grm::mla::ScreenBound screen_bound(const MlaDeviceArena* a, const BatchPlan& p, int ibits) {
+  grm::mla::ScreenBound b;
+  const bool split = a->dtype == kF32;
+  b.gamma = 2.0 * 18.0 * p.ks * ldexp(1.0, -24);
+  if (split) b.gamma *= 3.0 * (1.0 + ldexp(1.0, -6));
+  b.delta = split ? ldexp(1.0, -16) : -1.0;
+  b.absm = split ? 4.0 : 1.0;
+  b.dim = a->dim;
+  b.ibits = ibits;
+  return b;
 }
 
-// One pass: queries [0, qc) at q (device, dim values each) through the
-// screen and the merge; results at out[0, qc*topk), certificates at
-// status[0, qc).  ev (optional) is a pair of events recorded around the
-// screen kernel.
-int enqueue_batch_pass(MlaDeviceArena* a, const BatchPlan& p, const unsigned char* q, int q_dtype,
-                       int qc, int topk, Cand* out, unsigned* status, hipEvent_t* ev) {
-  const int ct = qc <= 32 ? 1 : (qc <= 64 ? 2 : (qc <= 128 ? 4 : 8));
-  const int qp = 32 * ct;
-  grm::mla::mla_batch_qprep_kernel<<<qp, grm::kWave, 0, a->stream>>>(
-      q, q_dtype, qc, a->dim, p.stride, a->d_qpad, a->d_inv_qn);
-  GRM_HIP_CHECK(hipGetLastError());
+// One pass: the screen and the merge of queries q; results at
+// out[0, count*topk), with done their completion flags (and end ticks).
+int enqueue_batch_pass(MlaDeviceArena* a, const BatchPlan& p, const PassQueries& q, int topk,
+                       Cand* out, unsigned* done, unsigned long long* end_tick, const PassMarks& m) {
+  const PassShape s = pass_shape(a, p, q.count);
+  GRM_CHECK_RC(launch_screen<false>(a, p, s, q, a->d_entries, m));
   const uint32_t n_tiles32 = static_cast<uint32_t>((a->high_water + 31) / 32);
-  const uint32_t n_waves = pass_subs(a, p, ct);
-  const int ibits = pass_ibits(p, ct);
-  const size_t lds = batch_lds(p, qp);
-  if (ev) GRM_HIP_CHECK(hipEventRecord(ev[0], a->stream));
-  GRM_CHECK_RC(dispatch_screen<false>(a, p, ct, n_tiles32, lds, a->d_entries));
-  if (ev) GRM_HIP_CHECK(hipEventRecord(ev[1], a->stream));
-  const double gamma = batch_gamma(p);
-  const double delta = batch_delta(q_dtype);
-  grm::mla::mla_batch_merge_kernel<<<qc, grm::mla::kMergeThreads, 0, a->stream>>>(
-      a->d_entries, n_waves, qp, n_tiles32, ibits, a->d_inv_qn, a->d_tiles, a->d_norms, a->d_ids,
-      a->capacity, a->dim, q, q_dtype, a->dim, gamma, delta, a->d_min_norm, topk, out, status);
+  auto kern = a->dtype == kF32 ? grm::mla::mla_batch_merge_kernel<kF32>
+                               : grm::mla::mla_batch_merge_kernel<kBF16>;
+  const size_t lds = grm::mla::merge_query_len(a->chunks, a->epc) * sizeof(double);
+  kern<<<q.count, grm::mla::kMergeThreads, lds, a->stream>>>(
+      a->d_entries, s.subs, s.qp, n_tiles32, a->d_inv_qn, a->d_tiles, a->d_norms, a->d_ids,
+      a->capacity, a->chunks, q.q, q.dtype, a->dim, screen_bound(a, p, s.ibits),
+      a->d_min_norm, topk, out, done, a->route_seq, end_tick,
+      m.screen_tick ? m.screen_tick + 1 : nullptr);
   GRM_HIP_CHECK(hipGetLastError());
   return 0;
+}
+
+// Buffers of the batched route.  False when the device has no room for
+// them: the queries then go one by one.
+bool reserve_batch(MlaDeviceArena* a, const BatchPlan& p) {
+  const size_t cols = std::max(p.qp_stream, p.qp_max);
+  const size_t subs = std::max(p.subs * static_cast<size_t>(p.qp_stream),
+                               p.ring ? a->cus * static_cast<size_t>(p.qp_max) : size_t{0});
+  const bool ok =
+      (!p.ring || reserve_device(&a->d_qpad, &a->d_qpad_count, cols * (16 * p.ks_ring + 8)) == 0) &&
+      reserve_device(&a->d_inv_qn, &a->d_inv_qn_count, cols) == 0 &&
+      reserve_device(&a->d_entries, &a->d_entries_count, grm::mla::kEntryPlanes * subs) == 0;
+  if (!ok) (void)hipGetLastError();
+  return ok;
 }
 
 // Completion flags a route may wait on (one per query and route block).
@@ -968,51 +1037,97 @@ int route_impl(MlaDeviceArena* a, const void* queries, int q_dtype,
   if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->ev_mut, 0));
   const size_t qstride = static_cast<size_t>(a->dim) * elem_size(q_dtype);
   BatchPlan bp;
-  const bool batched = !a->no_batch && batch_plan(a, q_count - warmup, &bp);
+  const bool batched = !a->no_batch && batch_plan(a, q_count - warmup, &bp) && reserve_batch(a, bp);
   a->screen_ms = 0.0f;
   std::vector<int> redo;  // queries for the single-query kernel
   if (batched) {
-    GRM_CHECK_RC(reserve_device(&a->d_qpad, &a->d_qpad_count, static_cast<size_t>(bp.qp_max) * bp.stride));
-    GRM_CHECK_RC(reserve_device(&a->d_inv_qn, &a->d_inv_qn_count, static_cast<size_t>(bp.qp_max)));
-    GRM_CHECK_RC(reserve_device(&a->d_entries, &a->d_entries_count,
-                                static_cast<size_t>(grm::mla::kEntryPlanes) * bp.qp_max * a->cus *
-                                    grm::mla::kBatchWaves));
     GRM_CHECK_RC(grm::reserve_mapped(&a->batch_out, static_cast<size_t>(q_count) * topk));
-    GRM_CHECK_RC(grm::reserve_mapped_bytes(&a->batch_status, static_cast<size_t>(q_count) * sizeof(unsigned)));
-    unsigned* st = static_cast<unsigned*>(a->batch_status.dev);
-    const int timed_passes = (q_count - warmup + bp.qp_max - 1) / bp.qp_max;
-    while (a->screen_ev.size() < 2 * static_cast<size_t>(timed_passes)) {
-      hipEvent_t e = nullptr;
-      GRM_HIP_CHECK(hipEventCreate(&e));
-      a->screen_ev.push_back(e);
-    }
     const int segments[2][2] = {{0, warmup}, {warmup, q_count}};
+    // Completion as for single queries (below): a flag per query, the
+    // times on the device clock; stream events where those cannot serve.
+    const size_t n_q = static_cast<size_t>(q_count);
+    const bool flags = n_q <= kMaxDoneFlags && !grm::blocking_sync() && a->ticks_per_ms > 0.0 &&
+                       !(elapsed_ms && grm::event_timing());
+    const int timed_passes = (q_count - warmup + bp.qp_max - 1) / bp.qp_max;
+    unsigned* d_done = nullptr;
+    if (flags) {
+      GRM_CHECK_RC(grm::begin_flags(&a->done_flags, kMaxDoneFlags, &a->route_seq));
+      GRM_CHECK_RC(grm::reserve_stamps(&a->stamps, kMaxDoneFlags));
+      if (a->screen_ticks.bytes < 16 * static_cast<size_t>(timed_passes)) {
+        const size_t bytes = 16 * static_cast<size_t>(timed_passes);
+        GRM_CHECK_RC(grm::reserve_mapped_bytes(&a->screen_ticks, bytes));
+        memset(a->screen_ticks.host, 0, bytes);
+      }
+      d_done = static_cast<unsigned*>(a->done_flags.dev);
+    } else {
+      while (a->screen_ev.size() < 2 * static_cast<size_t>(timed_passes)) {
+        hipEvent_t e = nullptr;
+        GRM_HIP_CHECK(hipEventCreate(&e));
+        a->screen_ev.push_back(e);
+      }
+    }
     int tp = 0;
     for (int si = 0; si < 2; ++si) {
-      if (si == 1) GRM_HIP_CHECK(hipEventRecord(a->ev_start, a->stream));
+      if (si == 1 && !flags) GRM_HIP_CHECK(hipEventRecord(a->ev_start, a->stream));
       for (int q0 = segments[si][0]; q0 < segments[si][1]; q0 += bp.qp_max) {
-        const int qc = std::min(bp.qp_max, segments[si][1] - q0);
-        hipEvent_t* ev = si == 1 ? &a->screen_ev[2 * tp++] : nullptr;
-        GRM_CHECK_RC(enqueue_batch_pass(a, bp, qbase + q0 * qstride, q_dtype, qc, topk,
-                                        a->batch_out.dev + static_cast<size_t>(q0) * topk, st + q0,
-                                        ev));
+        const PassQueries pq{qbase + q0 * qstride, q_dtype, std::min(bp.qp_max, segments[si][1] - q0)};
+        PassMarks m;
+        unsigned long long* end_tick = nullptr;
+        if (flags) {
+          const grm::RouteStamps st = grm::route_stamps(a->stamps, static_cast<size_t>(q0));
+          if (si == 1 && q0 == warmup) m.start.start = st.start;
+          end_tick = st.end;
+        }
+        if (si == 1) {
+          if (flags) {
+            m.screen_tick = static_cast<unsigned long long*>(a->screen_ticks.dev) + 2 * tp;
+          } else {
+            m.ev = &a->screen_ev[2 * tp];
+          }
+          ++tp;
+        }
+        GRM_CHECK_RC(enqueue_batch_pass(a, bp, pq, topk,
+                                        a->batch_out.dev + static_cast<size_t>(q0) * topk,
+                                        d_done ? d_done + q0 : nullptr, end_tick, m));
         a->batch_passes += 1;
       }
     }
     GRM_HIP_CHECK(hipEventRecord(a->ev_stop, a->stream));
-    GRM_CHECK_RC(grm::wait_event(a->ev_stop));
-    if (elapsed_ms) GRM_HIP_CHECK(hipEventElapsedTime(elapsed_ms, a->ev_start, a->ev_stop));
     a->screen_ms = 0.0f;
-    for (int i = 0; i < tp; ++i) {
+    if (flags) {
+      GRM_CHECK_RC(grm::wait_flags(a->done_flags, a->route_seq, n_q, a->ev_stop));
+      GRM_CHECK_RC(grm::wait_tagged(a->batch_out.host, n_q * topk, a->route_seq, a->ev_stop));
       float ms = 0.0f;
-      GRM_HIP_CHECK(hipEventElapsedTime(&ms, a->screen_ev[2 * i], a->screen_ev[2 * i + 1]));
-      a->screen_ms += ms;
+      GRM_CHECK_RC(grm::stamps_elapsed(a->stamps, a->route_seq, static_cast<size_t>(warmup), n_q,
+                                       a->ev_stop, a->ticks_per_ms, &ms));
+      if (elapsed_ms) *elapsed_ms = ms;
+      // a pass's screen ends where its merge starts; both ticks lie after
+      // the route's start (grm::stamps_elapsed has seen that stamp)
+      const volatile unsigned long long* tick =
+          static_cast<const volatile unsigned long long*>(a->screen_ticks.host);
+      const unsigned long long t0 = *static_cast<const volatile unsigned long long*>(a->stamps.host);
+      for (int i = 0; i < 2 * tp; ++i) {
+        if (tick[i] >= t0) continue;
+        GRM_CHECK_RC(grm::wait_event(a->ev_stop));
+        std::atomic_thread_fence(std::memory_order_acquire);
+        break;
+      }
+      for (int i = 0; i < tp; ++i) {
+        a->screen_ms += static_cast<float>(static_cast<double>(tick[2 * i + 1] - tick[2 * i]) / a->ticks_per_ms);
+      }
+    } else {
+      GRM_CHECK_RC(grm::wait_event(a->ev_stop));
+      if (elapsed_ms) GRM_HIP_CHECK(hipEventElapsedTime(elapsed_ms, a->ev_start, a->ev_stop));
+      for (int i = 0; i < tp; ++i) {
+        float ms = 0.0f;
+        GRM_HIP_CHECK(hipEventElapsedTime(&ms, a->screen_ev[2 * i], a->screen_ev[2 * i + 1]));
+        a->screen_ms += ms;
+      }
     }
-    const unsigned* hs = static_cast<const unsigned*>(a->batch_status.host);
     for (int qi = 0; qi < q_count; ++qi) {
-      if (hs[qi] == 1u) {
-        write_cands(a->batch_out.host + static_cast<size_t>(qi) * topk, topk,
-                    out_ids + static_cast<size_t>(qi) * topk,
+      const Cand* c = a->batch_out.host + static_cast<size_t>(qi) * topk;
+      if (c->id != kNoId) {
+        write_cands(c, topk, out_ids + static_cast<size_t>(qi) * topk,
                     out_scores ? out_scores + static_cast<size_t>(qi) * topk : nullptr);
       } else {
         redo.push_back(qi);
@@ -1832,7 +1947,7 @@ extern "C" int grm_mla_hip_screen_ms(MlaDeviceArena* a, float* ms) {
 // ------------------------------------------------------- screen-bound probe
 //
 // Test entry: runs the batched route's screen (the same kernel, in its
-// probe form) over every slot of a small bf16 bank and returns each
+// probe form) over every slot of a small bank and returns each
 // screened score s~ with its query's bound B, so a test can hold
 // |s~ - law score| <= B for every (query, node) pair.  Not on any route
 // path; allocates its own buffers.
@@ -1845,11 +1960,11 @@ extern "C" int grm_mla_hip_probe_screen(MlaDeviceArena* a, const void* queries_h
   if (query_dtype != kF32 && query_dtype != kBF16) return grm::fail(-1, "query dtype must be F32 or BF16");
   BatchPlan p;
   if (!batch_plan(a, std::numeric_limits<int>::max(), &p)) {
-    return grm::fail(-1, "bank has no batched screen (bf16 rows, dim <= 288)");
+    return grm::fail(-1, "bank has no batched screen (rows too long or too many)");
   }
   if (query_count <= 0 || query_count > p.qp_max) return grm::fail(-1, "query_count out of range");
-  const int ct = query_count <= 32 ? 1 : (query_count <= 64 ? 2 : (query_count <= 128 ? 4 : 8));
-  const int qp = 32 * ct;
+  const PassShape shape = pass_shape(a, p, query_count);
+  const int qp = shape.qp;
   const uint64_t n = a->high_water;
   if (n == 0) return grm::fail(-1, "empty bank");
   if (a->capacity * static_cast<uint64_t>(qp) > (1ull << 26)) {
@@ -1867,20 +1982,16 @@ extern "C" int grm_mla_hip_probe_screen(MlaDeviceArena* a, const void* queries_h
   GRM_HIP_CHECK(hipMalloc(&d_planes.p, static_cast<size_t>(qp) * a->capacity * sizeof(uint32_t)));
   GRM_HIP_CHECK(hipMalloc(&d_vals.p, static_cast<size_t>(query_count) * n * sizeof(float)));
   GRM_HIP_CHECK(hipMalloc(&d_bounds.p, static_cast<size_t>(query_count) * sizeof(double)));
-  GRM_CHECK_RC(reserve_device(&a->d_qpad, &a->d_qpad_count, static_cast<size_t>(p.qp_max) * p.stride));
-  GRM_CHECK_RC(reserve_device(&a->d_inv_qn, &a->d_inv_qn_count, static_cast<size_t>(p.qp_max)));
+  if (!reserve_batch(a, p)) return grm::fail(-1, "no memory for the probe's buffers");
   if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->ev_mut, 0));
   GRM_HIP_CHECK(hipMemcpyAsync(d_q.p, queries_host, qbytes, hipMemcpyHostToDevice, a->stream));
-  grm::mla::mla_batch_qprep_kernel<<<qp, grm::kWave, 0, a->stream>>>(
-      d_q.p, query_dtype, query_count, a->dim, p.stride, a->d_qpad, a->d_inv_qn);
-  GRM_HIP_CHECK(hipGetLastError());
-  const uint32_t n_tiles32 = static_cast<uint32_t>((n + 31) / 32);
-  GRM_CHECK_RC(dispatch_screen<true>(a, p, ct, n_tiles32, batch_lds(p, qp),
-                                     static_cast<uint32_t*>(d_planes.p)));
-  grm::mla::mla_batch_probe_finish_kernel<<<query_count, grm::kWave, 0, a->stream>>>(
+  const PassQueries pq{d_q.p, query_dtype, query_count};
+  GRM_CHECK_RC(launch_screen<true>(a, p, shape, pq, static_cast<uint32_t*>(d_planes.p), PassMarks{}));
+  const uint32_t len = grm::mla::merge_query_len(a->chunks, a->epc);
+  grm::mla::mla_batch_probe_finish_kernel<<<query_count, grm::kWave, len * sizeof(double), a->stream>>>(
       static_cast<const uint32_t*>(d_planes.p), a->capacity, static_cast<uint32_t>(n), a->d_inv_qn,
-      d_q.p, query_dtype, a->dim, a->dim, batch_gamma(p), batch_delta(query_dtype), a->d_min_norm,
-      pass_ibits(p, ct), static_cast<float*>(d_vals.p), static_cast<double*>(d_bounds.p));
+      d_q.p, query_dtype, a->dim, len, screen_bound(a, p, shape.ibits), a->d_min_norm,
+      static_cast<float*>(d_vals.p), static_cast<double*>(d_bounds.p));
   GRM_HIP_CHECK(hipGetLastError());
   GRM_HIP_CHECK(hipMemcpyAsync(out_values_host, d_vals.p, static_cast<size_t>(query_count) * n * sizeof(float),
                                hipMemcpyDeviceToHost, a->stream));
