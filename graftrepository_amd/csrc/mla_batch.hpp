@@ -67,10 +67,11 @@ constexpr int kEntryPlanes = 3;      // u1, u2, nk
 //   u1, u2  the two best u a sub-stream kept (float bits, slot code in
 //   the low ibits bits), nk the largest u it did not keep.
 //
-// Slot code of a value: (half << (ibits - 1)) | ((t - t_begin) << 4) | r
-// for result register r of lane half `half` in tile t of a sub-stream
-// whose tiles start at t_begin; ibits - 5 bits hold the tile offset, so
-// the host picks ibits from the longest run of tiles a sub-stream walks.
+// Slot code of a value: ((t - t_begin) << 4) | r for result register r in
+// tile t of a sub-stream whose tiles start at t_begin, in the stream screen
+// with the lane half at bit ibits - 1 (the ring screen's halves are
+// sub-streams of their own).  The host picks ibits from the longest run of
+// tiles a sub-stream walks.
 // Writing the code moves u by less than 2^(ibits-23) |u| (2^(ibits-149)
 // near zero), which the merge adds to B.
 
@@ -363,10 +364,16 @@ __global__ __launch_bounds__(kBatchWaves * kWave) void mla_batch_stream_kernel(
 //    straight-line region, each MFMA followed by its share of the
 //    reductions and a scheduling barrier: the matrix core and the VALU work
 //    side by side within the wavefront.
-//  * Block b is sub-stream b of W = blocks and walks tiles
-//    [b * n_tiles32 / W, (b + 1) * n_tiles32 / W), one per step, so the
-//    merge decodes its slot codes as for the wavefront sub-streams of
-//    mla_batch_stream_kernel.
+//  * Block b of W walks tiles [b * n_tiles32 / W, (b + 1) * n_tiles32 / W),
+//    one per step, as kRingSegs runs: run j = kRingSegs b + g starts at
+//    j * n_tiles32 / (kRingSegs W).  Each lane starts its lists afresh at a
+//    run's first tile and keeps the finished ones in registers, so
+//    sub-stream (2 b + half) kRingSegs + g is run j as seen by one lane
+//    half, and its slot code has no half bit.  With one sub-stream per
+//    block, three of a query's best rows in one of 256 sub-streams sent 0.3
+//    (k = 8) to 2.7 (k = 16) of 256 queries to the exact kernel, 100 us
+//    each at 1M x 288; with 2,048 about one call in a hundred has one, and
+//    the shorter code tightens the bound (2^-14 instead of 2^-11).
 //  * A ring of kRing tiles in LDS (2 KS chunk planes of 512 bytes each,
 //    chunk c of the tile at c * 512) with their 32 slot weights.  Direct
 //    loads (global_load_lds_dwordx4) fill it without registers.  A step is
@@ -396,6 +403,7 @@ struct RingShape {
 };
 
 constexpr int kRingWaves = 4;      // wavefronts per block, one block per CU
+constexpr int kRingSegs = 4;       // runs of tiles with lists of their own, per block
 constexpr int kRingQueries = 256;  // queries per ring pass
 
 // s_waitcnt vmcnt(n) lgkmcnt(0) (gfx9 encoding; expcnt left alone): the
@@ -506,6 +514,7 @@ __global__ __launch_bounds__(kRingWaves * kWave, 1) void mla_batch_ring_kernel(
     uint32_t t;
     uint32_t tcode;
   };
+  uint32_t base = 0;  // first step of the run in progress
   // Reduction of value v = 16 c + r of a finished tile.
   auto reduce_one = [&](const Res& R, int v) {
     const int c = v >> 4;
@@ -545,7 +554,7 @@ __global__ __launch_bounds__(kRingWaves * kWave, 1) void mla_batch_ring_kernel(
       R.w[4 * i + 3] = __uint_as_float(w4.w);
     }
     R.t = t_begin + s;
-    R.tcode = (static_cast<uint32_t>(half) << (ibits - 1)) | (s << 4);
+    R.tcode = (s - base) << 4;
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
@@ -574,54 +583,87 @@ __global__ __launch_bounds__(kRingWaves * kWave, 1) void mla_batch_ring_kernel(
     for (int v = 0; v < 32; ++v) reduce_one(R, v);
   };
 
+  // Lists of the finished runs, the latest last.
+  int done[kRingSegs - 1][2][3];
+#pragma unroll
+  for (int g = 0; g < kRingSegs - 1; ++g) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) done[g][c][0] = done[g][c][1] = done[g][c][2] = INT32_MIN;
+  }
+  auto next_run = [&]() {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+      for (int g = 0; g + 1 < kRingSegs - 1; ++g) {
+#pragma unroll
+        for (int x = 0; x < 3; ++x) done[g][c][x] = done[g + 1][c][x];
+      }
+      done[kRingSegs - 2][c][0] = b1[c];
+      done[kRingSegs - 2][c][1] = b2[c];
+      done[kRingSegs - 2][c][2] = b3[c];
+      b1[c] = b2[c] = b3[c] = INT32_MIN;
+    }
+  };
+  // first step of run g
+  auto run_start = [&](uint32_t g) -> uint32_t {
+    return static_cast<uint32_t>(static_cast<uint64_t>(blockIdx.x * kRingSegs + g) * n_tiles32 /
+                                 (static_cast<uint64_t>(W) * kRingSegs)) - t_begin;
+  };
+  uint32_t run = 0, next = run_start(1);  // next: first step of run + 1
+  // Step s, whose reductions are those of tile s - 1: a run that starts at
+  // step s (or empty runs before it) takes over once they are in.
+  auto step = [&](uint32_t s, Res& R, const Res& P, auto has_prev) {
+    const bool turn = run + 1 < kRingSegs && s == next;
+    if (turn) base = s;
+    enter_step(s);
+    step_tile(s, R, P, has_prev);
+    if (turn) {
+      do {
+        next_run();
+        ++run;
+        next = run_start(run + 1);
+      } while (run + 1 < kRingSegs && s == next);
+    }
+  };
   Res RA, RB;
   if (steps > 0) {
 #pragma unroll
     for (int s = 0; s < RS::kRing - 1; ++s) issue_step(static_cast<uint32_t>(s));
-    enter_step(0);
-    step_tile(0, RA, RB, std::false_type{});
+    step(0, RA, RB, std::false_type{});
   }
   uint32_t s = 1;
   for (; s + 1 < steps; s += 2) {
-    enter_step(s);
-    step_tile(s, RB, RA, std::true_type{});
-    enter_step(s + 1);
-    step_tile(s + 1, RA, RB, std::true_type{});
+    step(s, RB, RA, std::true_type{});
+    step(s + 1, RA, RB, std::true_type{});
   }
   if (s < steps) {
-    enter_step(s);
-    step_tile(s, RB, RA, std::true_type{});
+    step(s, RB, RA, std::true_type{});
     reduce_tile(RB);
   } else if (steps > 0) {
     reduce_tile(RA);
   }
+  // runs past the block's last tile are empty
+  for (; run + 1 < kRingSegs; ++run) next_run();
   // no load may still be writing LDS when the block ends
   asm volatile("" ::: "memory");
   wait_vmcnt_lds<0>();
   if constexpr (kProbe) return;
-  // merge the two lane halves (disjoint slots of one query), then one
-  // value per (plane, query, sub-stream)
-  const size_t n_sub = W;
+  // a lane's lists: one 16-byte store per (plane, query)
+  const size_t n_sub = static_cast<size_t>(W) * 2 * kRingSegs;
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    const int o1 = __shfl_xor(b1[c], 32);
-    const int o2 = __shfl_xor(b2[c], 32);
-    const int o3 = __shfl_xor(b3[c], 32);
+    const size_t q = static_cast<size_t>(64 * wv + 32 * c + col);
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const int v = j == 0 ? o1 : (j == 1 ? o2 : o3);
-      med3_i32_into(b2[c], b3[c], v);
-      med3_i32_into(b1[c], b2[c], v);
-      b1[c] = max(b1[c], v);
-    }
-    if (half == 0) {
-      const size_t q = static_cast<size_t>(64 * wv + 32 * c + col);
-      planes[(0 * QP + q) * n_sub + blockIdx.x] = static_cast<uint32_t>(b1[c]);
-      planes[(1 * QP + q) * n_sub + blockIdx.x] = static_cast<uint32_t>(b2[c]);
-      planes[(2 * QP + q) * n_sub + blockIdx.x] = static_cast<uint32_t>(b3[c]);
+    for (int x = 0; x < 3; ++x) {
+      u32x4 v;
+#pragma unroll
+      for (int g = 0; g < kRingSegs - 1; ++g) v[g] = static_cast<uint32_t>(done[g][c][x]);
+      v[kRingSegs - 1] = static_cast<uint32_t>(x == 0 ? b1[c] : (x == 1 ? b2[c] : b3[c]));
+      *reinterpret_cast<u32x4*>(planes + (x * QP + q) * n_sub + (2 * blockIdx.x + half) * kRingSegs) = v;
     }
   }
 }
+static_assert(kRingSegs == 4, "a lane's lists of one kind are one 16-byte store");
 
 // Query rows of one ring pass: qpad[j][0, stride) = query j's
 // values rounded to bf16 (nearest even; bf16 queries are copied), zero past
@@ -673,9 +715,8 @@ __device__ inline float wave_sort_desc(float v) {
 }
 
 // Merge, certificate and exact rescore; grid = one block of kMergeThreads
-// per query of the pass.  planes: the screen's rows (n_sub sub-streams =
-// the screen's wavefronts, QP queries; wavefront i walked tiles from
-// i * n_tiles32 / n_sub); query qi (pass column) has its `dim` values at
+// per query of the pass.  planes: the screen's rows (n_sub sub-streams
+// of the stream or ring screen, QP queries); query qi (pass column) has its `dim` values at
 // query + qi*qstride elements (F32 or BF16) and 1/||q|| at inv_qn[qi].
 // The screened score of a kept value u is s~ = u * inv_qn[qi], its slot
 // the code in u's low ibits bits.  The screen bound for the query
@@ -697,38 +738,83 @@ __device__ inline float wave_sort_desc(float v) {
 // |score| <= 1, and absolute near zero).  qn is the law's query norm and
 // nmin the smallest positive row norm.
 //
-// Steps: the last wavefront stages the query and one of its lanes forms
-// the law's qnorm while the others load the sub-streams' entries.  Each
-// of those wavefronts sorts its lanes' largest kept s~; the largest k-th
-// of those, L, is a lower bound on v_k, so every kept entry at or above t
-// lies at or above L - 2B.  Those entries (at most kSurvMax, else no
-// certificate) are collected in LDS, one thread each: it ranks its entry
-// by (s~ desc, sub-stream asc) and counts the entries above s~ + 2B.
+// Steps: the last wavefront stages the query while the others load the
+// sub-streams' entries and each sort their lanes' largest kept s~; the
+// largest k-th of those, L, is a lower bound on v_k, so every kept entry at
+// or above t lies at or above L - 2B.  Those entries (at most kSurvMax,
+// else no certificate) are collected in LDS, one thread each: it ranks its
+// entry by (s~ desc, sub-stream asc) and counts the entries above s~ + 2B.
 // Fewer than k such entries holds for every entry at or above t (those
 // above it then lie above v_k), so the entries passing that count -- a
 // prefix of the ranking -- form the law's dot products of their rows and
 // are ranked by law score (score desc, node id asc).  Rescoring entries
 // below t as well changes nothing: they are real nodes with law scores.
+//
+// The kernel is a chain of latencies (one block per query), so what can run
+// side by side does: the prefix's rows come in by all threads at once, a
+// chunk each, as doubles (a conversion costs more than its multiply-add),
+// while the last wavefront sums the law's norm; then a lane per row runs
+// the fp64 chain from LDS.  With the norm formed first and a lane loading
+// its row itself, 36 chunks at a time, the kernel took 17.2 us for 32 queries
+// x 100k x 280 fp32 and 25.6 for 256 x 1M x 288 bf16; it takes 14.0 and 21.3.
 // Writes out[qi*k ..) (host mapped): the law's top-k where certified, else
 // k entries without a node (kNoId: route qi again on the exact path).  With
 // `done` the entries carry the route's tag and done[qi] takes its number
 // (store_entry, block_done_flag).
 //
-// Dynamic LDS: the query as doubles, zero past dim up to whole batches of
-// kMergeChunks row chunks (merge_query_len).
-constexpr int kMergeChunks = 36;  // row chunks a rescoring thread has in flight
+// Dynamic LDS: the query as doubles, zero past dim up to whole stages of
+// kMergeStage values (merge_len), then merge_rows rows of as many, merge_pitch
+// apart (an odd number of 16-byte pieces: lanes read distinct banks).
+constexpr uint32_t kMergeStage = 16;
 
-__host__ __device__ inline uint32_t merge_query_len(uint32_t chunks, uint32_t epc) {
-  return (chunks + kMergeChunks - 1) / kMergeChunks * kMergeChunks * epc;
+__host__ __device__ inline uint32_t merge_len(uint32_t dim) {
+  return (dim + kMergeStage - 1) / kMergeStage * kMergeStage;
+}
+__host__ __device__ inline uint32_t merge_pitch(uint32_t dim) { return merge_len(dim) + 2; }
+// Rows staged at once: what fits 64 KiB, at most a wavefront's lanes.
+__host__ __device__ inline uint32_t merge_rows(uint32_t dim) {
+  const uint32_t fit = 65536u / (8u * merge_pitch(dim));
+  return fit < 1u ? 1u : (fit > 64u ? 64u : fit);
+}
+inline size_t merge_lds(uint32_t dim) {
+  return (merge_len(dim) + static_cast<size_t>(merge_rows(dim)) * merge_pitch(dim)) * sizeof(double);
+}
+
+// sum over d of a[d] * b[d], d ascending from 0, one fma each: the serial
+// chain, its values read from LDS a stage ahead.
+__device__ inline double serial_dot(const double* __restrict__ a, const double* __restrict__ b,
+                                    uint32_t len) {
+  constexpr int N = kMergeStage / 2;
+  double x[N], y[N], xn[N], yn[N];
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    x[e] = a[e];
+    y[e] = b[e];
+  }
+  double dot = 0.0;
+  for (uint32_t d = 0; d < len; d += 2 * N) {
+    auto half = [&](double (&p)[N], double (&q)[N], double (&pn)[N], double (&qn)[N], uint32_t ahead) {
+#pragma unroll
+      for (int e = 0; e < N; ++e) {
+        pn[e] = a[ahead + e];
+        qn[e] = b[ahead + e];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int e = 0; e < N; ++e) dot = fma(p[e], q[e], dot);
+    };
+    half(x, y, xn, yn, d + N);
+    half(xn, yn, x, y, d + 2 * N < len ? d + 2 * N : 0);
+  }
+  return dot;
 }
 
 // One wavefront stages query qi (`dim` values, F32 or BF16, qstride elements
-// apart) as doubles in s_q[0, len), zero past dim; its lane 0 returns the
-// law's norm (staged_norm; other lanes 0).  rest takes
-// ||q - bf16(q)||, every lane.
-__device__ inline double stage_query_norm(double* __restrict__ s_q, const void* __restrict__ query,
-                                          int q_dtype, size_t qstride, int qi, uint32_t dim,
-                                          uint32_t len, int lane, double& rest) {
+// apart) as doubles in s_q[0, len), zero past dim, and returns
+// ||q - bf16(q)|| in every lane.
+__device__ inline double stage_row_query(double* __restrict__ s_q, const void* __restrict__ query,
+                                         int q_dtype, size_t qstride, int qi, uint32_t dim,
+                                         uint32_t len, int lane) {
   const unsigned char* qbase = static_cast<const unsigned char*>(query) +
                                static_cast<size_t>(qi) * qstride * (q_dtype == kBF16 ? 2 : 4);
   constexpr int kAhead = 8;
@@ -751,11 +837,10 @@ __device__ inline double stage_query_norm(double* __restrict__ s_q, const void* 
   }
 #pragma unroll
   for (int off = 1; off < kWave; off <<= 1) rr += __shfl_xor(rr, off);
-  rest = sqrt(rr);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  return lane == 0 ? staged_norm(s_q, (dim + 3) / 4 * 4) : 0.0;
+  return sqrt(rr);
 }
 
 // What the screen bound of a pass rests on besides the norms.
@@ -768,8 +853,8 @@ struct ScreenBound {
 };
 
 // The screen bound B of a query (|s~ - score|, see mla_batch_merge_kernel)
-// from the law's query norm qn, rest = ||q - bf16(q)|| and the smallest
-// positive row norm nmin;
+// from the query's norm qn (or less), rest = ||q - bf16(q)|| and the
+// smallest positive row norm nmin;
 // it holds where screen_in_range(qn, nmax).
 __device__ inline double batch_screen_bound(const ScreenBound& b, double qn, double rest, double nmin) {
   const double dim = static_cast<double>(b.dim);
@@ -794,7 +879,7 @@ constexpr int kSurvMax = kMergeThreads;
 
 template <int DT>
 __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
-    const uint32_t* __restrict__ planes, uint32_t n_sub, int QP, uint32_t n_tiles32,
+    const uint32_t* __restrict__ planes, uint32_t n_sub, bool ring, int QP, uint32_t n_tiles32,
     const float* __restrict__ inv_qn, const u32x4* __restrict__ tiles,
     const float* __restrict__ norms, const uint64_t* __restrict__ ids, uint64_t cap,
     uint32_t chunks, const void* __restrict__ query, int q_dtype, size_t qstride, ScreenBound sb,
@@ -803,17 +888,19 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
     unsigned long long* __restrict__ screen_tick) {
   if (screen_tick && blockIdx.x == 0 && threadIdx.x == 0) *screen_tick = wall_clock64();
   constexpr uint32_t EPC = DT == kF32 ? 4 : 8;
-  extern __shared__ double s_q[];           // the query, zero past dim
+  extern __shared__ double s_q[];           // the query, zero past dim; the staged rows
+  double* s_rows = s_q + merge_len(sb.dim);
   __shared__ float s_lw[kMergeWavesB];      // per wavefront: k-th largest lane maximum
   __shared__ float s_nk[kMergeWavesB];      // per wavefront: largest dropped s~
   __shared__ __align__(16) float s_sv[kSurvMax];       // survivors: s~
+  __shared__ float s_su[kSurvMax];                     //   u
   __shared__ __align__(16) uint32_t s_key[kSurvMax];   //   2 * sub-stream + (second kept entry)
-  __shared__ uint32_t s_slot[kSurvMax];
-  __shared__ uint16_t s_byrank[kSurvMax];   // survivor holding each s~ rank
+  __shared__ float s_vrank[kMaxTopK];       // s~ of the k best survivors
+  __shared__ uint32_t s_rslot[kSurvMax];    // slots of the prefix, by rank
   __shared__ float s_es[kSurvMax];          // law scores of the ranked prefix (NaN: not finite)
   __shared__ uint64_t s_eid[kSurvMax];
   __shared__ Cand s_top[kMaxTopK];
-  __shared__ double s_qn, s_rest;
+  __shared__ double s_qn, s_bound, s_qhi;
   __shared__ float s_ek;
   __shared__ unsigned s_count;
   const int tid = threadIdx.x;
@@ -827,67 +914,66 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
   const float* p_nk = p_u2 + plane;
   const float iq = inv_qn[qi];
   const int ibits = sb.ibits;
-  const uint32_t cmask = (1u << ibits) - 1u;
-  // slot of coded value u kept by sub-stream i (see the screen's slot code)
+  // slot of coded value u kept by sub-stream i (see the screens' slot codes)
+  const uint32_t tbits = ring ? ibits - 4 : ibits - 5;
+  const uint32_t runs = ring ? n_sub / 2 : n_sub;
   auto slot_of = [&](float u, uint32_t i) -> uint32_t {
-    const uint32_t c = __float_as_uint(u) & cmask;
-    const uint32_t t_begin = static_cast<uint32_t>(static_cast<uint64_t>(i) * n_tiles32 / n_sub);
+    const uint32_t c = __float_as_uint(u);
+    const uint32_t run = ring ? i / (2 * kRingSegs) * kRingSegs + i % kRingSegs : i;
+    const uint32_t half = ring ? i / kRingSegs % 2 : (c >> (ibits - 1)) & 1u;
+    const uint32_t t_begin = static_cast<uint32_t>(static_cast<uint64_t>(run) * n_tiles32 / runs);
     const uint32_t r = c & 15u;
-    const uint32_t t = t_begin + ((c >> 4) & ((1u << (ibits - 5)) - 1u));
-    const uint32_t slot = t * 32u + 8u * (r >> 2) + 4u * (c >> (ibits - 1)) + (r & 3u);
+    const uint32_t t = t_begin + ((c >> 4) & ((1u << tbits) - 1u));
+    const uint32_t slot = t * 32u + 8u * (r >> 2) + 4u * half + (r & 3u);
     // every code the screen writes names a slot of a tile it walked; the
     // clamp only keeps a corrupted value from reading past the bank
     return slot < cap ? slot : static_cast<uint32_t>(cap - 1);
   };
 
-  float v1[kMergePer], v2[kMergePer];
-  uint32_t j1[kMergePer], j2[kMergePer];
+  float u1[kMergePer], u2[kMergePer];
   float nk = -INFINITY;
 #pragma unroll
   for (int j = 0; j < kMergePer; ++j) {
     const uint32_t i = static_cast<uint32_t>(j * kMergeLoaders + tid);
-    v1[j] = v2[j] = -INFINITY;
-    j1[j] = j2[j] = 0u;
+    u1[j] = u2[j] = -INFINITY;
     if (tid < kMergeLoaders && i < n_sub) {
-      const float u1 = p_u1[i], u2 = p_u2[i];
-      v1[j] = u1 * iq;
-      v2[j] = u2 * iq;
-      j1[j] = slot_of(u1, i);
-      j2[j] = slot_of(u2, i);
+      u1[j] = p_u1[i];
+      u2[j] = p_u2[i];
       nk = fmaxf(nk, p_nk[i] * iq);
     }
   }
   if (wave == kMergeWavesB - 1) {
-    // the last wavefront stages the query and forms the law's qnorm
-    double rest;
-    const double qn = stage_query_norm(s_q, query, q_dtype, qstride, qi, sb.dim,
-                                       merge_query_len(chunks, EPC), lane, rest);
+    const double rest = stage_row_query(s_q, query, q_dtype, qstride, qi, sb.dim, merge_len(sb.dim), lane);
     if (lane == 0) {
-      s_qn = qn;
-      s_rest = rest;
+      // 1/iq is the query's norm to within 2^-23
+      const double qa = 1.0 / static_cast<double>(iq);
+      s_qhi = qa * (1.0 + 0x1p-20);
+      s_bound = batch_screen_bound(sb, qa * (1.0 - 0x1p-20), rest,
+                                   static_cast<double>(__uint_as_float(norm_range[0])));
     }
   }
   if (tid == 0) s_count = 0u;
-  // largest finite kept s~ of the thread; a +inf s~ voids the certificate
-  float m = -INFINITY;
   bool pinf = false;
+  if (wave != kMergeWavesB - 1) {
+    // largest finite kept s~ of the thread; a +inf s~ voids the certificate
+    float m = -INFINITY;
 #pragma unroll
-  for (int j = 0; j < kMergePer; ++j) {
-    if (isfinite(v1[j])) m = fmaxf(m, v1[j]);
-    if (isfinite(v2[j])) m = fmaxf(m, v2[j]);
-    pinf = pinf || v1[j] == INFINITY || v2[j] == INFINITY;
+    for (int j = 0; j < kMergePer; ++j) {
+      const float v1 = u1[j] * iq, v2 = u2[j] * iq;
+      if (isfinite(v1)) m = fmaxf(m, v1);
+      if (isfinite(v2)) m = fmaxf(m, v2);
+      pinf = pinf || v1 == INFINITY || v2 == INFINITY;
+    }
+    const float ms = wave_sort_desc(m);
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) nk = fmaxf(nk, __shfl_xor(nk, off));
+    if (lane == k - 1) s_lw[wave] = ms;
+    if (lane == 0) s_nk[wave] = nk;
   }
-  const float ms = wave_sort_desc(m);
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) nk = fmaxf(nk, __shfl_xor(nk, off));
-  if (lane == k - 1) s_lw[wave] = ms;
-  if (lane == 0) s_nk[wave] = nk;
   const int any_pinf = __syncthreads_or(pinf ? 1 : 0);
 
-  const double qn = s_qn;
-  const double nmin = static_cast<double>(__uint_as_float(norm_range[0]));
   const double nmax = static_cast<double>(__uint_as_float(norm_range[1]));
-  const double bound = batch_screen_bound(sb, qn, s_rest, nmin);
+  const double bound = s_bound;
   float L = -INFINITY, nk_all = -INFINITY;
 #pragma unroll
   for (int w = 0; w < kMergeWavesB - 1; ++w) {
@@ -895,35 +981,34 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
     nk_all = fmaxf(nk_all, s_nk[w]);
   }
   const double floor_s = static_cast<double>(L) - 2.0 * bound - 0x1p-40;
-  auto offer = [&](float v, uint32_t key, uint32_t slot) {
+  auto offer = [&](float u, uint32_t key) {
+    const float v = u * iq;
     if (isfinite(v) && static_cast<double>(v) >= floor_s) {
       const unsigned at = atomicAdd(&s_count, 1u);
       if (at < static_cast<unsigned>(kSurvMax)) {
         s_sv[at] = v;
+        s_su[at] = u;
         s_key[at] = key;
-        s_slot[at] = slot;
       }
     }
   };
 #pragma unroll
   for (int j = 0; j < kMergePer; ++j) {
     const uint32_t i = static_cast<uint32_t>(j * kMergeLoaders + tid);
-    offer(v1[j], 2u * i, j1[j]);
-    offer(v2[j], 2u * i + 1u, j2[j]);
+    offer(u1[j], 2u * i);
+    offer(u2[j], 2u * i + 1u);
   }
   __syncthreads();
   const unsigned count = s_count;
   const int n = static_cast<int>(count < static_cast<unsigned>(kSurvMax) ? count : kSurvMax);
   int my_rank = 0;
   bool sup = false;
-  double dot = 0.0;
-  float nf = 0.0f;
-  uint64_t eid = kNoId;
-  uint32_t slot = 0u;
   if (tid < n) {
     const float sv = s_sv[tid];
     const uint32_t key = s_key[tid];
-    const double hi = static_cast<double>(sv) + 2.0 * bound + 0x1p-40;
+    // s~ + 2B rounded up: entries that round into it count as below
+    const double h = static_cast<double>(sv) + 2.0 * bound + 0x1p-40;
+    const float hi = static_cast<float>(h + fabs(h) * 0x1p-22 + 0x1p-140);
     int above = 0;
     int i = 0;
     for (; i + 4 <= n; i += 4) {
@@ -933,48 +1018,66 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
       my_rank += (o.y > sv || (o.y == sv && kk.y < key)) ? 1 : 0;
       my_rank += (o.z > sv || (o.z == sv && kk.z < key)) ? 1 : 0;
       my_rank += (o.w > sv || (o.w == sv && kk.w < key)) ? 1 : 0;
-      above += (static_cast<double>(o.x) > hi) + (static_cast<double>(o.y) > hi) +
-               (static_cast<double>(o.z) > hi) + (static_cast<double>(o.w) > hi);
+      above += (o.x > hi) + (o.y > hi) + (o.z > hi) + (o.w > hi);
     }
     for (; i < n; ++i) {
       const float o = s_sv[i];
       my_rank += (o > sv || (o == sv && s_key[i] < key)) ? 1 : 0;
-      above += static_cast<double>(o) > hi ? 1 : 0;
+      above += o > hi ? 1 : 0;
     }
-    s_byrank[my_rank] = static_cast<uint16_t>(tid);
+    if (my_rank < k) s_vrank[my_rank] = sv;
     sup = above < k;
-    if (sup) {
-      // the law's dot product of the row, d ascending (rows and the
-      // staged query are zero past dim: exact zeros)
-      slot = s_slot[tid];
-      nf = norms[slot];
-      eid = ids[slot];
-      for (uint32_t c0 = 0; c0 < chunks; c0 += kMergeChunks) {
-        u32x4 rv[kMergeChunks];
-#pragma unroll
-        for (uint32_t j = 0; j < kMergeChunks; ++j) {
-          const u32x4 zero = {0u, 0u, 0u, 0u};
-          rv[j] = c0 + j < chunks ? tiles[static_cast<size_t>(c0 + j) * cap + slot] : zero;
-        }
-        const double* q = s_q + c0 * EPC;
-#pragma unroll
-        for (uint32_t j = 0; j < kMergeChunks; ++j) dot = chunk_dot<DT>(rv[j], q + j * EPC, dot);
-      }
-    }
+    if (sup) s_rslot[my_rank] = slot_of(s_su[tid], key >> 1);
   }
   const int n_el = __syncthreads_count(sup ? 1 : 0);
-  const float vk = n >= k ? s_sv[s_byrank[k - 1]] : -INFINITY;
+  // the prefix's rows, merge_rows at a time; the row's thread (thread = rank
+  // within the round) keeps its dot product.  Rows are staged by chunk, zero
+  // past dim as they are stored, and on to whole stages.
+  const uint32_t rows = merge_rows(sb.dim);
+  const uint32_t len = merge_len(sb.dim), pitch = merge_pitch(sb.dim);
+  double dot = 0.0;
+  float nf = 0.0f;
+  uint64_t eid = kNoId;
+  for (uint32_t r0 = 0; r0 == 0 || r0 < static_cast<uint32_t>(n_el); r0 += rows) {
+    const uint32_t r1 = min(r0 + rows, static_cast<uint32_t>(n_el));
+    if (r0 > 0) __syncthreads();  // the rows before are done with
+    if (wave == kMergeWavesB - 1) {
+      if (r0 == 0 && lane == 0) s_qn = sqrt(serial_dot(s_q, s_q, len));
+    } else {
+      for (uint32_t r = r0 + wave; r < r1; r += kMergeWavesB - 1) {
+        const uint32_t slot = s_rslot[r];
+        for (uint32_t c = lane; c * EPC < len; c += kWave) {
+          u32x4 v = {0u, 0u, 0u, 0u};
+          if (c < chunks) v = tiles[static_cast<size_t>(c) * cap + slot];
+#pragma unroll
+          for (int e = 0; e < static_cast<int>(EPC); ++e) {
+            s_rows[(r - r0) * pitch + c * EPC + e] = chunk_value<DT>(v, e);
+          }
+        }
+      }
+    }
+    const uint32_t r = tid;
+    const bool mine = r >= r0 && r < r1;
+    if (mine) {
+      nf = norms[s_rslot[r]];
+      eid = ids[s_rslot[r]];
+    }
+    __syncthreads();
+    if (mine) dot = serial_dot(s_rows + (r - r0) * pitch, s_q, len);
+  }
+  const double qn = s_qn;
+  const float vk = n >= k ? s_vrank[k - 1] : -INFINITY;
   const double t = static_cast<double>(vk) - 2.0 * bound - 0x1p-40;
   // t > 0: the screen kept its values by their integer bits, the float
   // order only from +0 up.
   const bool pre = any_pinf == 0 && count <= static_cast<unsigned>(kSurvMax) && n >= k &&
-                   static_cast<double>(nk_all) < t && t > 0.0 && screen_in_range(qn, nmax);
+                   static_cast<double>(nk_all) < t && t > 0.0 && screen_in_range(s_qhi, nmax);
   // the rescored prefix: ranks [0, n_el)
-  if (sup) {
+  if (tid < n_el) {
     const float sc = static_cast<float>(dot / (qn * static_cast<double>(nf) + 1e-8));
     const bool fin = isfinite(sc);
-    s_es[my_rank] = fin ? sc : __builtin_nanf("");
-    s_eid[my_rank] = fin ? eid : kNoId;
+    s_es[tid] = fin ? sc : __builtin_nanf("");
+    s_eid[tid] = fin ? eid : kNoId;
   }
   __syncthreads();
   // rank the prefix by (law score desc, node id asc)
@@ -1021,9 +1124,9 @@ __global__ __launch_bounds__(kWave) void mla_batch_probe_finish_kernel(
   extern __shared__ double s_q[];  // len values
   const int qi = blockIdx.x;
   const int lane = threadIdx.x;
-  double rest;
-  const double qn = stage_query_norm(s_q, query, q_dtype, qstride, qi, sb.dim, len, lane, rest);
+  const double rest = stage_row_query(s_q, query, q_dtype, qstride, qi, sb.dim, len, lane);
   if (lane == 0) {
+    const double qn = staged_norm(s_q, len);
     const double nmin = static_cast<double>(__uint_as_float(norm_range[0]));
     const double nmax = static_cast<double>(__uint_as_float(norm_range[1]));
     out_bounds[qi] = screen_in_range(qn, nmax) ? batch_screen_bound(sb, qn, rest, nmin)

@@ -426,7 +426,7 @@ struct MlaDeviceArena {
   // engine instead)
   grm::MappedBuf q_map;
   bool query_dma = false;
-  int batch_min = 4;         // timed queries per call from which the batched path runs
+  int batch_min = 0;         // timed queries per call from which the batched path runs (0: by size)
   bool ring = true;          // full 256-query passes on the ring screen (GRM_HIP_BATCH_RING=0: off)
   float* d_winv = nullptr;   // slot weights of the ring screen (capacity), for bank epoch winv_epoch
   size_t d_winv_count = 0;
@@ -774,12 +774,10 @@ struct BatchPlan {
   int ibits = 0;       // width of the slot code the stream screen writes into its values
   bool ring = false;   // full passes of a bf16 bank run mla_batch_ring_kernel
   int ks_ring = 0;     // its K-steps (8, 16 or 18)
-  int ibits_ring = 0;  // its slot code width (one sub-stream per block)
+  int ibits_ring = 0;  // its slot code width
 };
 
-// Slot code width of the batched screen: 4 bits of result register, the
-// lane half, and enough bits for the longest run of tiles one sub-stream
-// walks.  The code costs the screen bound 2^(ibits-23) relative, so banks
+// Slot code width of the batched screens.  The code costs the screen bound 2^(ibits-23) relative, so banks
 // whose runs would need more than 16 bits route on the single-query path
 // instead.
 constexpr int kMaxSlotCodeBits = 16;
@@ -790,8 +788,19 @@ size_t stream_lds(const MlaDeviceArena* a, const BatchPlan& p, int qp) {
   return static_cast<size_t>(qp) * (16 * p.nb * p.p + 8) * (a->dtype == kF32 ? 4 : 2);
 }
 
+// Timed queries per call from which the batched path runs: three, or two on
+// banks of 8,192 slots and more.  A batched call costs 24 to 42 us on small
+// banks (64 to 576 values) whatever its queries, the single-query kernel
+// about 10 us a query after the first: two queries took 21 against 25 us at
+// 1,000 x 64 and 31 against 31 at 5,000 x 288, but 38 against 33 at 20,000 x
+// 288 and 97 against 74 at 100,000 x 576; three never less than the batched
+// call.
+int batch_threshold(const MlaDeviceArena* a) {
+  return a->batch_min > 0 ? a->batch_min : (a->high_water >= 8192 ? 2 : 3);
+}
+
 bool batch_plan(const MlaDeviceArena* a, int q_timed, BatchPlan* p) {
-  if (q_timed < a->batch_min) return false;
+  if (q_timed < batch_threshold(a)) return false;
   const uint32_t per_step = a->dtype == kF32 ? 4 : 2;  // chunks
   p->ks = static_cast<int>((a->chunks + per_step - 1) / per_step);
   // the steps in flight that pad the row least, the most of those
@@ -814,17 +823,18 @@ bool batch_plan(const MlaDeviceArena* a, int q_timed, BatchPlan* p) {
   if (waves > static_cast<uint32_t>(grm::mla::kMergeLoaders) * grm::mla::kMergePer) return false;
   const uint32_t n_tiles32 = static_cast<uint32_t>((a->high_water + 31) / 32);
   if (n_tiles32 == 0) return false;
-  auto code_bits = [&](uint32_t n_sub) {
-    const uint32_t max_run = (n_tiles32 + n_sub - 1) / n_sub;
-    int ibits = 5;
-    while ((1u << (ibits - 5)) < max_run) ++ibits;
-    return ibits;
+  // register, tile offset in the longest run, and (stream) the lane half
+  auto code_bits = [&](uint32_t runs, int half_bits) {
+    const uint32_t max_run = (n_tiles32 + runs - 1) / runs;
+    int bits = 0;
+    while ((1u << bits) < max_run) ++bits;
+    return 4 + bits + half_bits;
   };
   p->subs = std::min(waves, n_tiles32);
-  p->ibits = code_bits(p->subs);
+  p->ibits = code_bits(p->subs, 1);
   if (p->ibits > kMaxSlotCodeBits) return false;
   p->ks_ring = p->ks <= 8 ? 8 : (p->ks <= 16 ? 16 : (p->ks <= 18 ? 18 : 0));
-  p->ibits_ring = code_bits(a->cus);
+  p->ibits_ring = code_bits(a->cus * grm::mla::kRingSegs, 0);
   p->ring = a->ring && a->dtype == kBF16 && qp == grm::mla::kStreamMaxCols && p->ks_ring != 0 && a->planes >= 2u * p->ks_ring &&
             p->ibits_ring <= kMaxSlotCodeBits && grm::mla::RingShape<18>::kLds <= a->lds_max;
   p->qp_max = p->ring ? grm::mla::kRingQueries : qp;
@@ -840,7 +850,9 @@ struct PassShape {
   int ibits;
 };
 PassShape pass_shape(const MlaDeviceArena* a, const BatchPlan& p, int qc) {
-  if (qc > grm::mla::kStreamMaxCols) return {true, grm::mla::kRingQueries, a->cus, p.ibits_ring};
+  if (qc > grm::mla::kStreamMaxCols) {
+    return {true, grm::mla::kRingQueries, a->cus * 2 * grm::mla::kRingSegs, p.ibits_ring};
+  }
   return {false, qc <= 32 ? 32 : (qc <= 64 ? 64 : 128), p.subs, p.ibits};
 }
 
@@ -976,9 +988,12 @@ int enqueue_batch_pass(MlaDeviceArena* a, const BatchPlan& p, const PassQueries&
   const uint32_t n_tiles32 = static_cast<uint32_t>((a->high_water + 31) / 32);
   auto kern = a->dtype == kF32 ? grm::mla::mla_batch_merge_kernel<kF32>
                                : grm::mla::mla_batch_merge_kernel<kBF16>;
-  const size_t lds = grm::mla::merge_query_len(a->chunks, a->epc) * sizeof(double);
+  const size_t lds = grm::mla::merge_lds(a->dim);
+  GRM_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    static_cast<int>(lds)));
   kern<<<q.count, grm::mla::kMergeThreads, lds, a->stream>>>(
-      a->d_entries, s.subs, s.qp, n_tiles32, a->d_inv_qn, a->d_tiles, a->d_norms, a->d_ids,
+      a->d_entries, s.subs, s.ring, s.qp, n_tiles32, a->d_inv_qn, a->d_tiles, a->d_norms, a->d_ids,
       a->capacity, a->chunks, q.q, q.dtype, a->dim, screen_bound(a, p, s.ibits),
       a->d_min_norm, topk, out, done, a->route_seq, end_tick,
       m.screen_tick ? m.screen_tick + 1 : nullptr);
@@ -990,8 +1005,8 @@ int enqueue_batch_pass(MlaDeviceArena* a, const BatchPlan& p, const PassQueries&
 // them: the queries then go one by one.
 bool reserve_batch(MlaDeviceArena* a, const BatchPlan& p) {
   const size_t cols = std::max(p.qp_stream, p.qp_max);
-  const size_t subs = std::max(p.subs * static_cast<size_t>(p.qp_stream),
-                               p.ring ? a->cus * static_cast<size_t>(p.qp_max) : size_t{0});
+  size_t subs = p.subs * static_cast<size_t>(p.qp_stream);
+  if (p.ring) subs = std::max<size_t>(subs, a->cus * size_t{2 * grm::mla::kRingSegs} * p.qp_max);
   const bool ok =
       (!p.ring || reserve_device(&a->d_qpad, &a->d_qpad_count, cols * (16 * p.ks_ring + 8)) == 0) &&
       reserve_device(&a->d_inv_qn, &a->d_inv_qn_count, cols) == 0 &&
@@ -1987,7 +2002,7 @@ extern "C" int grm_mla_hip_probe_screen(MlaDeviceArena* a, const void* queries_h
   GRM_HIP_CHECK(hipMemcpyAsync(d_q.p, queries_host, qbytes, hipMemcpyHostToDevice, a->stream));
   const PassQueries pq{d_q.p, query_dtype, query_count};
   GRM_CHECK_RC(launch_screen<true>(a, p, shape, pq, static_cast<uint32_t*>(d_planes.p), PassMarks{}));
-  const uint32_t len = grm::mla::merge_query_len(a->chunks, a->epc);
+  const uint32_t len = grm::mla::merge_len(a->dim);
   grm::mla::mla_batch_probe_finish_kernel<<<query_count, grm::kWave, len * sizeof(double), a->stream>>>(
       static_cast<const uint32_t*>(d_planes.p), a->capacity, static_cast<uint32_t>(n), a->d_inv_qn,
       d_q.p, query_dtype, a->dim, len, screen_bound(a, p, shape.ibits), a->d_min_norm,

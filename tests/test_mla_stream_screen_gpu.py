@@ -56,6 +56,16 @@ def test_query_counts(hip_lib, nq, k, n):
         assert bank.route_stats()["batched"] == nq
 
 
+# the ring screen's runs: none, one or several tiles each
+@pytest.mark.parametrize("n", [20, 33, 5000, 32_768, 33_001, 100_003])
+def test_ring_runs(hip_lib, n):
+    rows = wl.mla_rows(n, 72, seed=n, dtype="bf16")
+    qs = wl.mla_queries(200, 72, seed=n + 1, dtype="bf16")
+    with MlaNodeBank(rows, dtype="bf16") as bank:
+        check(bank, rows, qs, 16, query_dtype="bf16")
+        assert bank.route_stats()["batched"] == 200
+
+
 def test_churn_warmup_and_bf16_queries(hip_lib):
     rng = np.random.default_rng(3)
     rows = wl.mla_rows(5000, 280, seed=5)
