@@ -569,30 +569,89 @@ constexpr int kMaxSmaxCols = 128;  // per screen-only pass (gqa_smax_kernel, NT 
 // below 2^127 in magnitude (Cauchy-Schwarz; 1 + 2^-6 covers the roundings
 // of query, key and sums), so no screened value overflows; for K >= kcap
 // the bound is not established and the screen's users take E = +inf.
-// Ends with a barrier.
-template <int HD, int QS = HD>
+// Threads tid < THREADS (whole wavefronts) share the work on at most MAXC
+// columns; a block may run one such group of threads per query pass, as
+// long as all of it comes here: it ends with a barrier.
+//
+// What bounds it is latency, in front of a block's whole stream: a thread
+// loads 8 values at a time, up to 8 such pieces before it stores any, so
+// 64 columns of 128 values cost a block one trip to memory instead of 32
+// (one value per thread and trip): gqa_smax_kernel 220 -> 185 us with 4
+// passes of 64 columns (64 query tokens, 256 nodes, 553 MB of bf16 keys),
+// 260 -> 240 us with one (4000 INT8 nodes), gqa_sr_kernel 44.6 -> 42.0 us
+// with 16 columns on 128 fp32 nodes, unchanged with 4 columns on 512
+// nodes.  Queries not aligned to 16 bytes (a caller's own device buffer)
+// go value by value.
+template <int HD, int QS, int MAXC, int THREADS>
 __device__ inline void stage_columns(float* __restrict__ s_q, float4* __restrict__ s_ec,
                                      unsigned* __restrict__ s_bad, const void* __restrict__ query,
                                      int q_dtype, size_t q_elems, int cols, int R, int Qt, int Rc,
                                      int Qc, int g, int emax, double gamma, double delta,
                                      double rho, double sigma_q, double sigma_k, double sigma_p,
-                                     double eps_rel, double eps_abs) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const int nwaves = blockDim.x / kWave;
+                                     double eps_rel, double eps_abs, int tid) {
+  static_assert(QS % 4 == 0, "16-byte aligned rows");
+  constexpr int nt = THREADS;
+  // pieces of 8 values that one thread holds at most before it stores them
+  constexpr int kNeed = (MAXC * (HD / 8) + THREADS - 1) / THREADS;
+  constexpr int kHold = kNeed < 8 ? kNeed : 8;
+  const int lane = tid & (kWave - 1);
+  const int wave = tid / kWave;
+  const int nwaves = nt / kWave;
   const int RQc = Rc * Qc;
-  {
-    // thread t stages value t % HD of columns t / HD, t / HD + per, ...
-    const int per = static_cast<int>(blockDim.x) / HD;
-    const int d = static_cast<int>(threadIdx.x) % HD;
-    const int first = static_cast<int>(threadIdx.x) / HD;
-    for (int cg = first; cg < cols && first < per; cg += per) {
-      const int qb = cg / RQc;
-      const int r = (cg % RQc) / Qc;
-      const uint64_t src = static_cast<uint64_t>(qb) * q_elems +
-                           (static_cast<uint64_t>(g * R + r) * Qt + cg % Qc) * HD + d;
-      s_q[cg * QS + d] = q_dtype == kBF16 ? bf16_to_f32(static_cast<const uint16_t*>(query)[src])
-                                          : static_cast<const float*>(query)[src];
+  // first value of column cg in the query
+  auto column = [&](int cg) -> uint64_t {
+    const int qb = cg / RQc;
+    const int rem = cg - qb * RQc;
+    const int r = rem / Qc;
+    return static_cast<uint64_t>(qb) * q_elems +
+           (static_cast<uint64_t>(g * R + r) * Qt + (rem - r * Qc)) * HD;
+  };
+  constexpr int P = HD / 8;  // pieces of 8 values per column
+  const int n = cols * P;
+  if ((reinterpret_cast<uintptr_t>(query) & 15u) != 0u || q_elems % 8 != 0) {
+    for (int i = tid; i < cols * HD; i += nt) {
+      const uint64_t src = column(i / HD) + i % HD;
+      s_q[(i / HD) * QS + i % HD] = q_dtype == kBF16
+                                        ? bf16_to_f32(static_cast<const uint16_t*>(query)[src])
+                                        : static_cast<const float*>(query)[src];
+    }
+  } else if (q_dtype == kBF16) {
+    constexpr int B = kHold;
+    for (int i0 = tid; i0 < n; i0 += B * nt) {
+      u32x4 w[B];
+#pragma unroll
+      for (int j = 0; j < B; ++j) {
+        const int i = min(i0 + j * nt, n - 1);
+        w[j] = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(query) + column(i / P) + (i % P) * 8);
+      }
+#pragma unroll
+      for (int j = 0; j < B; ++j) {
+        const int i = i0 + j * nt;
+        if (i >= n) break;
+        u32x4* out = reinterpret_cast<u32x4*>(s_q + (i / P) * QS + (i % P) * 8);
+        out[0] = u32x4{w[j].x << 16, w[j].x & 0xffff0000u, w[j].y << 16, w[j].y & 0xffff0000u};
+        out[1] = u32x4{w[j].z << 16, w[j].z & 0xffff0000u, w[j].w << 16, w[j].w & 0xffff0000u};
+      }
+    }
+  } else {
+    constexpr int B = kHold < 4 ? kHold : 4;
+    for (int i0 = tid; i0 < n; i0 += B * nt) {
+      u32x4 w[B][2];
+#pragma unroll
+      for (int j = 0; j < B; ++j) {
+        const int i = min(i0 + j * nt, n - 1);
+        const u32x4* in = reinterpret_cast<const u32x4*>(static_cast<const float*>(query) + column(i / P) + (i % P) * 8);
+        w[j][0] = in[0];
+        w[j][1] = in[1];
+      }
+#pragma unroll
+      for (int j = 0; j < B; ++j) {
+        const int i = i0 + j * nt;
+        if (i >= n) break;
+        u32x4* out = reinterpret_cast<u32x4*>(s_q + (i / P) * QS + (i % P) * 8);
+        out[0] = w[j][0];
+        out[1] = w[j][1];
+      }
     }
   }
   __syncthreads();
@@ -668,7 +727,7 @@ __device__ inline int frag_dim(int ks, int quarter, int j) {
 // is the sum of its slot and the slot cols lanes up: the query's rounding
 // error drops from u |q| to u^2 |q| per value (u the type's unit
 // roundoff); the remainder is exact in fp32 (Sterbenz: within u of q).
-template <int MT, bool PERM, int KS, int NT, int QS = 32 * KS>
+template <int MT, bool PERM, int KS, int NT, int QS>
 __device__ inline void query_frags(u32x4 (&bq)[NT][KS], const float* __restrict__ s_q,
                                    const float4* __restrict__ s_ec, int cols, int r16,
                                    int quarter, bool split = false) {
@@ -979,9 +1038,9 @@ __global__ __launch_bounds__(kUnitWaves * kWave, (sr_waves_per_simd<KDT, KS, NT,
     load_tile(x2, 2);
     load_tile(x3, 3);
   }
-  stage_columns<HD, QS>(s_q, s_ec, s_bad, query, q_dtype, q_elems, cols, R, Qt, Rc, Qc, g, emax,
-                        gamma, delta, 0.0, sigma_q, sigma_k, sigma_p, eps_rel, eps_abs);
-  __syncthreads();
+  stage_columns<HD, QS, NT * 16, kUnitWaves * kWave>(
+      s_q, s_ec, s_bad, query, q_dtype, q_elems, cols, R, Qt, Rc, Qc, g, emax, gamma, delta, 0.0,
+      sigma_q, sigma_k, sigma_p, eps_rel, eps_abs, static_cast<int>(threadIdx.x));
   if (item_block == 0 && threadIdx.x < static_cast<unsigned>(Qb)) {
     unsigned bad = 0u;
     for (int j = 0; j < RQc; ++j) bad |= s_bad[threadIdx.x * RQc + j];
@@ -1282,22 +1341,23 @@ __global__ __launch_bounds__((NP == 1 ? kUnitWaves : 8) * kWave,
   static_assert(NP == 1 || NT <= 4, "split passes hold at most 64 columns each");
   constexpr int WPB = NP == 1 ? kUnitWaves : 8 / NP;  // walkers per block
   constexpr int kPassCols = NP == 1 ? kMaxSmaxCols : kMaxCols;
-  extern __shared__ float s_q[];                    // [NP][NT*16][HD]
+  // rows padded as in gqa_sr_kernel: 16 lanes read one offset of 16 columns
+  constexpr int QS = HD + 4;
+  extern __shared__ __align__(16) float s_q[];      // [NP][NT*16][QS]
   __shared__ float4 s_ec[NP * kPassCols];
   __shared__ unsigned s_bad[NP * kPassCols];
   const int lane = threadIdx.x & (kWave - 1);
   const int g = blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int pi = NP == 1 ? 0 : wave % NP;           // this wavefront's pass
-  // the query's full column index of column cg of pass p
-  auto full_col_of = [&](int p, int cg) {
-    const int RQp = ps.rc[p] * ps.qc[p];
+  // the query's full column index of the pass's column cg
+  auto full_col = [&](int cg) {
+    const int RQp = ps.rc[pi] * ps.qc[pi];
     const int qb = cg / RQp;
     const int rem = cg - qb * RQp;
-    return qb * R * Qt + (ps.r0[p] + rem / ps.qc[p]) * Qt + ps.t0[p] + rem % ps.qc[p];
+    return qb * R * Qt + (ps.r0[pi] + rem / ps.qc[pi]) * Qt + ps.t0[pi] + rem % ps.qc[pi];
   };
   const int cols = Qb * ps.rc[pi] * ps.qc[pi];
-  auto full_col = [&](int cg) { return full_col_of(pi, cg); };
   const int quarter = lane >> 4;
   const int r16 = lane & 15;
   const uint32_t stride = gridDim.x * WPB;
@@ -1408,29 +1468,31 @@ __global__ __launch_bounds__((NP == 1 ? kUnitWaves : 8) * kWave,
     load_next(x2);
     load_next(x3);
   }
-  // every pass's columns, each in its own LDS region (the query advanced
-  // to the pass's first value, see "Query passes")
-  const size_t esz = q_dtype == kBF16 ? 2 : 4;
-#pragma unroll
-  for (int p = 0; p < NP; ++p) {
+  // every pass's columns, each in its own LDS region, staged by the pass's
+  // own wavefronts (the query advanced to the pass's first value, see
+  // "Query passes")
+  {
+    constexpr int kPassThreads = (NP == 1 ? kUnitWaves : 8 / NP) * kWave;
+    const size_t esz = q_dtype == kBF16 ? 2 : 4;
+    const int tid = (wave / NP) * kWave + lane;
     const unsigned char* qp = static_cast<const unsigned char*>(query) +
-                              static_cast<size_t>(ps.r0[p] * Qt + ps.t0[p]) * HD * esz;
-    const int cols_p = Qb * ps.rc[p] * ps.qc[p];
-    stage_columns<HD>(s_q + static_cast<size_t>(p) * NT * 16 * HD, s_ec + p * kPassCols,
-                      s_bad + p * kPassCols, qp, q_dtype, q_elems, cols_p, R, Qt, ps.rc[p],
-                      ps.qc[p], g, emax, gamma, delta, rho, sigma_q, sigma_k, sigma_p, eps_rel,
-                      eps_abs);
+                              static_cast<size_t>(ps.r0[pi] * Qt + ps.t0[pi]) * HD * esz;
+    float4* ec = s_ec + pi * kPassCols;
+    stage_columns<HD, QS, NT * 16, kPassThreads>(
+        s_q + static_cast<size_t>(pi) * NT * 16 * QS, ec, s_bad + pi * kPassCols, qp, q_dtype, q_elems,
+        cols, R, Qt, ps.rc[pi], ps.qc[pi], g, emax, gamma, delta, rho, sigma_q, sigma_k, sigma_p,
+        eps_rel, eps_abs, tid);
     if (blockIdx.x == 0) {
-      for (int cg = threadIdx.x; cg < cols_p; cg += blockDim.x) {
-        colinfo[static_cast<size_t>(g) * colstride + full_col_of(p, cg)] = s_ec[p * kPassCols + cg];
+      for (int cg = tid; cg < cols; cg += kPassThreads) {
+        colinfo[static_cast<size_t>(g) * colstride + full_col(cg)] = ec[cg];
       }
     }
   }
   if (!has_item) return;
 
   u32x4 bq[NT][KS];
-  query_frags<MT, PERM, KS, NT>(bq, s_q + static_cast<size_t>(pi) * NT * 16 * HD,
-                                s_ec + pi * kPassCols, cols, r16, quarter);
+  query_frags<MT, PERM, KS, NT, QS>(bq, s_q + static_cast<size_t>(pi) * NT * 16 * QS,
+                                    s_ec + pi * kPassCols, cols, r16, quarter);
 
   // key fragment ks of half h of a tile: 8 values of the lane's token in
   // the MFMA type

@@ -1109,8 +1109,8 @@ int launch_smax(GqaDeviceArena* a, const SrPlan& p, const unsigned char* qptr, i
   const unsigned threads = (np == 1 ? grm::gqa::kUnitWaves : 8) * grm::kWave;
   if (a->n_units > 0) {
     // one LDS region of NT*16 columns per pass when passes are split
-    const size_t lds = np == 1 ? static_cast<size_t>(cols) * a->hd * sizeof(float)
-                               : static_cast<size_t>(np) * NT * 16 * a->hd * sizeof(float);
+    // (rows of hd + 4 floats, see gqa_smax_kernel)
+    const size_t lds = static_cast<size_t>(np == 1 ? cols : np * NT * 16) * (a->hd + 4) * sizeof(float);
 #define GRM_SMAX_NP(KDT, KS, NTT, FACT, SF16, NPP)                                                \
   do {                                                                                            \
     auto fn = grm::gqa::gqa_smax_kernel<KDT, KS, NTT, FACT, SF16, NPP>;                           \

@@ -1,0 +1,44 @@
+"""Query columns staged in pieces of 8 values: device queries at any
+alignment, every head dim and query type, and the sizes at which a route
+takes another path (screen and refine, batched bound and verify, passes of
+a long query).  Ids and score bits equal the oracle's."""
+
+import numpy as np
+import pytest
+
+import oracle
+from graftrepository_amd import GqaNodeBank, workloads as wl
+from graftrepository_amd.node_bank import bf16_bits_to_f32
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+def device_query(q, shift, dtype):
+    """q on the GPU, its first value `shift` values past an aligned address."""
+    flat = torch.zeros(q.size + 64, dtype=torch.float32, device="cuda")
+    flat[shift:shift + q.size] = torch.from_numpy(q.reshape(-1))
+    if dtype == "bf16":
+        flat = flat.bfloat16()
+    return flat[shift:shift + q.size].view(q.shape)
+
+
+# (queries, tokens, heads per kv head): one column, a full column block and
+# one more, batched bound and verify, a long query of odd length in one
+# launch of passes, and one whose heads share 1, 4 and 16 lanes in the bounds
+@pytest.mark.parametrize("queries,tokens,group", [(1, 1, 1), (1, 4, 4), (1, 17, 1), (5, 1, 8),
+                                                  (1, 33, 4), (1, 67, 4), (1, 3, 90), (1, 130, 2)])
+@pytest.mark.parametrize("dtype,shift", [("bf16", 0), ("bf16", 1), ("f32", 0), ("f32", 3)])
+@pytest.mark.parametrize("hd", [64, 128, 256])
+def test_query_alignment(hip_lib, hd, dtype, shift, queries, tokens, group):
+    kv = 4
+    lens = wl.gqa_lengths(30, hd, lo=1, hi=90)
+    keys, offs = wl.gqa_bank(lens, kv, hd, 5, dtype="bf16")
+    q = np.random.default_rng(7).standard_normal((queries, kv * group, tokens, hd), dtype=np.float32)
+    dev = device_query(q, shift, dtype)
+    q = dev.float().cpu().numpy()
+    with GqaNodeBank(keys, offs, kv_heads=kv, head_dim=hd, dtype="bf16") as bank:
+        res = bank.route(dev, 5, on_device=True, query_dtype=dtype, timed=False)
+    ids, sc, _ = oracle.gqa_route(keys, oracle.BF16, offs, kv, hd, q, 5)
+    np.testing.assert_array_equal(res.ids, ids)
+    np.testing.assert_array_equal(res.scores.view(np.uint32), sc.view(np.uint32))
