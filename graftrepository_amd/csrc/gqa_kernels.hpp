@@ -171,6 +171,12 @@ __device__ inline void decode_chunk(u32x4 v, float scale, float* out) {
 // load.  qflags[qb * kv + g] = 1 when a value of query qb read by kv head g
 // is non-finite; the first pass (flags_or = 0) writes 0 otherwise, later
 // passes leave the flag as it is.  grid (kv, Qb).
+//
+// Latency and the d-major store bound it.  Where rows are 16-byte aligned a
+// thread loads 8 values of one row and stores one value of each of 8 output
+// rows, neighbouring threads neighbouring columns; loading value by value
+// in the output's order read one 2-byte value per line and lane: 24.3 ->
+// 11.1 us for 128 heads x 64 tokens x 128.
 __global__ __launch_bounds__(1024) void gqa_q64_kernel(
     const void* __restrict__ query, int q_dtype, size_t q_elems, int Qt, int Qc,
     int hd, int kv, int R, int Rc, int RQP, double* __restrict__ q64,
@@ -179,7 +185,34 @@ __global__ __launch_bounds__(1024) void gqa_q64_kernel(
   const int qb = blockIdx.y;
   const int rq = Rc * Qc;
   bool bad = false;
-  for (int idx = threadIdx.x; idx < RQP * hd; idx += blockDim.x) {
+  const bool wide = (reinterpret_cast<uintptr_t>(query) & 15u) == 0u && hd % 8 == 0 && q_elems % 8 == 0;
+  double* __restrict__ out = q64 + static_cast<size_t>(qb * kv + g) * hd * RQP;
+  for (int idx = threadIdx.x; wide && idx < RQP * (hd / 8); idx += blockDim.x) {
+    const int dp = idx / RQP;
+    const int j = idx - dp * RQP;
+    float f[8] = {};
+    if (j < rq) {
+      const uint64_t src = static_cast<uint64_t>(qb) * q_elems +
+                           (static_cast<uint64_t>(g * R + j / Qc) * Qt + j % Qc) * hd + dp * 8;
+      if (q_dtype == kBF16) {
+        decode_chunk<kBF16>(*reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(query) + src), 0.0f, f);
+      } else {
+        const u32x4* in = reinterpret_cast<const u32x4*>(static_cast<const float*>(query) + src);
+        const u32x4 lo = in[0], hi = in[1];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          f[e] = __uint_as_float(lo[e]);
+          f[4 + e] = __uint_as_float(hi[e]);
+        }
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      bad = bad || !isfinite(f[e]);
+      out[static_cast<size_t>(dp * 8 + e) * RQP + j] = static_cast<double>(f[e]);
+    }
+  }
+  for (int idx = threadIdx.x; !wide && idx < RQP * hd; idx += blockDim.x) {
     const int d = idx / RQP;
     const int j = idx - d * RQP;
     double v = 0.0;
@@ -192,7 +225,7 @@ __global__ __launch_bounds__(1024) void gqa_q64_kernel(
       bad = bad || !isfinite(f);
       v = static_cast<double>(f);
     }
-    q64[(static_cast<size_t>(qb * kv + g) * hd + d) * RQP + idx % RQP] = v;
+    out[static_cast<size_t>(d) * RQP + j] = v;
   }
   bad = __syncthreads_or(bad);
   if (threadIdx.x == 0 && (bad || !flags_or)) qflags[qb * kv + g] = bad ? 1u : 0u;
@@ -1805,14 +1838,18 @@ __global__ __launch_bounds__(kFinWaves * kWave) void gqa_bounds_kernel(
 }
 
 // The same bounds for queries of many tokens (H*Qt cells per node): one
-// wavefront per node at a time, its lanes over heads -- lane l takes heads
-// l, l + 64, ..., each the max over its Qt query tokens' bounds -- and the
-// heads' sums formed by a reduction across the wavefront (a different
-// order than the sequential sum, which the 2^-40 widening covers many
-// times over: the fp64 sum of H non-negative terms is within H * 2^-53 of
-// exact).  grid (queries, blocks), kFinWaves wavefronts; wavefront w of
-// block b takes nodes (b * kFinWaves + w) + i * blocks * kFinWaves.
-// Outputs as gqa_bounds_kernel.
+// block per node at a time.  `lph` lanes (a power of two, at most 16) share
+// a head, reading neighbouring tokens' cells and column parameters, so a
+// wavefront takes 64/lph heads at once; each head is the max over its Qt
+// query tokens' bounds, and the heads' sums form by a reduction across the
+// wavefront and the block (a different order than the sequential sum, which
+// the 2^-40 widening covers many times over: the fp64 sum of H non-negative
+// terms is within H * 2^-53 of exact).  grid (queries, blocks); block b
+// takes nodes b + i * blocks.  Outputs as gqa_bounds_kernel.
+//
+// Bound by the latency of its loads.  A lane per head, one wavefront per
+// node, left a 256-node bank with 256 wavefronts on the chip whose lanes
+// read 64 different lines: 39.1 -> 16.0 us (8192 cells per node).
 __global__ __launch_bounds__(kFinWaves * kWave) void gqa_bounds_wide_kernel(
     const unsigned* __restrict__ hmaxf, int colstride, size_t cap, int H, int Qt, int R, int cols,
     int kv, uint32_t n_slots, const uint32_t* __restrict__ lens,
@@ -1820,11 +1857,15 @@ __global__ __launch_bounds__(kFinWaves * kWave) void gqa_bounds_wide_kernel(
     const unsigned* __restrict__ kmax, const float4* __restrict__ colinfo,
     const unsigned* __restrict__ qbad, int fact, int hd, int k, float2* __restrict__ lbub,
     Cand* __restrict__ block_out, uint32_t* __restrict__ counters, int n_counters) {
-  __shared__ Cand s_lists[kFinWaves][kMaxTopK];
+  __shared__ double s_sum[2][kFinWaves][2];  // (lo, hi) per wavefront, by the node's parity
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int qb = blockIdx.x;
   const uint32_t sblk = blockIdx.y, nsblk = gridDim.y;
+  int lph = 1;
+  while (lph < 16 && lph < Qt) lph *= 2;
+  const int hpw = kWave / lph;  // heads per wavefront at a time
+  const int sl = lane % lph;
   if (sblk == 0 && threadIdx.x == 0) {
     counters[qb] = 0u;
     if (qb == 0) counters[n_counters - 1] = 0u;
@@ -1837,7 +1878,8 @@ __global__ __launch_bounds__(kFinWaves * kWave) void gqa_bounds_wide_kernel(
   q_bad = __ballot(q_bad) != 0ull;
   WaveList Lw;
   wl_init(Lw);
-  for (uint32_t slot = sblk * kFinWaves + wave; slot < n_slots; slot += nsblk * kFinWaves) {
+  int parity = 0;
+  for (uint32_t slot = sblk; slot < n_slots; slot += nsblk) {
     const uint32_t f = flags[slot];
     const uint32_t len = lens[slot];
     const uint64_t id = ids[slot];
@@ -1846,46 +1888,68 @@ __global__ __launch_bounds__(kFinWaves * kWave) void gqa_bounds_wide_kernel(
     double lo_sum = 0.0, hi_sum = 0.0;
     if (screened) {
       const unsigned* cells = hmaxf + static_cast<size_t>(slot) * kv * colstride;
-      for (int h = lane; h < H; h += kWave) {
+      for (int h = wave * hpw + lane / lph; h < H; h += kFinWaves * hpw) {
         const size_t c0 = static_cast<size_t>(h / R) * colstride + (qb * R + h % R) * Qt;
         const size_t i0 = static_cast<size_t>(h / R) * cols + (qb * R + h % R) * Qt;
         double lo_h = 0.0, hi_h = 0.0;
-        // the head's Qt cells and column parameters, 8 loaded before any
-        // is used
-        constexpr int kB = 8;
-        for (int t0 = 0; t0 < Qt; t0 += kB) {
+        // the lane's tokens sl, sl + lph, ..., 4 loaded before any is used
+        // (past the end: the last token again, which a max already holds)
+        constexpr int kB = 4;
+        for (int t0 = sl; t0 < Qt; t0 += kB * lph) {
           float4 ci[kB];
           float mv[kB];
 #pragma unroll
           for (int j = 0; j < kB; ++j) {
-            const int t = min(t0 + j, Qt - 1);
+            const int t = min(t0 + j * lph, Qt - 1);
             ci[j] = colinfo[i0 + t];
             mv[j] = __uint_as_float(cells[c0 + t]);
           }
 #pragma unroll
           for (int j = 0; j < kB; ++j) {
-            if (t0 + j >= Qt) break;
             const double e = K < static_cast<double>(ci[j].w)
                                  ? (static_cast<double>(ci[j].x) * K + static_cast<double>(ci[j].y)) * (1.0 + 0x1p-50)
                                  : static_cast<double>(INFINITY);
             const double m = static_cast<double>(mv[j]);
-            const double inv = 1.0 / static_cast<double>(ci[j].z);  // a power of two: exact
+            // the scale is a power of two: its inverse is exact
+            const double inv = static_cast<double>(1.0f / ci[j].z);
             const double lo = fmax(0.0, m - e) * inv;
             const double hi = (m + e) * inv;
             lo_h = fmax(lo_h, lo);
             hi_h = (hi > hi_h || isnan(hi)) ? hi : hi_h;
           }
         }
-        lo_sum += lo_h;
-        hi_sum += hi_h;
+        for (int off = 1; off < lph; off <<= 1) {
+          lo_h = fmax(lo_h, __shfl_xor(lo_h, off));
+          const double o = __shfl_xor(hi_h, off);
+          hi_h = (o > hi_h || isnan(o)) ? o : hi_h;
+        }
+        if (sl == 0) {
+          lo_sum += lo_h;
+          hi_sum += hi_h;
+        }
       }
 #pragma unroll
       for (int off = 1; off < kWave; off <<= 1) {
         lo_sum += __shfl_xor(lo_sum, off);
-        const double o = __shfl_xor(hi_sum, off);
-        hi_sum = isnan(o) ? o : hi_sum + o;
+        hi_sum += __shfl_xor(hi_sum, off);
       }
     }
+    if (lane == 0) {
+      s_sum[parity][wave][0] = lo_sum;
+      s_sum[parity][wave][1] = hi_sum;
+    }
+    __syncthreads();  // (the other parity's sums are read until the next one)
+    if (wave != 0) {
+      parity ^= 1;
+      continue;
+    }
+    lo_sum = hi_sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < kFinWaves; ++w) {
+      lo_sum += s_sum[parity][w][0];
+      hi_sum += s_sum[parity][w][1];
+    }
+    parity ^= 1;
     const double lb = lo_sum / denom / static_cast<double>(H) * (1.0 - 0x1p-40);
     const double ub = hi_sum / denom / static_cast<double>(H) * (1.0 + 0x1p-40);
     float lbf = __builtin_nanf(""), ubf = __builtin_nanf("");
@@ -1902,13 +1966,7 @@ __global__ __launch_bounds__(kFinWaves * kWave) void gqa_bounds_wide_kernel(
     if (lane == 0) lbub[static_cast<size_t>(qb) * cap + slot] = make_float2(lbf, ubf);
     wl_consume(Lw, k, lbf, id, slot, lane == 0 && isfinite(lbf) && isfinite(ubf) && lbf >= Lw.th_s);
   }
-  if (lane < kMaxTopK) s_lists[wave][lane] = wl_entry(Lw);
-  __syncthreads();
-  if (wave == 0) {
-    WaveList B;
-    block_merge(s_lists, kFinWaves, k, B);
-    if (lane < k) block_out[(static_cast<size_t>(qb) * nsblk + sblk) * k + lane] = wl_entry(B);
-  }
+  if (wave == 0 && lane < k) block_out[(static_cast<size_t>(qb) * nsblk + sblk) * k + lane] = wl_entry(Lw);
 }
 
 // The law on the candidates of a query of many tokens (one query, every
@@ -1924,7 +1982,15 @@ __global__ __launch_bounds__(kFinWaves * kWave) void gqa_bounds_wide_kernel(
 // unchanged: the column that holds it has an upper bound at or above every
 // column's lower bound.  A NaN bound keeps its column.  q64 holds the query
 // columns as doubles, value d of column gc at q64[(g*hd + d)*rqp + gc].
-// Wavefronts walk pairs p = w, w + W, ... (p = candidate * kv + g).
+// Blocks walk pairs p = b, b + gridDim.x, ... (p = candidate * kv + g); a
+// pair's tokens go to the block's wavefronts in runs of 64, each of which
+// finds the kept columns for itself (a few cached reads).
+//
+// Bound by latency, not by its fp64 sums: a few hundred pairs on the chip.
+// One wavefront per pair, one piece of a row in flight, took a trip to
+// memory per piece and 64 tokens; now the tokens are spread over four
+// wavefronts and 8 pieces are in flight: 72.2 -> 29.7 us (256 nodes of 16
+// to 512 tokens, 64 query tokens, 32 kv heads of 128).
 constexpr int kSparseCols = 4;  // columns evaluated per read of a pair's key rows
 template <int KDT>
 __global__ __launch_bounds__(kUnitWaves * kWave) void gqa_exact_sparse_kernel(
@@ -1939,18 +2005,17 @@ __global__ __launch_bounds__(kUnitWaves * kWave) void gqa_exact_sparse_kernel(
   extern __shared__ double s_qv[];  // [kUnitWaves][kSparseCols][hd]
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
-  const uint32_t W = gridDim.x * kUnitWaves;
   const uint32_t n_pairs = cand_count[0] * static_cast<uint32_t>(kv);
   const int C = hd / T::kEpc;
   const int G = KDT == kI8 ? hd / group_size : 1;
   const int cpg = KDT == kI8 ? group_size / T::kEpc : 1;
   const int ses = scale_dtype == kF16 ? 2 : 4;
-  for (uint32_t pr = blockIdx.x * kUnitWaves + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-       pr < n_pairs; pr += W) {
+  for (uint32_t pr = blockIdx.x; pr < n_pairs; pr += gridDim.x) {
     const uint32_t slot = cand_slots[pr / kv];
     const int g = static_cast<int>(pr % kv);
     const uint32_t L = lens[slot];
-    if (L == 0u) continue;
+    const uint32_t first = static_cast<uint32_t>(wave) * kWave;  // the wavefront's first token
+    if (first >= L) continue;
     const double K = screen_key_norm(__uint_as_float(kmax[slot]), fact != 0, hd);
     const unsigned* cells = hmaxf + (static_cast<size_t>(slot) * kv + g) * colstride;
     const float4* cinf = colinfo + static_cast<size_t>(g) * colstride;
@@ -2036,26 +2101,37 @@ __global__ __launch_bounds__(kUnitWaves * kWave) void gqa_exact_sparse_kernel(
       double best[kSparseCols];
 #pragma unroll
       for (int j = 0; j < kSparseCols; ++j) best[j] = 0.0;
-      for (uint32_t t0 = 0; t0 < L; t0 += kWave) {
+      for (uint32_t t0 = first; t0 < L; t0 += kUnitWaves * kWave) {
         const uint32_t t = min(t0 + static_cast<uint32_t>(lane), L - 1u);
         double acc[kSparseCols];
 #pragma unroll
         for (int j = 0; j < kSparseCols; ++j) acc[j] = 0.0;
-        for (int c = 0; c < C; ++c) {
-          const u32x4 v = piece_ptr(kb, Lp, sS, t, c)[0];
-          float sc = 0.0f;
-          if constexpr (KDT == kI8) {
-            sc = load_scale(scales + (row0 * G + t) * ses, scale_dtype,
-                            static_cast<uint64_t>(c / cpg) * Lp);
+        constexpr int kHold = 8;  // pieces of the row in flight
+        for (int c0 = 0; c0 < C; c0 += kHold) {
+          u32x4 v[kHold];
+          float sc[kHold];
+#pragma unroll
+          for (int i = 0; i < kHold; ++i) {
+            const int c = min(c0 + i, C - 1);
+            v[i] = piece_ptr(kb, Lp, sS, t, c)[0];
+            sc[i] = 0.0f;
+            if constexpr (KDT == kI8) {
+              sc[i] = load_scale(scales + (row0 * G + t) * ses, scale_dtype,
+                                 static_cast<uint64_t>(c / cpg) * Lp);
+            }
           }
-          float f[T::kEpc];
-          decode_chunk<KDT>(v, sc, f);
 #pragma unroll
-          for (int e = 0; e < T::kEpc; ++e) {
-            const double fe = static_cast<double>(f[e]);
-            const int d = c * T::kEpc + e;
+          for (int i = 0; i < kHold; ++i) {
+            if (c0 + i >= C) break;
+            float f[T::kEpc];
+            decode_chunk<KDT>(v[i], sc[i], f);
 #pragma unroll
-            for (int j = 0; j < kSparseCols; ++j) acc[j] = fma(fe, qv[j * hd + d], acc[j]);
+            for (int e = 0; e < T::kEpc; ++e) {
+              const double fe = static_cast<double>(f[e]);
+              const int d = (c0 + i) * T::kEpc + e;
+#pragma unroll
+              for (int j = 0; j < kSparseCols; ++j) acc[j] = fma(fe, qv[j * hd + d], acc[j]);
+            }
           }
         }
         if (t0 + lane < L) {

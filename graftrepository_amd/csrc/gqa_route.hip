@@ -1217,13 +1217,12 @@ int enqueue_bv(GqaDeviceArena* a, const SrPlan& p, const unsigned char* qptr, in
   const bool wide = H * p.Qt >= kWideCells;
   const uint32_t n_slots = static_cast<uint32_t>(a->high_water);
   // the bounds blocks, and so the candidates kernel's lists per query: a
-  // wavefront per slot (wide), else a lane per slot and about two rounds
+  // block per slot (wide), else a lane per slot and about two rounds
   // of slots per wavefront (a block's fixed cost -- column parameters,
   // list merge -- would dominate one round)
   constexpr uint32_t kBoundsSlots = 2 * grm::gqa::kFinWaves * grm::kWave;
   const uint32_t bblocks =
-      wide ? std::max<uint32_t>(1, std::min<uint32_t>(kWideBlocks, (n_slots + grm::gqa::kFinWaves - 1) /
-                                                                        grm::gqa::kFinWaves))
+      wide ? std::max<uint32_t>(1, std::min<uint32_t>(kWideBlocks, n_slots))
            : (std::max<uint32_t>(1, std::min<uint32_t>(fin_blocks, (n_slots + kBoundsSlots - 1) / kBoundsSlots)) +
               7u) / 8u * 8u;  // a multiple of 8 (the kernel's XCD mapping)
 #define GRM_BOUNDS(ST)                                                                           \
@@ -1264,7 +1263,7 @@ int enqueue_bv(GqaDeviceArena* a, const SrPlan& p, const unsigned char* qptr, in
   if (qb == 1 && a->sparse_exact) {
     const uint64_t pairs = a->cap_nodes * a->kv;
     const unsigned blocks = static_cast<unsigned>(
-        std::max<uint64_t>(1, std::min<uint64_t>((pairs + grm::gqa::kUnitWaves - 1) / grm::gqa::kUnitWaves, 2048)));
+        std::max<uint64_t>(1, std::min<uint64_t>(pairs, 2048)));  // a block per (candidate, kv head)
     const int rqp = rq_pad_of(p.R * p.Qt);
     const double denom = sqrt(static_cast<double>(a->hd));
 #define GRM_SPARSE(KDT)                                                                           \
