@@ -278,67 +278,133 @@ __global__ __launch_bounds__(kMaxNW * kWave) void mla_route_kernel(
 // NaN whatever its norm; such a row is stored as zeros with a NaN norm,
 // which every route scores NaN as well (0 / NaN), and which the batched
 // screen's products can then never overflow on.
+//
+// A row's norm is one fp64 chain in d order, so a row has one lane for it;
+// what bounds a batch of few rows is latency.  A block takes kPlaceRows
+// rows: its wavefronts load them along d into LDS, one wavefront runs the
+// chains from there while the others write the tiles.  (A thread per row,
+// loading value by value, took a trip to memory per value: 68 us for 1000
+// rows of 288, where these blocks take 8 to 15 us per 450 rows straight
+// from host memory.)  Rows longer than kPlaceCols go slice by slice, the chains'
+// sums carried along; values past dim are zeros, which leave a sum as it is.
+constexpr int kPlaceRows = 16;
+constexpr int kPlaceCols = 320;  // values per slice
+constexpr int kPlaceWaves = 4;
 template <int DT>
-__global__ void mla_place_rows_kernel(const void* __restrict__ rows,
-                                      uint64_t count, uint32_t dim,
-                                      uint32_t chunks, size_t plane,
-                                      const uint64_t* __restrict__ slots,
-                                      const uint64_t* __restrict__ ids,
-                                      uint64_t slot0, u32x4* __restrict__ tiles,
-                                      float* __restrict__ norms,
-                                      uint64_t* __restrict__ slot_ids,
-                                      unsigned* __restrict__ norm_range) {
+__global__ __launch_bounds__(kPlaceWaves * kWave) void mla_place_rows_kernel(
+    const void* __restrict__ rows, uint64_t count, uint32_t dim, uint32_t chunks, size_t plane,
+    const uint64_t* __restrict__ slots, const uint64_t* __restrict__ ids, uint64_t slot0,
+    u32x4* __restrict__ tiles, float* __restrict__ norms, uint64_t* __restrict__ slot_ids,
+    unsigned* __restrict__ norm_range) {
   constexpr int EPC = DT == kF32 ? 4 : 8;
-  for (uint64_t r = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
-       r < count; r += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
-    const uint64_t slot = slots ? slots[r] : slot0 + r;
-    const uint64_t tile = slot / kWave;
-    const uint32_t lane = static_cast<uint32_t>(slot % kWave);
-    u32x4* dst = tiles + tile * kWave + lane;
-    double acc = 0.0;
-    for (uint32_t c = 0; c < chunks; ++c) {
-      uint32_t w[4] = {0u, 0u, 0u, 0u};
-      for (int e = 0; e < EPC; ++e) {
-        const uint32_t d = c * EPC + e;
-        float f = 0.0f;
-        uint32_t bits = 0u;
-        if (d < dim) {
-          if constexpr (DT == kF32) {
-            f = static_cast<const float*>(rows)[r * dim + d];
-            bits = __float_as_uint(f);
-          } else {
-            bits = static_cast<const uint16_t*>(rows)[r * dim + d];
-            f = bf16_to_f32(bits);
-          }
-          acc = fma(static_cast<double>(f), static_cast<double>(f), acc);
-        }
-        if constexpr (DT == kF32) {
-          w[e] = bits;
-        } else {
-          w[e / 2] |= (e & 1) ? (bits << 16) : bits;
+  constexpr int kLoads = kPlaceCols / kWave;                // values per lane and row
+  constexpr int kRowsPerWave = kPlaceRows / kPlaceWaves;
+  // row stride: 16 lanes reading 16 bytes at one offset of 16 rows fall in
+  // distinct banks
+  constexpr int kStride = kPlaceCols + 4;
+  __shared__ __align__(16) float s_v[kPlaceRows][kStride];
+  __shared__ uint64_t s_slot[kPlaceRows];
+  __shared__ unsigned s_bad[kPlaceRows];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+  const uint32_t width = chunks * EPC;  // dim rounded up to whole pieces
+  for (uint64_t r0 = blockIdx.x * static_cast<uint64_t>(kPlaceRows); r0 < count;
+       r0 += static_cast<uint64_t>(gridDim.x) * kPlaceRows) {
+    const int n = static_cast<int>(min(static_cast<uint64_t>(kPlaceRows), count - r0));
+    if (static_cast<int>(threadIdx.x) < n) {
+      s_slot[threadIdx.x] = slots ? slots[r0 + threadIdx.x] : slot0 + r0 + threadIdx.x;
+    }
+    double acc = 0.0;  // wavefront 0: lane's row
+    for (uint32_t d0 = 0; d0 < width; d0 += kPlaceCols) {
+      float v[kRowsPerWave][kLoads];
+#pragma unroll
+      for (int i = 0; i < kRowsPerWave; ++i) {
+        const int r = wave + i * kPlaceWaves;
+        const uint64_t row = (r0 + static_cast<uint64_t>(min(r, n - 1))) * dim;
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+          const uint32_t d = d0 + static_cast<uint32_t>(j * kWave + lane);
+          const uint64_t src = row + min(d, dim - 1u);
+          const float f = DT == kF32 ? static_cast<const float*>(rows)[src]
+                                     : bf16_to_f32(static_cast<const uint16_t*>(rows)[src]);
+          v[i][j] = d < dim ? f : 0.0f;
         }
       }
-      u32x4 v;
-      v.x = w[0];
-      v.y = w[1];
-      v.z = w[2];
-      v.w = w[3];
-      dst[static_cast<size_t>(c) * plane] = v;
+#pragma unroll
+      for (int i = 0; i < kRowsPerWave; ++i) {
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) s_v[wave + i * kPlaceWaves][j * kWave + lane] = v[i][j];
+      }
+      __syncthreads();
+      const uint32_t w = min(width - d0, static_cast<uint32_t>(kPlaceCols));
+      if (wave == 0) {
+        if (lane < n) {
+          const float4* row = reinterpret_cast<const float4*>(s_v[lane]);
+#pragma unroll 4
+          for (uint32_t q = 0; q < w / 4; ++q) {
+            const float4 f = row[q];
+            acc = fma(static_cast<double>(f.x), static_cast<double>(f.x), acc);
+            acc = fma(static_cast<double>(f.y), static_cast<double>(f.y), acc);
+            acc = fma(static_cast<double>(f.z), static_cast<double>(f.z), acc);
+            acc = fma(static_cast<double>(f.w), static_cast<double>(f.w), acc);
+          }
+        }
+      } else {
+        for (uint32_t i = threadIdx.x - kWave; i < w / EPC * kPlaceRows;
+             i += (kPlaceWaves - 1) * kWave) {
+          const int r = static_cast<int>(i % kPlaceRows);
+          const uint32_t c = i / kPlaceRows;
+          if (r >= n) continue;
+          const float* f = s_v[r] + c * EPC;
+          u32x4 out;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            if constexpr (DT == kF32) {
+              out[e] = __float_as_uint(f[e]);
+            } else {
+              out[e] = (__float_as_uint(f[2 * e]) >> 16) | (__float_as_uint(f[2 * e + 1]) & 0xffff0000u);
+            }
+          }
+          const uint64_t slot = s_slot[r];
+          tiles[slot / kWave * kWave + slot % kWave + static_cast<size_t>(d0 / EPC + c) * plane] = out;
+        }
+      }
+      __syncthreads();  // the slice is read; the tiles' stores are ordered
     }
-    // squares of finite fp32 / bf16 values cannot overflow fp64
-    const bool finite_row = isfinite(acc);
-    if (!finite_row) {
-      const u32x4 zero = {0u, 0u, 0u, 0u};
-      for (uint32_t c = 0; c < chunks; ++c) dst[static_cast<size_t>(c) * plane] = zero;
+    if (wave == 0) {
+      // squares of finite fp32 / bf16 values cannot overflow fp64
+      const bool mine = lane < n;
+      const bool finite_row = isfinite(acc);
+      const float nf = finite_row ? static_cast<float>(sqrt(acc)) : __builtin_nanf("");
+      if (mine) {
+        s_bad[lane] = finite_row ? 0u : 1u;
+        const uint64_t slot = s_slot[lane];
+        norms[slot] = nf;
+        slot_ids[slot] = ids ? ids[r0 + lane] : slot;
+      }
+      // norm range (non-negative floats order like their bits)
+      const bool counts = mine && nf > 0.0f && isfinite(nf);
+      unsigned lo = counts ? __float_as_uint(nf) : 0xffffffffu;
+      unsigned hi = counts ? __float_as_uint(nf) : 0u;
+#pragma unroll
+      for (int off = 1; off < kPlaceRows; off <<= 1) {
+        lo = min(lo, static_cast<unsigned>(__shfl_xor(static_cast<int>(lo), off)));
+        hi = max(hi, static_cast<unsigned>(__shfl_xor(static_cast<int>(hi), off)));
+      }
+      if (lane == 0 && hi != 0u) {
+        atomicMin(norm_range, lo);
+        atomicMax(norm_range + 1, hi);
+      }
     }
-    const float nf = finite_row ? static_cast<float>(sqrt(acc)) : __builtin_nanf("");
-    norms[slot] = nf;
-    slot_ids[slot] = ids ? ids[r] : slot;
-    // norm range (non-negative floats order like their bits)
-    if (nf > 0.0f && isfinite(nf)) {
-      atomicMin(norm_range, __float_as_uint(nf));
-      atomicMax(norm_range + 1, __float_as_uint(nf));
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < chunks * kPlaceRows; i += kPlaceWaves * kWave) {
+      const int r = static_cast<int>(i % kPlaceRows);
+      if (r >= n || s_bad[r] == 0u) continue;
+      const uint64_t slot = s_slot[r];
+      tiles[slot / kWave * kWave + slot % kWave + static_cast<size_t>(i / kPlaceRows) * plane] =
+          u32x4{0u, 0u, 0u, 0u};
     }
+    __syncthreads();
   }
 }
 
@@ -524,9 +590,9 @@ int launch_place(MlaDeviceArena* a, const void* d_rows, uint64_t count,
                  const uint64_t* d_slots, const uint64_t* d_ids, uint64_t slot0,
                  hipStream_t stream) {
   if (count == 0) return 0;
-  const unsigned threads = 256;
+  const unsigned threads = grm::mla::kPlaceWaves * grm::kWave;
   const unsigned blocks = static_cast<unsigned>(
-      std::min<uint64_t>((count + threads - 1) / threads, 4096));
+      std::min<uint64_t>((count + grm::mla::kPlaceRows - 1) / grm::mla::kPlaceRows, 4096));
   if (a->dtype == kF32) {
     grm::mla::mla_place_rows_kernel<kF32><<<blocks, threads, 0, stream>>>(
         d_rows, count, a->dim, a->chunks, a->capacity, d_slots, d_ids, slot0,
