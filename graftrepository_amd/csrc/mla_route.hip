@@ -29,6 +29,7 @@
 // bound on the screen's rounding error and rescores the shortlist with the
 // exact law; queries without a certificate are routed again here.
 #include "grm_common.hpp"
+#include "slot_tables.hpp"
 #include "grm_hip_router.h"
 
 #include <stdlib.h>
@@ -38,8 +39,6 @@
 #include <atomic>
 #include <limits>
 #include <mutex>
-#include <set>
-#include <unordered_map>
 #include <vector>
 
 namespace grm {
@@ -433,6 +432,14 @@ using grm::mla::u32x4;
 
 // ------------------------------------------------------------------ host side
 
+// Rows and ids of one bank update on their way to the device: pinned host
+// memory, read by the update's kernels in place.  ev marks when they have.
+struct MutStage {
+  grm::MappedBuf buf;
+  hipEvent_t ev = nullptr;
+  bool pending = false;
+};
+
 struct MlaDeviceArena {
   int device = 0;
   int dtype = kF32;
@@ -449,8 +456,8 @@ struct MlaDeviceArena {
   float* d_norms = nullptr;
   uint64_t* d_ids = nullptr;
   std::vector<uint64_t> slot_id;  // kNoId when free
-  std::unordered_map<uint64_t, uint64_t> slot_of;
-  std::set<uint64_t> free_slots;  // freed slots below high_water
+  grm::IdTable slot_of;
+  grm::FreeSlots free_slots;  // freed slots below high_water
   void* d_queries = nullptr;
   size_t d_queries_bytes = 0;
   float* d_latent_q = nullptr;  // route key formed from a device latent (dim floats)
@@ -476,7 +483,11 @@ struct MlaDeviceArena {
   hipStream_t side = nullptr;
   hipEvent_t ev_start = nullptr;
   hipEvent_t ev_stop = nullptr;
-  hipEvent_t ev_mut = nullptr;
+  // updates take the two stages in turn, so one may be filled while the
+  // kernels of the other still read; both run on `side`, so the newer
+  // stage's event (mut[mut_last]) covers every update
+  MutStage mut[2];
+  int mut_last = 0;
   bool mut_pending = false;
   unsigned* d_min_norm = nullptr;  // [smallest positive, largest finite] row norm placed (float bits)
   // batched route: pass buffers and per-query results
@@ -543,7 +554,10 @@ void destroy_arena(MlaDeviceArena* a) {
   if (a->h_stage) (void)hipHostFree(a->h_stage);
   if (a->ev_start) (void)hipEventDestroy(a->ev_start);
   if (a->ev_stop) (void)hipEventDestroy(a->ev_stop);
-  if (a->ev_mut) (void)hipEventDestroy(a->ev_mut);
+  for (MutStage& m : a->mut) {
+    grm::release_mapped_bytes(&m.buf);
+    if (m.ev) (void)hipEventDestroy(m.ev);
+  }
   for (hipEvent_t e : a->screen_ev) (void)hipEventDestroy(e);
   if (a->stream) (void)hipStreamDestroy(a->stream);
   if (a->side) (void)hipStreamDestroy(a->side);
@@ -579,11 +593,17 @@ int reserve_pinned(T** ptr, size_t* have, size_t want) {
 
 int wait_mutations(MlaDeviceArena* a) {
   if (a->mut_pending) {
-    GRM_HIP_CHECK(hipEventSynchronize(a->ev_mut));
-    a->mut_pending = false;
+    GRM_HIP_CHECK(hipEventSynchronize(a->mut[a->mut_last].ev));
+    a->mut_pending = a->mut[0].pending = a->mut[1].pending = false;
   }
   return 0;
 }
+
+// Appends of up to this many bytes are placed straight from the pinned
+// stage, in parts of kAppendPartBytes (one launch each); larger ones keep
+// the copy engine, whose transfers do not hold compute units.
+constexpr size_t kDirectAppendBytes = 8u << 20;
+constexpr size_t kAppendPartBytes = 512u << 10;
 
 // Launch the placement kernel over `count` staged rows on `stream`.
 int launch_place(MlaDeviceArena* a, const void* d_rows, uint64_t count,
@@ -677,16 +697,16 @@ int create_arena(const void* rows, int dtype, uint64_t nodes, int dim,
     }
   }
   a->slot_id.assign(a->capacity, kNoId);
+  a->free_slots.resize(a->capacity);
+  a->slot_of.reserve(nodes);
   if (node_ids) {
-    a->slot_of.reserve(nodes * 2);
     for (uint64_t i = 0; i < nodes; ++i) {
-      if (!a->slot_of.emplace(node_ids[i], i).second) {
+      if (!a->slot_of.emplace(node_ids[i], i)) {
         return bail(grm::fail(-1, "duplicate node id"));
       }
       a->slot_id[i] = node_ids[i];
     }
   } else {
-    a->slot_of.reserve(nodes * 2);
     for (uint64_t i = 0; i < nodes; ++i) {
       a->slot_of.emplace(i, i);
       a->slot_id[i] = i;
@@ -703,7 +723,7 @@ int create_arena(const void* rows, int dtype, uint64_t nodes, int dim,
   BAIL_HIP(hipStreamCreateWithFlags(&a->side, hipStreamNonBlocking));
   BAIL_HIP(hipEventCreate(&a->ev_start));
   BAIL_HIP(hipEventCreate(&a->ev_stop));
-  BAIL_HIP(hipEventCreateWithFlags(&a->ev_mut, hipEventDisableTiming));
+  for (MutStage& m : a->mut) BAIL_HIP(hipEventCreateWithFlags(&m.ev, hipEventDisableTiming));
   BAIL_HIP(hipMalloc(reinterpret_cast<void**>(&a->d_tiles), tiles * tile_bytes));
   BAIL_HIP(hipMalloc(reinterpret_cast<void**>(&a->d_norms), a->capacity * sizeof(float)));
   BAIL_HIP(hipMalloc(reinterpret_cast<void**>(&a->d_ids), a->capacity * sizeof(uint64_t)));
@@ -1115,7 +1135,7 @@ int route_impl(MlaDeviceArena* a, const void* queries, int q_dtype,
     }
     qbase = static_cast<const unsigned char*>(a->d_queries);
   }
-  if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->ev_mut, 0));
+  if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->mut[a->mut_last].ev, 0));
   const size_t qstride = static_cast<size_t>(a->dim) * elem_size(q_dtype);
   BatchPlan bp;
   const bool batched = !a->no_batch && batch_plan(a, q_count - warmup, &bp) && reserve_batch(a, bp);
@@ -1279,6 +1299,28 @@ int route_impl(MlaDeviceArena* a, const void* queries, int q_dtype,
     }
   }
   grm::clear_error();
+  return 0;
+}
+
+// The next update's stage, of at least `bytes`, once the kernels of the
+// update before the last have read it.
+int next_stage(MlaDeviceArena* a, size_t bytes, MutStage** out) {
+  MutStage& m = a->mut[a->mut_last ^ 1];
+  if (m.pending) {
+    GRM_HIP_CHECK(hipEventSynchronize(m.ev));
+    m.pending = false;
+  }
+  GRM_CHECK_RC(grm::reserve_mapped_bytes(&m.buf, bytes));
+  *out = &m;
+  return 0;
+}
+
+// The update's kernels are all on the side stream.
+int end_update(MlaDeviceArena* a, MutStage* m) {
+  GRM_HIP_CHECK(hipEventRecord(m->ev, a->side));
+  m->pending = true;
+  a->mut_last ^= 1;
+  a->mut_pending = true;
   return 0;
 }
 
@@ -1576,7 +1618,7 @@ int route_noalloc(MlaDeviceArena* a, const void* d_queries, int q_dtype, int q_c
   const size_t qstride = static_cast<size_t>(a->dim) * elem_size(q_dtype);
   const unsigned char* qbase = static_cast<const unsigned char*>(d_queries);
   auto launch_all = [&]() -> int {
-    if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->ev_mut, 0));
+    if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->mut[a->mut_last].ev, 0));
     for (int qi = 0; qi < q_count; ++qi) {
       GRM_CHECK_RC(launch_single(a, g, qbase + qi * qstride, q_dtype, topk, lists));
       mla_merge_out_kernel<<<1, grm::kMergeWaves * grm::kWave, 0, a->stream>>>(
@@ -1743,9 +1785,9 @@ extern "C" int grm_mla_hip_set_filter_bits(MlaDeviceArena* a, const uint64_t* no
   std::vector<uint64_t> pairs;
   pairs.reserve(2 * count);
   for (uint64_t i = 0; i < count; ++i) {
-    auto it = a->slot_of.find(node_ids[i]);
-    if (it == a->slot_of.end()) return grm::fail(-1, "filter bits for an id that is not live");
-    pairs.push_back(it->second);
+    const uint64_t* slot = a->slot_of.find(node_ids[i]);
+    if (!slot) return grm::fail(-1, "filter bits for an id that is not live");
+    pairs.push_back(*slot);
     pairs.push_back(bits[i]);
   }
   GRM_HIP_CHECK(hipSetDevice(a->device));
@@ -1791,7 +1833,7 @@ extern "C" int grm_mla_hip_route_filtered(MlaDeviceArena* a, const void* query, 
                             a->capacity * sizeof(uint64_t)));
     GRM_HIP_CHECK(hipMemsetAsync(a->d_fbits, 0, a->capacity * sizeof(uint64_t), a->stream));
   }
-  if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->ev_mut, 0));
+  if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->mut[a->mut_last].ev, 0));
   // every slot the route scans: whole 64-slot tiles up to the high water
   // (capacity is a multiple of 64; the tail slots stay NaN)
   const uint64_t n = (a->high_water + grm::kWave - 1) / grm::kWave * grm::kWave;
@@ -1831,9 +1873,9 @@ extern "C" int grm_mla_hip_score_nodes(MlaDeviceArena* a, const void* query_host
   if (count == 0) return 0;
   std::vector<uint64_t> slots(count);
   for (uint64_t i = 0; i < count; ++i) {
-    auto it = a->slot_of.find(node_ids[i]);
-    if (it == a->slot_of.end()) return grm::fail(-1, "score of an id that is not live");
-    slots[i] = it->second;
+    const uint64_t* slot = a->slot_of.find(node_ids[i]);
+    if (!slot) return grm::fail(-1, "score of an id that is not live");
+    slots[i] = *slot;
   }
   GRM_HIP_CHECK(hipSetDevice(a->device));
   GRM_CHECK_RC(wait_mutations(a));
@@ -1885,50 +1927,74 @@ extern "C" int grm_mla_hip_append(MlaDeviceArena* a, const void* rows_host,
     if (out_epoch) *out_epoch = a->epoch;
     return 0;
   }
-  {
-    std::unordered_map<uint64_t, int> seen;
-    seen.reserve(count * 2);
-    for (uint64_t i = 0; i < count; ++i) {
-      if (a->slot_of.count(node_ids[i]) || !seen.emplace(node_ids[i], 1).second) {
-        return grm::fail(-1, "append id already live or repeated");
-      }
-      if (node_ids[i] == kNoId) return grm::fail(-1, "node id UINT64_MAX is reserved");
+  // the ids enter the table at once, which finds live and repeated ones,
+  // and leave it again if the append does not come about
+  struct Entered {
+    MlaDeviceArena* a;
+    const uint64_t* ids;
+    uint64_t n = 0;
+    ~Entered() {
+      for (uint64_t i = 0; i < n; ++i) a->slot_of.erase(ids[i]);
     }
+  } entered{a, node_ids};
+  a->slot_of.reserve(a->slot_of.size() + count);
+  for (uint64_t i = 0; i < count; ++i) {
+    if (!a->slot_of.emplace(node_ids[i], 0)) {
+      return grm::fail(-1, "append id already live or repeated");
+    }
+    entered.n = i + 1;
+    if (node_ids[i] == kNoId) return grm::fail(-1, "node id UINT64_MAX is reserved");
   }
   const uint64_t room = a->free_slots.size() + (a->capacity - a->high_water);
   if (count > room) return grm::fail(-3, "MLA bank capacity exceeded");
   GRM_HIP_CHECK(hipSetDevice(a->device));
   const size_t row_bytes = static_cast<size_t>(a->dim) * elem_size(a->dtype);
   const size_t bytes = count * (2 * sizeof(uint64_t) + row_bytes);
-  void* h = nullptr;
-  void* d = nullptr;
-  GRM_CHECK_RC(stage_upload(a, bytes, &h, &d));
-  uint64_t* h_slots = static_cast<uint64_t*>(h);
+  MutStage* stage = nullptr;
+  GRM_CHECK_RC(next_stage(a, bytes, &stage));
+  uint64_t* h_slots = static_cast<uint64_t*>(static_cast<void*>(stage->buf.host));
   uint64_t* h_ids = h_slots + count;
   unsigned char* h_rows = reinterpret_cast<unsigned char*>(h_ids + count);
-  std::vector<uint64_t> taken;
-  taken.reserve(count);
+  entered.n = 0;
   for (uint64_t i = 0; i < count; ++i) {
-    uint64_t slot;
-    if (!a->free_slots.empty()) {
-      slot = *a->free_slots.begin();
-      a->free_slots.erase(a->free_slots.begin());
-    } else {
-      slot = a->high_water++;
-    }
+    uint64_t slot = a->free_slots.pop_lowest();
+    if (slot == kNoId) slot = a->high_water++;
     h_slots[i] = slot;
     h_ids[i] = node_ids[i];
     a->slot_id[slot] = node_ids[i];
-    a->slot_of[node_ids[i]] = slot;
+    *a->slot_of.find(node_ids[i]) = slot;
   }
-  memcpy(h_rows, rows_host, count * row_bytes);
-  uint64_t* d_slots = static_cast<uint64_t*>(d);
-  uint64_t* d_ids = d_slots + count;
-  unsigned char* d_rows = reinterpret_cast<unsigned char*>(d_ids + count);
-  GRM_HIP_CHECK(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, a->side));
-  GRM_CHECK_RC(launch_place(a, d_rows, count, d_slots, d_ids, 0, a->side));
-  GRM_HIP_CHECK(hipEventRecord(a->ev_mut, a->side));
-  a->mut_pending = true;
+  if (bytes <= kDirectAppendBytes) {
+    // The placement reads the rows over the bus itself, in parts that
+    // follow the host's copy: no copy on the device side, and the bus is
+    // busy while the host still copies.  1000 rows of 288 fp32 values out
+    // and in, then a route over 100k: 370 -> 123 us a call, with the
+    // placement kernel, the flat tables and the second stage (an append no
+    // longer waits for the evict's kernel).  The parts' launches take 8 to
+    // 15 us each, the bus's time for 512 KiB.
+    const uint64_t part = std::max<uint64_t>(grm::mla::kPlaceRows,
+                                             kAppendPartBytes / row_bytes / grm::mla::kPlaceRows *
+                                                 grm::mla::kPlaceRows);
+    const uint64_t* s_slots = static_cast<const uint64_t*>(static_cast<const void*>(stage->buf.dev));
+    const unsigned char* s_rows = reinterpret_cast<const unsigned char*>(s_slots + 2 * count);
+    for (uint64_t r0 = 0; r0 < count; r0 += part) {
+      const uint64_t n = std::min<uint64_t>(part, count - r0);
+      memcpy(h_rows + r0 * row_bytes, static_cast<const unsigned char*>(rows_host) + r0 * row_bytes,
+             n * row_bytes);
+      GRM_CHECK_RC(launch_place(a, s_rows + r0 * row_bytes, n, s_slots + r0, s_slots + count + r0, 0, a->side));
+    }
+  } else {
+    memcpy(h_rows, rows_host, count * row_bytes);
+    // the device copy is shared by every large append: its last reader is
+    // on the same stream; growing it waits for that
+    if (bytes > a->d_stage_bytes) GRM_CHECK_RC(wait_mutations(a));
+    GRM_CHECK_RC(reserve_device(reinterpret_cast<unsigned char**>(&a->d_stage), &a->d_stage_bytes, bytes));
+    GRM_HIP_CHECK(hipMemcpyAsync(a->d_stage, stage->buf.host, bytes, hipMemcpyHostToDevice, a->side));
+    uint64_t* d_slots = static_cast<uint64_t*>(a->d_stage);
+    uint64_t* d_ids = d_slots + count;
+    GRM_CHECK_RC(launch_place(a, d_ids + count, count, d_slots, d_ids, 0, a->side));
+  }
+  GRM_CHECK_RC(end_update(a, stage));
   a->live += count;
   a->epoch += 1;
   if (out_epoch) *out_epoch = a->epoch;
@@ -1943,26 +2009,32 @@ extern "C" int grm_mla_hip_evict(MlaDeviceArena* a, const uint64_t* node_ids,
     if (out_epoch) *out_epoch = a->epoch;
     return 0;
   }
-  std::vector<uint64_t> slots;
-  slots.reserve(count);
-  {
-    std::unordered_map<uint64_t, int> seen;
-    seen.reserve(count * 2);
-    for (uint64_t i = 0; i < count; ++i) {
-      auto it = a->slot_of.find(node_ids[i]);
-      if (it == a->slot_of.end() || !seen.emplace(node_ids[i], 1).second) {
-        return grm::fail(-1, "evict id not live or repeated");
-      }
-      slots.push_back(it->second);
+  // the slots are marked free at once, which finds repeated ids, and
+  // unmarked again if the evict does not come about
+  struct Marked {
+    MlaDeviceArena* a;
+    std::vector<uint64_t> slots;
+    bool keep = false;
+    ~Marked() {
+      if (keep) return;
+      for (uint64_t s : slots) a->free_slots.erase(s);
     }
+  } marked{a, {}};
+  marked.slots.reserve(count);
+  for (uint64_t i = 0; i < count; ++i) {
+    const uint64_t* slot = a->slot_of.find(node_ids[i]);
+    if (!slot || !a->free_slots.insert(*slot)) {
+      return grm::fail(-1, "evict id not live or repeated");
+    }
+    marked.slots.push_back(*slot);
   }
+  const std::vector<uint64_t>& slots = marked.slots;
   GRM_HIP_CHECK(hipSetDevice(a->device));
   const size_t bytes = count * sizeof(uint64_t);
-  void* h = nullptr;
-  void* d = nullptr;
-  GRM_CHECK_RC(stage_upload(a, bytes, &h, &d));
-  memcpy(h, slots.data(), bytes);
-  GRM_HIP_CHECK(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, a->side));
+  MutStage* stage = nullptr;
+  GRM_CHECK_RC(next_stage(a, bytes, &stage));
+  void* d = stage->buf.dev;  // read in place by the kernels
+  memcpy(stage->buf.host, slots.data(), bytes);
   const unsigned threads = 256;
   const unsigned blocks = static_cast<unsigned>(std::min<uint64_t>((count + threads - 1) / threads, 1024));
   grm::mla::mla_evict_kernel<<<blocks, threads, 0, a->side>>>(
@@ -1974,12 +2046,11 @@ extern "C" int grm_mla_hip_evict(MlaDeviceArena* a, const uint64_t* node_ids,
                                                           a->d_fbits);
     GRM_HIP_CHECK(hipGetLastError());
   }
-  GRM_HIP_CHECK(hipEventRecord(a->ev_mut, a->side));
-  a->mut_pending = true;
+  GRM_CHECK_RC(end_update(a, stage));
+  marked.keep = true;
   for (uint64_t s : slots) {
     a->slot_of.erase(a->slot_id[s]);
     a->slot_id[s] = kNoId;
-    a->free_slots.insert(s);
   }
   // Trailing free slots shrink the scanned range.
   while (a->high_water > 0 && a->slot_id[a->high_water - 1] == kNoId) {
@@ -2064,7 +2135,7 @@ extern "C" int grm_mla_hip_probe_screen(MlaDeviceArena* a, const void* queries_h
   GRM_HIP_CHECK(hipMalloc(&d_vals.p, static_cast<size_t>(query_count) * n * sizeof(float)));
   GRM_HIP_CHECK(hipMalloc(&d_bounds.p, static_cast<size_t>(query_count) * sizeof(double)));
   if (!reserve_batch(a, p)) return grm::fail(-1, "no memory for the probe's buffers");
-  if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->ev_mut, 0));
+  if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->mut[a->mut_last].ev, 0));
   GRM_HIP_CHECK(hipMemcpyAsync(d_q.p, queries_host, qbytes, hipMemcpyHostToDevice, a->stream));
   const PassQueries pq{d_q.p, query_dtype, query_count};
   GRM_CHECK_RC(launch_screen<true>(a, p, shape, pq, static_cast<uint32_t*>(d_planes.p), PassMarks{}));
