@@ -1282,16 +1282,47 @@ __global__ __launch_bounds__(kUnitWaves * kWave, (sr_waves_per_simd<KDT, KS, NT,
 // scores < tau, in float as well (lb rounded down, ub rounded up), so the
 // top-k of the candidates is the law's top-k, ties included.
 
-// Maximum over the 16 lanes of a DPP row (lanes 16j .. 16j + 15), in every
-// lane of the row: quad_perm [1,0,3,2] and [2,3,0,1] give each lane its
-// quad's maximum, row_half_mirror (lane i of 8 reads lane 7 - i) the other
-// quad's, row_mirror (lane i of 16 reads lane 15 - i) the other half's.
-__device__ inline uint32_t row_max16(uint32_t x) {
-  x = max(x, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0xB1, 0xF, 0xF, false)));
-  x = max(x, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x4E, 0xF, 0xF, false)));
-  x = max(x, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x141, 0xF, 0xF, false)));
-  x = max(x, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x140, 0xF, 0xF, false)));
-  return x;
+// Exchange with another lane of a DPP row (16 lanes): STEP 0 is lane i and
+// 15 - i (row_mirror), 1 lane i and 7 - i of each half (row_half_mirror),
+// 2 lanes two apart in a quad, 3 neighbours.  In each step the partners
+// differ in bit 3 - STEP of the lane number, and agree in the bits above it.
+template <int STEP>
+__device__ inline uint32_t row_exchange(uint32_t x) {
+  constexpr int kCtrl = STEP == 0 ? 0x140 : (STEP == 1 ? 0x141 : (STEP == 2 ? 0x4E : 0xB1));
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), kCtrl, 0xF, 0xF, false));
+}
+
+// One step of row_max16x: of N values halved by lane bit 3 - STEP while
+// there are more than the remaining steps need, else a plain maximum.
+template <int N, int STEP>
+__device__ inline void row_max_step(uint32_t* x, int r16) {
+  if constexpr (N == (1 << (4 - STEP))) {
+    const bool up = (r16 >> (3 - STEP)) & 1;
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+      const uint32_t give = up ? x[i] : x[i + N / 2];
+      const uint32_t keep = up ? x[i + N / 2] : x[i];
+      x[i] = max(keep, row_exchange<STEP>(give));
+    }
+    if constexpr (STEP < 3) row_max_step<N / 2, STEP + 1>(x, r16);
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = max(x[i], row_exchange<STEP>(x[i]));
+    if constexpr (STEP < 3) row_max_step<N, STEP + 1>(x, r16);
+  }
+}
+
+// Maxima of N (4, 8 or 16) values over the 16 lanes of each DPP row: lane
+// r16 of the row returns value r16 % N's.  A step exchanges half of the
+// values that are left, so 16 values take 15 exchanges, not 64.
+// (With the running maxima's one instruction per value and the turning item
+// order, see gqa_smax_kernel: 185.0 -> 180.1 us for 4 passes of a 64-token
+// query over 256 bf16 nodes, 240.1 -> 234.4 for 16 queries over 4000 INT8
+// nodes; the vector instructions fell from 57 to 34 per tile and pass.)
+template <int N>
+__device__ inline uint32_t row_max16x(uint32_t (&x)[N], int r16) {
+  row_max_step<N, 0>(x, r16);
+  return x[0];
 }
 
 // Four stored int8 codes (one dword) as four exact f16 values (two dwords,
@@ -1311,10 +1342,13 @@ struct SmaxPasses {
   int r0[4], rc[4], t0[4], qc[4];
 };
 
-// Screen-only pass; grid (P, kv heads), persistent: wave w of block b walks
-// the work items b*4 + w, b*4 + w + 4P, ... -- one item per live node with
-// key tokens, all of its tokens, so each (node, kv head) has one writer --
-// as one stream of 16-token tiles,
+// Screen-only pass; grid (P, kv heads), persistent: of the S = 4P waves of
+// a kv head, wave w walks the work items w, 2S-1-w, 2S+w, 4S-1-w, ... --
+// one item per live node with key tokens, all of its tokens, so each (node,
+// kv head) has one writer; the list falls in token count, and turning back
+// each round keeps the waves' totals within about half an item's spread
+// (always the same direction gave wave 0 the longest item of every round)
+// -- as one stream of 16-token tiles,
 // four tiles in flight ahead of the one being screened, across item
 // boundaries.  The block stages kv head g's query columns once
 // (stage_columns); blocks with blockIdx.x == 0 write colinfo[g*cols + cg]
@@ -1442,7 +1476,9 @@ __global__ __launch_bounds__((NP == 1 ? kUnitWaves : 8) * kWave,
   };
   Src ld = source(items[has_item ? li : 0]);
   uint32_t lt = 0;
-  uint32_t lnext = li + stride;
+  // to the next round's item, there and back
+  uint32_t to_next = 2 * (stride - li) - 1, to_after = 2 * li + 1;
+  uint32_t lnext = li + to_next;
   Item nx = items[min(lnext, n_items - 1)];
   bool ldone = false;
   auto load_tile = [&](Tile& b, uint32_t tile) {
@@ -1491,7 +1527,10 @@ __global__ __launch_bounds__((NP == 1 ? kUnitWaves : 8) * kWave,
     }
     ld = source(nx);
     lt = 0;
-    lnext += stride;
+    const uint32_t hop = to_after;
+    to_after = to_next;
+    to_next = hop;
+    lnext += hop;
     nx = items[min(lnext, n_items - 1)];
   };
   Tile x0, x1, x2, x3, x4;
@@ -1564,15 +1603,21 @@ __global__ __launch_bounds__((NP == 1 ? kUnitWaves : 8) * kWave,
     }
   };
   // running maxima as float bits: the values are non-negative, so their
-  // bit patterns order like the values (a NaN, possible only from
-  // non-finite keys or query values, wins; such a node or query is never
-  // ranked, by its flags)
+  // bit patterns order like the values (a NaN comes only from non-finite
+  // keys or query values, whose node or query is never ranked, by its
+  // flags, or from an overflow, which E = +inf allows for; it may or may
+  // not reach the maximum)
   uint32_t m[NT][4];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) m[nt][v] = 0u;
   }
+  // +inf as the compiler cannot know it (it would turn the medians below
+  // back into canonicalising maxima)
+  uint32_t inf_bits = 0x7f800000u;
+  asm("" : "+s"(inf_bits));
+  const float inf = __uint_as_float(inf_bits);
   auto fold = [&](const Tile& b) {
     f32x4 c[NH][NT];
     float sc[NH];
@@ -1594,11 +1639,17 @@ __global__ __launch_bounds__((NP == 1 ? kUnitWaves : 8) * kWave,
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const float x0 = FACT ? fabsf(c[0][nt][v]) * sc[0] : fabsf(c[0][nt][v]);
-        if constexpr (NH == 2) {
-          const float x1 = FACT ? fabsf(c[1][nt][v]) * sc[1] : fabsf(c[1][nt][v]);
+        if constexpr (FACT && NH == 2) {
+          const float x1 = fabsf(c[1][nt][v]) * sc[1];
           m[nt][v] = max(max(m[nt][v], __float_as_uint(x0)), __float_as_uint(x1));  // v_max3_u32
         } else {
-          m[nt][v] = max(m[nt][v], __float_as_uint(x0));
+          // median of (m, |x|, inf) = max(m, |x|): one instruction, which
+          // takes the magnitude as an operand modifier (the compiler's
+          // float maximum canonicalises x first, an integer one needs the
+          // sign bit cleared)
+          float mx = __builtin_amdgcn_fmed3f(__uint_as_float(m[nt][v]), x0, inf);
+          if constexpr (NH == 2) mx = __builtin_amdgcn_fmed3f(mx, fabsf(c[1][nt][v]), inf);
+          m[nt][v] = __float_as_uint(mx);
         }
       }
     }
@@ -1617,27 +1668,17 @@ __global__ __launch_bounds__((NP == 1 ? kUnitWaves : 8) * kWave,
     my_gc[i] = my_col[i] ? full_col(cg) : 0;
   }
   auto emit = [&](uint32_t slot) {
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        m[nt][v] = row_max16(m[nt][v]);
-      }
-    }
-    uint32_t mine[kStores];
-#pragma unroll
-    for (int i = 0; i < kStores; ++i) mine[i] = 0u;
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        if (r16 == (nt % 4) * 4 + v) mine[nt / 4] = m[nt][v];
-        m[nt][v] = 0u;
-      }
-    }
+    constexpr int kGroup = NT < 4 ? NT : 4;  // column blocks of one store
 #pragma unroll
     for (int i = 0; i < kStores; ++i) {
-      if (my_col[i]) hmaxf[(static_cast<size_t>(slot) * kv + g) * colstride + my_gc[i]] = mine[i];
+      uint32_t x[kGroup * 4];
+#pragma unroll
+      for (int j = 0; j < kGroup * 4; ++j) {
+        x[j] = m[i * 4 + j / 4][j % 4];
+        m[i * 4 + j / 4][j % 4] = 0u;
+      }
+      const uint32_t mine = row_max16x(x, r16);
+      if (my_col[i]) hmaxf[(static_cast<size_t>(slot) * kv + g) * colstride + my_gc[i]] = mine;
     }
   };
   // Groups of five steps with one exit, at the bottom: steps after the
