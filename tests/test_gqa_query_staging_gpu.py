@@ -42,3 +42,32 @@ def test_query_alignment(hip_lib, hd, dtype, shift, queries, tokens, group):
     ids, sc, _ = oracle.gqa_route(keys, oracle.BF16, offs, kv, hd, q, 5)
     np.testing.assert_array_equal(res.ids, ids)
     np.testing.assert_array_equal(res.scores.view(np.uint32), sc.view(np.uint32))
+
+
+# Four query passes to a launch, the nodes dealt to the wavefronts there and
+# back: one node, fewer nodes than wavefronts, several to a wavefront, nodes
+# from one token to 700; passes that are full and, with 3 heads and 5 tokens
+# past four passes, that are not
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("nodes,hi", [(1, 9), (5, 40), (90, 40), (20, 700)])
+@pytest.mark.parametrize("hd,group,tokens", [(64, 4, 64), (128, 4, 64), (128, 3, 89)])
+def test_four_pass_screen(hip_lib, hd, group, tokens, nodes, hi, dtype):
+    kv = 32
+    lens = wl.gqa_lengths(nodes, hd + nodes, lo=1, hi=hi)
+    keys, offs = wl.gqa_bank(lens, kv, hd, 5, dtype="f32")
+    if dtype == "f16":
+        keys = keys.astype(np.float16)
+        values = keys.astype(np.float32)
+    elif dtype == "bf16":
+        keys = (keys.view(np.uint32) >> 16).astype(np.uint16)
+        values = bf16_bits_to_f32(keys).reshape(keys.shape)
+    else:
+        values = keys
+    q = np.random.default_rng(7).standard_normal((1, kv * group, tokens, hd), dtype=np.float32)
+    k = min(4, nodes)
+    bits = keys.view(np.uint16) if dtype == "f16" else keys
+    with GqaNodeBank(bits, offs, kv_heads=kv, head_dim=hd, dtype=dtype) as bank:
+        res = bank.route(q, k, timed=False)
+    ids, sc, _ = oracle.gqa_route(values, oracle.F32, offs, kv, hd, q, k)
+    np.testing.assert_array_equal(res.ids, ids)
+    np.testing.assert_array_equal(res.scores.view(np.uint32), sc.view(np.uint32))
