@@ -410,7 +410,7 @@ def bench_mla_batched(steps: int, warmup: int, cpu_queries: int, traffic: dict |
     flops = 2.0 * nq * n * d
     bytes_screen = n * d * 2 + n * 4
     # the screen kernel bench.py's bank takes: the LDS-ring screen unless
-    # GRM_HIP_BATCH_RING=0 selects the previous one (not profiled)
+    # GRM_HIP_BATCH_RING=0 selects the stream screen (not profiled)
     ring = os.environ.get("GRM_HIP_BATCH_RING", "1") != "0"
     prof = (traffic or {}).get("mla_batch_ring", {}) if ring else {}
     scr = float(np.mean(screens))
@@ -431,7 +431,7 @@ def bench_mla_batched(steps: int, warmup: int, cpu_queries: int, traffic: dict |
                      "unit": "TFLOP/s", "frac": round(tflops / 2500.0, 4),
                      "traffic": prof.get("fetch_bytes"),
                      "mfma_util_counters": prof.get("mfma_util"),
-                     "kernel": "mla_batch_ring_kernel<18>" if ring else "mla_batch_screen_kernel<18, 8>",
+                     "kernel": "mla_batch_ring_kernel<18>" if ring else "mla_batch_stream_kernel",
                      "flops_per_launch": flops, "kernel_ms_mean": round(scr, 5)},
         "roofline_hbm": {"achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": round(gbs / HBM_PEAK_GBS, 4),
@@ -1279,7 +1279,7 @@ def main() -> int:
                          "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": round(m["achieved"] / HBM_PEAK_GBS, 4),
                          "traffic": traffic.get("mla_route", {}).get("bytes_per_launch"),
-                         "kernel": "mla_route_pipe_kernel<f32, 16, 9>",
+                         "kernel": "mla_route_kernel<f32, 9, 16>",
                          "bytes_per_launch": m["bytes"]},
         }
     if g is not None:
