@@ -228,12 +228,16 @@ __global__ __launch_bounds__(kBatchWaves * kWave) void mla_batch_stream_kernel(
   // merge (rounding is monotone, so the largest u give the largest s~).
   // A slot that never ranks (tombstone, unused slot, non-finite row: the
   // bank stores its row as zeros) has 1/norm_f = -0, so u is a zero and
-  // never outranks a positive value.  The accumulation cannot overflow
-  // where the merge certifies (it checks the norms), so a u that is not
-  // finite comes from a query that the merge never certifies.  u's low
-  // bits take the slot code, and the three largest move by two medians and
-  // a maximum of the integer bits: b3 = med3(b2, b3, v),
-  // b2 = med3(b1, b2, v), b1 = max(b1, v) keep b1 >= b2 >= b3 the three
+  // never outranks a positive value.  An accumulation may overflow only
+  // where the merge does not certify (it checks the norms), or on a row
+  // whose own norm overflowed (a law score of zero; the norms' range leaves
+  // it out): its u is then a NaN.  One with a set sign bit, as gfx950 forms
+  // it, lies below +0 in the integer order and decides nothing; one with a
+  // clear sign bit would lie above every number, and so be its sub-stream's
+  // largest, which voids the query's certificate.  u's low bits take the
+  // slot code, and the three largest move by two medians and a maximum of
+  // the integer bits: b3 = med3(b2, b3, v), b2 = med3(b1, b2, v),
+  // b1 = max(b1, v) keep b1 >= b2 >= b3 the three
   // largest values seen.
   auto offer = [&](int v, int ct) {
     med3_i32_into(b2[ct], b3[ct], v);
@@ -953,16 +957,18 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
     }
   }
   if (tid == 0) s_count = 0u;
-  bool pinf = false;
+  bool over = false;
   if (wave != kMergeWavesB - 1) {
-    // largest finite kept s~ of the thread; a +inf s~ voids the certificate
+    // largest finite kept s~ of the thread; a +inf s~ voids the certificate,
+    // and so does a NaN u that lies above every number (see the screen): it
+    // may have pushed real entries out of its sub-stream
     float m = -INFINITY;
 #pragma unroll
     for (int j = 0; j < kMergePer; ++j) {
       const float v1 = u1[j] * iq, v2 = u2[j] * iq;
       if (isfinite(v1)) m = fmaxf(m, v1);
       if (isfinite(v2)) m = fmaxf(m, v2);
-      pinf = pinf || v1 == INFINITY || v2 == INFINITY;
+      over = over || v1 == INFINITY || v2 == INFINITY || __float_as_int(u1[j]) >= 0x7f800000;
     }
     const float ms = wave_sort_desc(m);
 #pragma unroll
@@ -970,7 +976,7 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
     if (lane == k - 1) s_lw[wave] = ms;
     if (lane == 0) s_nk[wave] = nk;
   }
-  const int any_pinf = __syncthreads_or(pinf ? 1 : 0);
+  const int any_over = __syncthreads_or(over ? 1 : 0);
 
   const double nmax = static_cast<double>(__uint_as_float(norm_range[1]));
   const double bound = s_bound;
@@ -1070,7 +1076,7 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
   const double t = static_cast<double>(vk) - 2.0 * bound - 0x1p-40;
   // t > 0: the screen kept its values by their integer bits, the float
   // order only from +0 up.
-  const bool pre = any_pinf == 0 && count <= static_cast<unsigned>(kSurvMax) && n >= k &&
+  const bool pre = any_over == 0 && count <= static_cast<unsigned>(kSurvMax) && n >= k &&
                    static_cast<double>(nk_all) < t && t > 0.0 && screen_in_range(s_qhi, nmax);
   // the rescored prefix: ranks [0, n_el)
   if (tid < n_el) {

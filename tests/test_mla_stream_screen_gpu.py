@@ -118,6 +118,29 @@ def test_rows_the_screen_cannot_certify(hip_lib):
         check(bank, rows, qs, 6)
 
 
+# the stream screen's column tiles, and the ring (200 bf16 queries)
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("nq", [2, 3, 40, 200])
+@pytest.mark.parametrize("dim", [64, 600])
+def test_rows_whose_norm_overflows(hip_lib, dim, nq, dtype):
+    # Four rows that score 0 by the law (an infinite norm) in one tile with
+    # some queries' best row: their screened values are NaN and must not
+    # push that row out.  Slots 1, 2, 9 and 18 share a lane half with 10, 11
+    # and 16, 17.
+    rng = np.random.default_rng(nq + dim)
+    rows = rng.standard_normal((9000, dim)).astype(np.float32)
+    qs = rng.standard_normal((nq, dim)).astype(np.float32)
+    for slot, query in zip((10, 11, 16, 17), range(nq)):
+        rows[slot] = qs[query] + 0.1 * rows[slot]
+    for slot in (1, 2, 9, 18):
+        rows[slot] = np.float32(3.38e38 if dtype == "bf16" else 3.4e38) * np.sign(rows[slot])
+    bits = as_bf16_bits(rows) if dtype == "bf16" else rows
+    qb = as_bf16_bits(qs) if dtype == "bf16" else qs
+    with MlaNodeBank(bits, dtype=dtype) as bank:
+        check(bank, bits, qb, 6, query_dtype=dtype)
+        assert bank.route_stats()["batched"] == nq
+
+
 @pytest.mark.parametrize("adversarial", [False, True])
 @pytest.mark.parametrize("count,dim", [(80, 288), (30, 570)])
 def test_fp32_screen_obeys_its_bound(hip_lib, adversarial, count, dim):
