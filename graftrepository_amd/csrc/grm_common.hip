@@ -26,6 +26,8 @@ int fail_hip(hipError_t rc, const char* what) {
   msg += ": ";
   msg += hipGetErrorString(rc);
   g_last_error = msg;
+  // reported here: the check after the next kernel launch must not find it
+  (void)hipGetLastError();
   return hip_code(rc);
 }
 

@@ -1,0 +1,176 @@
+"""Bank updates whose HIP calls fail.
+
+The route library's host code runs here against a stand-in for the HIP
+runtime (device memory is host memory, kernels do not run except that row
+placement and eviction set norms and ids), which can be told to fail the
+n-th call of a function from now on."""
+
+import subprocess
+import sys
+
+import pytest
+
+from graftrepository_amd import _lib
+
+RUNTIME = r"""
+#include <math.h>
+#include <stdint.h>
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+typedef struct { uint32_t x, y, z; } dim3;
+static char fail_name[64];
+static int fail_in;
+void fake_fail(const char* name, int nth) { snprintf(fail_name, 64, "%s", name); fail_in = nth; }
+int fake_failed(void) { return fail_in == 0; }
+static int last;
+static int fails(const char* name) {
+  if (strcmp(name, fail_name) != 0 || fail_in == 0 || --fail_in > 0) return 0;
+  return last = 2;
+}
+#define CALL(name) if (fails(#name)) return 2
+static size_t pinned, device;
+size_t fake_pinned(void) { return pinned; }
+size_t fake_device(void) { return device; }
+static void* take(size_t n, size_t* sum) {
+  size_t* p = calloc(1, n + 64);
+  *p = n;
+  *sum += n;
+  return p + 8;
+}
+static int give(void* q, size_t* sum) {
+  if (q) { size_t* p = (size_t*)q - 8; *sum -= *p; free(p); }
+  return 0;
+}
+int hipMalloc(void** p, size_t n) { CALL(hipMalloc); *p = take(n, &device); return 0; }
+int hipHostMalloc(void** p, size_t n, unsigned f) { CALL(hipHostMalloc); *p = take(n, &pinned); return 0; }
+int hipFree(void* p) { return give(p, &device); }
+int hipHostFree(void* p) { return give(p, &pinned); }
+int hipHostGetDevicePointer(void** d, void* h, unsigned f) { *d = h; return 0; }
+int hipMemcpyAsync(void* d, const void* s, size_t n, int k, void* q) { CALL(hipMemcpyAsync); memcpy(d, s, n); return 0; }
+int hipMemcpy(void* d, const void* s, size_t n, int k) { memcpy(d, s, n); return 0; }
+int hipMemsetAsync(void* d, int v, size_t n, void* q) { memset(d, v, n); return 0; }
+int hipGetDevice(int* d) { *d = 0; return 0; }
+int hipSetDevice(int d) { return 0; }
+int hipDeviceGetAttribute(int* v, int a, int d) { *v = 0; return 1; }
+int hipStreamCreateWithFlags(void** s, unsigned f) { *s = malloc(1); return 0; }
+int hipStreamDestroy(void* s) { free(s); return 0; }
+int hipStreamSynchronize(void* s) { return 0; }
+int hipStreamWaitEvent(void* s, void* e, unsigned f) { return 0; }
+int hipEventCreate(void** e) { *e = malloc(1); return 0; }
+int hipEventCreateWithFlags(void** e, unsigned f) { *e = malloc(1); return 0; }
+int hipEventDestroy(void* e) { free(e); return 0; }
+int hipEventRecord(void* e, void* s) { CALL(hipEventRecord); return 0; }
+int hipEventSynchronize(void* e) { return 0; }
+int hipEventQuery(void* e) { return 0; }
+int hipEventElapsedTime(float* ms, void* a, void* b) { *ms = 1.0f; return 0; }
+int hipFuncSetAttribute(const void* f, int a, int v) { return 0; }
+int hipGetLastError(void) { const int e = last; last = 0; return e; }
+const char* hipGetErrorString(int e) { return "stand-in failure"; }
+static struct { const void* host; const char* name; } kernels[4096];
+static int n_kernels;
+void** __hipRegisterFatBinary(const void* d) { static void* m[1]; return m; }
+void __hipUnregisterFatBinary(void** m) {}
+void __hipRegisterFunction(void** m, const void* host, char* dev, const char* name, unsigned t,
+                           void* a, void* b, void* c, void* d, int* e) {
+  kernels[n_kernels].host = host;
+  kernels[n_kernels++].name = strdup(name);
+}
+void __hipRegisterVar(void** m, void* v, char* h, char* d, int e, size_t n, int c, int g) {}
+static struct { dim3 g, b; size_t lds; void* s; } pushed;
+int __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, void* s) {
+  pushed.g = g; pushed.b = b; pushed.lds = lds; pushed.s = s;
+  return 0;
+}
+int __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, void** s) {
+  *g = pushed.g; *b = pushed.b; *lds = pushed.lds; *s = pushed.s;
+  return 0;
+}
+static float* norms;
+static uint64_t* ids;
+#define ARG(i, T) (*(T*)args[i])
+int hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t lds, void* s) {
+  const char* name = "";
+  for (int i = 0; i < n_kernels; ++i) if (kernels[i].host == f) name = kernels[i].name;
+  CALL(hipLaunchKernel);
+  if (strstr(name, "mla_place_rows_kernel")) {
+    const uint64_t* slots = ARG(5, const uint64_t*);
+    const uint64_t* from = ARG(6, const uint64_t*);
+    norms = ARG(9, float*);
+    ids = ARG(10, uint64_t*);
+    for (uint64_t r = 0; r < ARG(1, uint64_t); ++r) {
+      const uint64_t slot = slots ? slots[r] : ARG(7, uint64_t) + r;
+      norms[slot] = 1.0f;
+      ids[slot] = from ? from[r] : slot;
+    }
+  }
+  if (strstr(name, "mla_evict_kernel")) {
+    for (uint64_t r = 0; r < ARG(1, uint64_t); ++r) {
+      ARG(2, float*)[ARG(0, const uint64_t*)[r]] = NAN;
+      ARG(3, uint64_t*)[ARG(0, const uint64_t*)[r]] = ~0ull;
+    }
+  }
+  return 0;
+}
+/* ids of the slots below n whose norm is a number, in slot order */
+uint64_t fake_live(uint64_t n, uint64_t* out) {
+  uint64_t k = 0;
+  for (uint64_t i = 0; i < n; ++i) if (norms[i] == norms[i]) out[k++] = ids[i];
+  return k;
+}
+"""
+
+# run in a process of its own: loading the stand-in first binds the library to it
+PRELUDE = r"""
+import ctypes, sys
+hip = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+for f in (hip.fake_live, hip.fake_pinned, hip.fake_device):
+    f.restype = ctypes.c_uint64
+import numpy as np
+from graftrepository_amd import MlaNodeBank
+CAP = 20_032
+
+def fail(name, nth=1):
+    hip.fake_fail(name.encode(), nth)
+
+def device_ids():
+    out = np.empty(CAP, np.uint64)
+    n = hip.fake_live(ctypes.c_uint64(CAP), out.ctypes.data_as(ctypes.c_void_p))
+    return sorted(out[:n].tolist())
+
+def refused(call, *args):
+    try:
+        call(*args)
+    except RuntimeError:
+        assert hip.fake_failed()
+        return
+    raise AssertionError("the call did not fail")
+
+def state(bank):
+    i = bank.info()
+    return i["live"], i["epoch"], i["slots_in_use"], device_ids()
+"""
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    d = tmp_path_factory.mktemp("hip")
+    (d / "hip.c").write_text(RUNTIME)
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-w", str(d / "hip.c"), "-o", str(d / "hip.so"), "-lm"],
+                   check=True)
+    return d / "hip.so"
+
+
+def run(runtime, body):
+    root = _lib.PKG.parent
+    subprocess.run([sys.executable, "-c", PRELUDE + body, str(runtime)], check=True, cwd=root, timeout=120)
+
+
+def test_a_failure_is_reported_once(runtime):
+    run(runtime, r"""
+with MlaNodeBank(np.ones((100, 32), np.float32), capacity=CAP) as bank:
+    fail("hipHostMalloc")
+    refused(bank.evict, np.asarray([5, 7], np.uint64))
+    bank.evict(np.asarray([5, 7], np.uint64))  # its launch succeeds
+    assert state(bank)[0] == 98
+""")
