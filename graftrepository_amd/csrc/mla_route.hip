@@ -1315,9 +1315,14 @@ int next_stage(MlaDeviceArena* a, size_t bytes, MutStage** out) {
   return 0;
 }
 
-// The update's kernels are all on the side stream.
+// The update's kernels are all on the side stream.  Without an event to mark
+// their end, they are waited for.
 int end_update(MlaDeviceArena* a, MutStage* m) {
-  GRM_HIP_CHECK(hipEventRecord(m->ev, a->side));
+  if (hipEventRecord(m->ev, a->side) != hipSuccess) {
+    (void)hipGetLastError();
+    GRM_HIP_CHECK(hipStreamSynchronize(a->side));
+    return 0;
+  }
   m->pending = true;
   a->mut_last ^= 1;
   a->mut_pending = true;
@@ -1512,6 +1517,20 @@ __global__ __launch_bounds__(256) void mla_score_slots_kernel(
     const float sc = static_cast<float>(acc / (qnorm * static_cast<double>(nrm) + 1.0e-8));
     out[i] = isfinite(sc) ? sc : __builtin_nanf("");
   }
+}
+
+// Evict the `count` slots at d_slots on the side stream.
+int launch_evict(MlaDeviceArena* a, const uint64_t* d_slots, uint64_t count) {
+  const unsigned threads = 256;
+  const unsigned blocks = static_cast<unsigned>(std::min<uint64_t>((count + threads - 1) / threads, 1024));
+  grm::mla::mla_evict_kernel<<<blocks, threads, 0, a->side>>>(d_slots, count, a->d_norms, a->d_ids);
+  GRM_HIP_CHECK(hipGetLastError());
+  if (a->d_fbits) {
+    // a slot reused by a later append starts with no filter bits
+    mla_zero_bits_kernel<<<blocks, threads, 0, a->side>>>(d_slots, count, a->d_fbits);
+    GRM_HIP_CHECK(hipGetLastError());
+  }
+  return 0;
 }
 
 int enqueue_latent_query(MlaDeviceArena* a, const void* d_latent, int dtype, uint64_t tokens,
@@ -1927,13 +1946,27 @@ extern "C" int grm_mla_hip_append(MlaDeviceArena* a, const void* rows_host,
     if (out_epoch) *out_epoch = a->epoch;
     return 0;
   }
-  // the ids enter the table at once, which finds live and repeated ones,
-  // and leave it again if the append does not come about
+  // The ids enter the table at once, which finds live and repeated ones.
+  // An append that does not come about leaves nothing behind: what it put
+  // into the tables goes, and rows already placed are evicted.
   struct Entered {
     MlaDeviceArena* a;
     const uint64_t* ids;
-    uint64_t n = 0;
+    uint64_t n = 0;            // ids in the table
+    MutStage* stage = nullptr;
+    const uint64_t* slots = nullptr;  // the slots taken, in order (in the stage)
+    uint64_t taken = 0;
+    uint64_t high_water = 0;   // before the first was
     ~Entered() {
+      if (taken > 0) {
+        (void)launch_evict(a, static_cast<const uint64_t*>(stage->buf.dev), taken);
+        (void)hipStreamSynchronize(a->side);  // the stage is read no more
+      }
+      for (uint64_t i = 0; i < taken; ++i) {
+        a->slot_id[slots[i]] = kNoId;
+        if (slots[i] < high_water) a->free_slots.insert(slots[i]);
+      }
+      if (taken > 0) a->high_water = high_water;
       for (uint64_t i = 0; i < n; ++i) a->slot_of.erase(ids[i]);
     }
   } entered{a, node_ids};
@@ -1950,12 +1983,21 @@ extern "C" int grm_mla_hip_append(MlaDeviceArena* a, const void* rows_host,
   GRM_HIP_CHECK(hipSetDevice(a->device));
   const size_t row_bytes = static_cast<size_t>(a->dim) * elem_size(a->dtype);
   const size_t bytes = count * (2 * sizeof(uint64_t) + row_bytes);
+  const bool direct = bytes <= kDirectAppendBytes;
   MutStage* stage = nullptr;
   GRM_CHECK_RC(next_stage(a, bytes, &stage));
+  if (!direct) {
+    // the device copy is shared by every large append: its last reader is
+    // on the same stream; growing it waits for that
+    if (bytes > a->d_stage_bytes) GRM_CHECK_RC(wait_mutations(a));
+    GRM_CHECK_RC(reserve_device(reinterpret_cast<unsigned char**>(&a->d_stage), &a->d_stage_bytes, bytes));
+  }
   uint64_t* h_slots = static_cast<uint64_t*>(static_cast<void*>(stage->buf.host));
   uint64_t* h_ids = h_slots + count;
   unsigned char* h_rows = reinterpret_cast<unsigned char*>(h_ids + count);
-  entered.n = 0;
+  entered.stage = stage;
+  entered.slots = h_slots;
+  entered.high_water = a->high_water;
   for (uint64_t i = 0; i < count; ++i) {
     uint64_t slot = a->free_slots.pop_lowest();
     if (slot == kNoId) slot = a->high_water++;
@@ -1963,8 +2005,9 @@ extern "C" int grm_mla_hip_append(MlaDeviceArena* a, const void* rows_host,
     h_ids[i] = node_ids[i];
     a->slot_id[slot] = node_ids[i];
     *a->slot_of.find(node_ids[i]) = slot;
+    entered.taken = i + 1;
   }
-  if (bytes <= kDirectAppendBytes) {
+  if (direct) {
     // The placement reads the rows over the bus itself, in parts that
     // follow the host's copy: no copy on the device side, and the bus is
     // busy while the host still copies.  1000 rows of 288 fp32 values out
@@ -1985,16 +2028,13 @@ extern "C" int grm_mla_hip_append(MlaDeviceArena* a, const void* rows_host,
     }
   } else {
     memcpy(h_rows, rows_host, count * row_bytes);
-    // the device copy is shared by every large append: its last reader is
-    // on the same stream; growing it waits for that
-    if (bytes > a->d_stage_bytes) GRM_CHECK_RC(wait_mutations(a));
-    GRM_CHECK_RC(reserve_device(reinterpret_cast<unsigned char**>(&a->d_stage), &a->d_stage_bytes, bytes));
     GRM_HIP_CHECK(hipMemcpyAsync(a->d_stage, stage->buf.host, bytes, hipMemcpyHostToDevice, a->side));
     uint64_t* d_slots = static_cast<uint64_t*>(a->d_stage);
     uint64_t* d_ids = d_slots + count;
     GRM_CHECK_RC(launch_place(a, d_ids + count, count, d_slots, d_ids, 0, a->side));
   }
   GRM_CHECK_RC(end_update(a, stage));
+  entered.n = entered.taken = 0;
   a->live += count;
   a->epoch += 1;
   if (out_epoch) *out_epoch = a->epoch;
@@ -2014,9 +2054,11 @@ extern "C" int grm_mla_hip_evict(MlaDeviceArena* a, const uint64_t* node_ids,
   struct Marked {
     MlaDeviceArena* a;
     std::vector<uint64_t> slots;
+    bool staged = false;
     bool keep = false;
     ~Marked() {
       if (keep) return;
+      if (staged) (void)hipStreamSynchronize(a->side);  // the stage is read no more
       for (uint64_t s : slots) a->free_slots.erase(s);
     }
   } marked{a, {}};
@@ -2033,19 +2075,9 @@ extern "C" int grm_mla_hip_evict(MlaDeviceArena* a, const uint64_t* node_ids,
   const size_t bytes = count * sizeof(uint64_t);
   MutStage* stage = nullptr;
   GRM_CHECK_RC(next_stage(a, bytes, &stage));
-  void* d = stage->buf.dev;  // read in place by the kernels
   memcpy(stage->buf.host, slots.data(), bytes);
-  const unsigned threads = 256;
-  const unsigned blocks = static_cast<unsigned>(std::min<uint64_t>((count + threads - 1) / threads, 1024));
-  grm::mla::mla_evict_kernel<<<blocks, threads, 0, a->side>>>(
-      static_cast<const uint64_t*>(d), count, a->d_norms, a->d_ids);
-  GRM_HIP_CHECK(hipGetLastError());
-  if (a->d_fbits) {
-    // a slot reused by a later append starts with no filter bits
-    mla_zero_bits_kernel<<<blocks, threads, 0, a->side>>>(static_cast<const uint64_t*>(d), count,
-                                                          a->d_fbits);
-    GRM_HIP_CHECK(hipGetLastError());
-  }
+  marked.staged = true;
+  GRM_CHECK_RC(launch_evict(a, static_cast<const uint64_t*>(stage->buf.dev), count));  // read in place
   GRM_CHECK_RC(end_update(a, stage));
   marked.keep = true;
   for (uint64_t s : slots) {

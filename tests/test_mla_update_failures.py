@@ -1,4 +1,4 @@
-"""Bank updates whose HIP calls fail.
+"""Bank updates whose HIP calls fail leave the bank as it was.
 
 The route library's host code runs here against a stand-in for the HIP
 runtime (device memory is host memory, kernels do not run except that row
@@ -173,4 +173,60 @@ with MlaNodeBank(np.ones((100, 32), np.float32), capacity=CAP) as bank:
     refused(bank.evict, np.asarray([5, 7], np.uint64))
     bank.evict(np.asarray([5, 7], np.uint64))  # its launch succeeds
     assert state(bank)[0] == 98
+""")
+APPEND = r"""
+COUNT, WHAT, NTH = {count}, "{what}", {nth}
+rows = np.ones((100, 288), np.float32)
+new = np.ones((COUNT, 288), np.float32)
+ids = np.arange(COUNT, dtype=np.uint64) + 1000
+with MlaNodeBank(rows, capacity=CAP) as bank:
+    bank.evict(np.asarray([3, 50, 98, 99], np.uint64))  # holes and a tail
+    before = state(bank)
+    assert before[0] == 96 and before[2] == 98
+    fail(WHAT, NTH)
+    refused(bank.append, new, ids)
+    assert state(bank) == before, (state(bank)[:3], before[:3])
+    bank.append(new, ids)  # not "already live"
+    after = state(bank)
+    assert after[0] == 96 + COUNT and after[1] == before[1] + 1 and after[2] == 96 + COUNT
+    assert after[3] == sorted(before[3] + ids.tolist())
+    bank.evict(ids)
+    assert state(bank)[3] == before[3] and state(bank)[0] == 96
+"""
+
+
+# 2,000 rows: placed from the stage in parts; 9,000: through the copy engine
+@pytest.mark.parametrize("count,what,nth", [
+    (2_000, "hipHostMalloc", 1), (2_000, "hipLaunchKernel", 1), (2_000, "hipLaunchKernel", 3),
+    (9_000, "hipHostMalloc", 1), (9_000, "hipMalloc", 1), (9_000, "hipMemcpyAsync", 1),
+    (9_000, "hipLaunchKernel", 1)])
+def test_failed_append_changes_nothing(runtime, count, what, nth):
+    run(runtime, APPEND.format(count=count, what=what, nth=nth))
+
+
+def test_failed_evict_changes_nothing(runtime):
+    run(runtime, r"""
+with MlaNodeBank(np.ones((100, 32), np.float32), capacity=CAP) as bank:
+    for what in ("hipHostMalloc", "hipLaunchKernel"):
+        before = state(bank)
+        fail(what)
+        refused(bank.evict, np.asarray([5, 7], np.uint64))
+        assert state(bank) == before
+        bank.evict(np.asarray([5, 7], np.uint64))
+        assert state(bank)[0] == before[0] - 2
+        bank.append(np.ones((2, 32), np.float32), np.asarray([5, 7], np.uint64))
+""")
+
+
+# an update whose event cannot be recorded waits for its kernels instead
+def test_update_without_its_event(runtime):
+    run(runtime, r"""
+with MlaNodeBank(np.ones((100, 32), np.float32), capacity=CAP) as bank:
+    fail("hipEventRecord")
+    bank.evict(np.asarray([5, 7], np.uint64))
+    assert hip.fake_failed()
+    fail("hipEventRecord")
+    bank.append(np.ones((2, 32), np.float32), np.asarray([200, 201], np.uint64))
+    assert hip.fake_failed()
+    assert state(bank)[0] == 100 and state(bank)[3] == sorted([i for i in range(100) if i not in (5, 7)] + [200, 201])
 """)
