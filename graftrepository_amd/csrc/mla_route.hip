@@ -942,9 +942,9 @@ PassShape pass_shape(const MlaDeviceArena* a, const BatchPlan& p, int qc) {
   return {false, qc <= 32 ? 32 : (qc <= 64 ? 64 : 128), p.subs, p.ibits};
 }
 
-// The ring screen's slot weights, formed again when the bank changed.
+// The ring screen's slot weights (reserve_batch has their memory), formed
+// again when the bank changed.
 int ensure_weights(MlaDeviceArena* a) {
-  GRM_CHECK_RC(reserve_device(&a->d_winv, &a->d_winv_count, static_cast<size_t>(a->capacity)));
   if (a->winv_epoch != a->epoch) {
     const unsigned blocks = static_cast<unsigned>((a->capacity + 255) / 256);
     grm::mla::mla_batch_weights_kernel<<<blocks, 256, 0, a->stream>>>(a->d_norms, a->capacity,
@@ -1087,14 +1087,21 @@ int enqueue_batch_pass(MlaDeviceArena* a, const BatchPlan& p, const PassQueries&
   return 0;
 }
 
-// Buffers of the batched route.  False when the device has no room for
-// them: the queries then go one by one.
-bool reserve_batch(MlaDeviceArena* a, const BatchPlan& p) {
-  const size_t cols = std::max(p.qp_stream, p.qp_max);
+// Whether a segment of `queries` has a pass for the ring screen.
+bool has_ring_pass(const BatchPlan& p, int queries) {
+  return std::min(queries, p.qp_max) > grm::mla::kStreamMaxCols;
+}
+
+// Buffers of the batched route, with those of the ring screen where it has
+// a pass.  False when the device has no room for them: the queries then go
+// one by one.
+bool reserve_batch(MlaDeviceArena* a, const BatchPlan& p, bool ring) {
+  const size_t cols = ring ? p.qp_max : p.qp_stream;
   size_t subs = p.subs * static_cast<size_t>(p.qp_stream);
-  if (p.ring) subs = std::max<size_t>(subs, a->cus * size_t{2 * grm::mla::kRingSegs} * p.qp_max);
+  if (ring) subs = std::max<size_t>(subs, a->cus * size_t{2 * grm::mla::kRingSegs} * p.qp_max);
   const bool ok =
-      (!p.ring || reserve_device(&a->d_qpad, &a->d_qpad_count, cols * (16 * p.ks_ring + 8)) == 0) &&
+      (!ring || (reserve_device(&a->d_winv, &a->d_winv_count, static_cast<size_t>(a->capacity)) == 0 &&
+                 reserve_device(&a->d_qpad, &a->d_qpad_count, cols * (16 * p.ks_ring + 8)) == 0)) &&
       reserve_device(&a->d_inv_qn, &a->d_inv_qn_count, cols) == 0 &&
       reserve_device(&a->d_entries, &a->d_entries_count, grm::mla::kEntryPlanes * subs) == 0;
   if (!ok) (void)hipGetLastError();
@@ -1138,7 +1145,8 @@ int route_impl(MlaDeviceArena* a, const void* queries, int q_dtype,
   if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->mut[a->mut_last].ev, 0));
   const size_t qstride = static_cast<size_t>(a->dim) * elem_size(q_dtype);
   BatchPlan bp;
-  const bool batched = !a->no_batch && batch_plan(a, q_count - warmup, &bp) && reserve_batch(a, bp);
+  const bool batched = !a->no_batch && batch_plan(a, q_count - warmup, &bp) &&
+                       reserve_batch(a, bp, has_ring_pass(bp, std::max(warmup, q_count - warmup)));
   a->screen_ms = 0.0f;
   std::vector<int> redo;  // queries for the single-query kernel
   if (batched) {
@@ -2166,7 +2174,7 @@ extern "C" int grm_mla_hip_probe_screen(MlaDeviceArena* a, const void* queries_h
   GRM_HIP_CHECK(hipMalloc(&d_planes.p, static_cast<size_t>(qp) * a->capacity * sizeof(uint32_t)));
   GRM_HIP_CHECK(hipMalloc(&d_vals.p, static_cast<size_t>(query_count) * n * sizeof(float)));
   GRM_HIP_CHECK(hipMalloc(&d_bounds.p, static_cast<size_t>(query_count) * sizeof(double)));
-  if (!reserve_batch(a, p)) return grm::fail(-1, "no memory for the probe's buffers");
+  if (!reserve_batch(a, p, shape.ring)) return grm::fail(-1, "no memory for the probe's buffers");
   if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->mut[a->mut_last].ev, 0));
   GRM_HIP_CHECK(hipMemcpyAsync(d_q.p, queries_host, qbytes, hipMemcpyHostToDevice, a->stream));
   const PassQueries pq{d_q.p, query_dtype, query_count};

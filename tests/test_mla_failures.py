@@ -1,4 +1,5 @@
-"""Bank updates whose HIP calls fail leave the bank as it was.
+"""Calls on a bank whose HIP calls fail: an update leaves the bank as it was,
+a batched route without memory goes query by query.
 
 The route library's host code runs here against a stand-in for the HIP
 runtime (device memory is host memory, kernels do not run except that row
@@ -52,7 +53,8 @@ int hipMemcpy(void* d, const void* s, size_t n, int k) { memcpy(d, s, n); return
 int hipMemsetAsync(void* d, int v, size_t n, void* q) { memset(d, v, n); return 0; }
 int hipGetDevice(int* d) { *d = 0; return 0; }
 int hipSetDevice(int d) { return 0; }
-int hipDeviceGetAttribute(int* v, int a, int d) { *v = 0; return 1; }
+/* LDS a block may have (hipDeviceAttributeSharedMemPerBlockOptin); no clock */
+int hipDeviceGetAttribute(int* v, int a, int d) { *v = a == 75 ? 163840 : 0; return *v == 0; }
 int hipStreamCreateWithFlags(void** s, unsigned f) { *s = malloc(1); return 0; }
 int hipStreamDestroy(void* s) { free(s); return 0; }
 int hipStreamSynchronize(void* s) { return 0; }
@@ -229,4 +231,28 @@ with MlaNodeBank(np.ones((100, 32), np.float32), capacity=CAP) as bank:
     bank.append(np.ones((2, 32), np.float32), np.asarray([200, 201], np.uint64))
     assert hip.fake_failed()
     assert state(bank)[0] == 100 and state(bank)[3] == sorted([i for i in range(100) if i not in (5, 7)] + [200, 201])
+""")
+
+
+# each buffer of the batched route in turn; the ring screen takes 200 bf16 queries
+@pytest.mark.parametrize("dtype,nq,buffers", [("f32", 8, 2), ("bf16", 200, 4)])
+def test_batched_route_without_memory(runtime, dtype, nq, buffers):
+    run(runtime, f"""
+import os
+os.environ["GRM_HIP_BLOCKING_SYNC"] = "1"  # kernels do not run: no flags
+dtype, nq = "{dtype}", {nq}
+rows = np.ones((20_000, 64), np.float32 if dtype == "f32" else np.uint16)
+q = np.ones((nq, 64), rows.dtype)
+for nth in range(1, {buffers} + 2):
+    with MlaNodeBank(rows, dtype=dtype) as bank:
+        bank.route(q[:1], 3, query_dtype=dtype)  # the single-query route's buffers
+        bank.route(np.ones((nq, 64), rows.dtype), 3, query_dtype=dtype, warmup=nq - 1)
+        assert bank.route_stats()["batched"] == 0
+        fail("hipMalloc", nth)
+        bank.route(q, 3, query_dtype=dtype)
+        stats = bank.route_stats()
+        if nth <= {buffers}:
+            assert hip.fake_failed() and stats["batched"] == 0, (nth, stats)
+        else:
+            assert not hip.fake_failed() and stats["batched"] == nq, (nth, stats)
 """)
