@@ -169,20 +169,24 @@ int stamps_elapsed(const MappedBuf& buf, unsigned seq, size_t first, size_t n, h
   std::atomic_thread_fence(std::memory_order_acquire);
   const unsigned long long t0 = st[0];
   unsigned long long t1 = t0;
-  // A timed block's end tick below t0 is an earlier route's (the stream
-  // ran those kernels before this route's first timed one started); it is
-  // replaced before the route's event completes.
+  // A timed block's end tick below t0 may be an earlier route's, which is
+  // replaced before the route's event completes.  It may also be the
+  // route's own: block 0 stamps the start, and a block of a few microseconds
+  // on another XCD can be through before block 0 gets that far.  Once the
+  // event has completed every tick is the route's.
   bool stale = false;
   for (size_t i = first; i < n; ++i) stale |= st[kStampHead + i] < t0;
   if (stale) {
     GRM_CHECK_RC(wait_event(ev));
     std::atomic_thread_fence(std::memory_order_acquire);
   }
+  bool ended = false;  // block 0 itself ends after the start
   for (size_t i = first; i < n; ++i) {
     const unsigned long long e = st[kStampHead + i];
-    if (e < t0) return fail(-1, "route finished without its end stamps");
+    ended |= e >= t0;
     if (e > t1) t1 = e;
   }
+  if (!ended) return fail(-1, "route finished without its end stamps");
   *ms = static_cast<float>(static_cast<double>(t1 - t0) / ticks_per_ms);
   return 0;
 }

@@ -361,8 +361,10 @@ int wait_tagged(const Cand* entries, size_t n, unsigned seq, hipEvent_t ev);
 // end tick of the timed flags [first, n) less the start tick, at
 // `ticks_per_ms`.  As with list entries, the host may see a flag before
 // the stores ahead of it: a start stamp of another route, or a timed end
-// tick below the start tick (an earlier route's), is waited for through
-// `ev` and is an error if the kernels end without the new one.
+// tick below the start tick (an earlier route's, or of a block that ended
+// before block 0 stamped the start), is waited for through `ev`; it is an
+// error if the kernels end without the new start stamp, or with no end tick
+// after it.
 // wall_ticks_per_ms: the constant clock's rate on `device` (0 when the
 // device does not report it; such routes keep stream events).
 int reserve_stamps(MappedBuf* buf, size_t max);

@@ -53,8 +53,12 @@ int hipMemcpy(void* d, const void* s, size_t n, int k) { memcpy(d, s, n); return
 int hipMemsetAsync(void* d, int v, size_t n, void* q) { memset(d, v, n); return 0; }
 int hipGetDevice(int* d) { *d = 0; return 0; }
 int hipSetDevice(int d) { return 0; }
-/* LDS a block may have (hipDeviceAttributeSharedMemPerBlockOptin); no clock */
-int hipDeviceGetAttribute(int* v, int a, int d) { *v = a == 75 ? 163840 : 0; return *v == 0; }
+/* LDS a block may have (hipDeviceAttributeSharedMemPerBlockOptin), and the
+   device clock's kHz (hipDeviceAttributeWallClockRate) */
+int hipDeviceGetAttribute(int* v, int a, int d) {
+  *v = a == 75 ? 163840 : (a == 10017 ? 100000 : 0);
+  return *v == 0;
+}
 int hipStreamCreateWithFlags(void** s, unsigned f) { *s = malloc(1); return 0; }
 int hipStreamDestroy(void* s) { free(s); return 0; }
 int hipStreamSynchronize(void* s) { return 0; }
@@ -90,6 +94,10 @@ int __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, void** s) {
 }
 static float* norms;
 static uint64_t* ids;
+static uint64_t end_tick[4];
+void fake_ticks(uint64_t a, uint64_t b, uint64_t c, uint64_t d) {
+  end_tick[0] = a; end_tick[1] = b; end_tick[2] = c; end_tick[3] = d;
+}
 #define ARG(i, T) (*(T*)args[i])
 int hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t lds, void* s) {
   const char* name = "";
@@ -104,6 +112,21 @@ int hipLaunchKernel(const void* f, dim3 g, dim3 b, void** args, size_t lds, void
       const uint64_t slot = slots ? slots[r] : ARG(7, uint64_t) + r;
       norms[slot] = 1.0f;
       ids[slot] = from ? from[r] : slot;
+    }
+  }
+  if (strstr(name, "mla_route_kernel") && ARG(11, unsigned*)) {
+    /* no node found; the blocks' flags, and their ticks as told */
+    for (unsigned i = 0; i < g.x; ++i) {
+      for (int j = 0; j < ARG(9, int); ++j) {
+        uint32_t* e = ARG(10, uint32_t*) + 4 * (i * ARG(9, int) + j);
+        e[0] = 0x7fc00000u;
+        e[1] = 0x80000000u | ARG(12, unsigned);
+        e[2] = e[3] = ~0u;
+      }
+      ARG(11, unsigned*)[i] = ARG(12, unsigned);
+      uint64_t** stamps = (uint64_t**)args[13];
+      if (stamps[0] && i == 0) { stamps[0][0] = 1000; stamps[0][1] = ARG(12, unsigned); }
+      if (stamps[1]) stamps[1][i] = i < 4 ? end_tick[i] : end_tick[3];
     }
   }
   if (strstr(name, "mla_evict_kernel")) {
@@ -255,4 +278,23 @@ for nth in range(1, {buffers} + 2):
             assert hip.fake_failed() and stats["batched"] == 0, (nth, stats)
         else:
             assert not hip.fake_failed() and stats["batched"] == nq, (nth, stats)
+""")
+
+
+# Block 0 stamps the start (tick 1000 of a 100 MHz clock); a short block of
+# another XCD may have ended by then
+@pytest.mark.parametrize("ticks,us", [((1600, 1500, 1700, 1400), 7.0), ((1600, 900, 1500, 999), 6.0),
+                                      ((999, 900, 1, 999), None)])
+def test_blocks_that_end_before_the_start_stamp(runtime, ticks, us):
+    run(runtime, f"""
+with MlaNodeBank(np.ones((200, 32), np.float32)) as bank:  # 4 blocks
+    hip.fake_ticks(*(ctypes.c_uint64(t) for t in {ticks}))
+    q = np.ones((1, 32), np.float32)
+    for _ in range(2):
+        try:
+            ms = bank.route(q, 3).device_ms
+        except RuntimeError:
+            assert {us} is None
+        else:
+            assert abs(ms * 1e3 - {us}) < 1e-3
 """)
