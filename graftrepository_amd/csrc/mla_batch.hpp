@@ -745,8 +745,9 @@ __device__ inline float wave_sort_desc(float v) {
 // Steps: the last wavefront stages the query while the others load the
 // sub-streams' entries and each sort their lanes' largest kept s~; the
 // largest k-th of those, L, is a lower bound on v_k, so every kept entry at
-// or above t lies at or above L - 2B.  Those entries (at most kSurvMax,
-// else no certificate) are collected in LDS, one thread each: it ranks its
+// or above t lies at or above L - 2B.  The positive ones of those (at most
+// kSurvMax, else no certificate; fewer than k, and t is not positive) are
+// collected in LDS, one thread each: it ranks its
 // entry by (s~ desc, sub-stream asc) and counts the entries above s~ + 2B.
 // Fewer than k such entries holds for every entry at or above t (those
 // above it then lie above v_k), so the entries passing that count -- a
@@ -988,8 +989,10 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
   }
   const double floor_s = static_cast<double>(L) - 2.0 * bound - 0x1p-40;
   auto offer = [&](float u, uint32_t key) {
+    // an entry at or above t is positive; zeros (a list without a tile holds
+    // -0) would only fill the survivors' places
     const float v = u * iq;
-    if (isfinite(v) && static_cast<double>(v) >= floor_s) {
+    if (v > 0.0f && isfinite(v) && static_cast<double>(v) >= floor_s) {
       const unsigned at = atomicAdd(&s_count, 1u);
       if (at < static_cast<unsigned>(kSurvMax)) {
         s_sv[at] = v;

@@ -56,14 +56,17 @@ def test_query_counts(hip_lib, nq, k, n):
         assert bank.route_stats()["batched"] == nq
 
 
-# the ring screen's runs: none, one or several tiles each
-@pytest.mark.parametrize("n", [20, 33, 5000, 32_768, 33_001, 100_003])
-def test_ring_runs(hip_lib, n):
+# The ring screen's runs: none, one or several tiles each, with k that a lane
+# half's two entries per tile certify for nearly every query
+@pytest.mark.parametrize("n,k", [(20, 2), (33, 2), (600, 8), (1000, 12), (5000, 16), (32_768, 16), (33_001, 16),
+                                 (100_003, 16)])
+def test_ring_runs(hip_lib, n, k):
     rows = wl.mla_rows(n, 72, seed=n, dtype="bf16")
     qs = wl.mla_queries(200, 72, seed=n + 1, dtype="bf16")
     with MlaNodeBank(rows, dtype="bf16") as bank:
-        check(bank, rows, qs, 16, query_dtype="bf16")
-        assert bank.route_stats()["batched"] == 200
+        check(bank, rows, qs, k, query_dtype="bf16")
+        stats = bank.route_stats()
+        assert stats["batched"] == 200 and stats["fallbacks"] <= 20
 
 
 def test_churn_warmup_and_bf16_queries(hip_lib):
