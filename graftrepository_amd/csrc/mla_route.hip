@@ -37,7 +37,7 @@
 
 #include <algorithm>
 #include <atomic>
-#include <limits>
+#include <cmath>
 #include <mutex>
 #include <vector>
 
@@ -874,19 +874,54 @@ size_t stream_lds(const MlaDeviceArena* a, const BatchPlan& p, int qp) {
   return static_cast<size_t>(qp) * (16 * p.nb * p.p + 8) * (a->dtype == kF32 ? 4 : 2);
 }
 
-// Timed queries per call from which the batched path runs: three, or two on
-// banks of 8,192 slots and more.  A batched call costs 24 to 42 us on small
-// banks (64 to 576 values) whatever its queries, the single-query kernel
-// about 10 us a query after the first: two queries took 21 against 25 us at
-// 1,000 x 64 and 31 against 31 at 5,000 x 288, but 38 against 33 at 20,000 x
-// 288 and 97 against 74 at 100,000 x 576; three never less than the batched
-// call.
-int batch_threshold(const MlaDeviceArena* a) {
-  return a->batch_min > 0 ? a->batch_min : (a->high_water >= 8192 ? 2 : 3);
+// Whether a segment of `queries` has a pass for the ring screen.
+bool has_ring_pass(const BatchPlan& p, int queries) {
+  return std::min(queries, p.qp_max) > grm::mla::kStreamMaxCols;
 }
 
-bool batch_plan(const MlaDeviceArena* a, int q_timed, BatchPlan* p) {
-  if (q_timed < batch_threshold(a)) return false;
+// Whether a batched call of q queries for the k best is worth it.
+//
+// A batched call costs 24 to 42 us on small banks (64 to 576 values)
+// whatever its queries; a call of the single-query kernel costs about 10 us
+// a query (8 to 13, by row length and k) and 10 us more.  So the batched
+// call saves nothing up to two queries on small banks, and up to one and a
+// half on banks of 8,192 slots and more: three queries took 31 against 41 us
+// at 5,000 x 288 (k = 1) and two 31 against 31, but two took 33 against 38
+// us at 20,000 x 288 and 74 against 97 at 100,000 x 576.
+//
+// Queries without a certificate are routed again on the single-query
+// kernel, as many as they are and 12 us for the second round.  A list of the
+// screen keeps two entries, so a query has no certificate when three of its
+// k best fall into one list's slots; with them spread evenly over S lists,
+// each holds three or more with probability p = P(Bin(k, 1/S) >= 3), and
+// none does with (1 - p)^S.  Measured at 288 values, batched against single
+// us: 300 slots, k = 8 (a third without certificate) 3 queries 47/41, 8
+// queries 63/93; k = 16 (all) 64 queries 810/779; 600 slots, k = 16 (0.65)
+// 8 queries 101/107, 3 queries 68/47; 1,000 slots, k = 16 (0.33) 3 queries
+// 52/47, 8 queries 74/109; 2,000 slots, k = 16 (0.1) 3 queries 40/49.  Above
+// 0.85 the most a call could save is less than its screen costs.
+bool batch_pays(const MlaDeviceArena* a, const BatchPlan& p, int q, int k) {
+  if (a->batch_min > 0) return q >= a->batch_min;
+  // lists: a sub-stream's, or on the ring a lane half's of each run
+  const bool ring = has_ring_pass(p, q);
+  const double tiles = static_cast<double>(a->high_water) / 32.0;
+  const double runs = ring ? static_cast<double>(a->cus) * grm::mla::kRingSegs : static_cast<double>(p.subs);
+  const double lists = (ring ? 2.0 : 1.0) * std::min(tiles, runs);
+  if (2.0 * std::ceil(lists) < k) return false;  // fewer entries than results: never a certificate
+  const double x = std::min(1.0, 1.0 / lists);
+  double two = 1.0;  // P(Bin(k, x) <= 2)
+  if (k >= 3) {
+    const double rest = std::pow(1.0 - x, k - 2);
+    two = rest * ((1.0 - x) * (1.0 - x) + k * x * (1.0 - x) + 0.5 * k * (k - 1) * x * x);
+  }
+  const double certain = std::pow(two, lists);  // of a query
+  if (certain < 0.15) return false;
+  const double none = std::pow(certain, q);     // of all of them
+  return q * certain > (a->high_water >= 8192 ? 1.5 : 2.0) + 1.2 * (1.0 - none);
+}
+
+// False where the screens do not take the bank.
+bool batch_plan(const MlaDeviceArena* a, BatchPlan* p) {
   const uint32_t per_step = a->dtype == kF32 ? 4 : 2;  // chunks
   p->ks = static_cast<int>((a->chunks + per_step - 1) / per_step);
   // the steps in flight that pad the row least, the most of those
@@ -1087,11 +1122,6 @@ int enqueue_batch_pass(MlaDeviceArena* a, const BatchPlan& p, const PassQueries&
   return 0;
 }
 
-// Whether a segment of `queries` has a pass for the ring screen.
-bool has_ring_pass(const BatchPlan& p, int queries) {
-  return std::min(queries, p.qp_max) > grm::mla::kStreamMaxCols;
-}
-
 // Buffers of the batched route, with those of the ring screen where it has
 // a pass.  False when the device has no room for them: the queries then go
 // one by one.
@@ -1145,8 +1175,10 @@ int route_impl(MlaDeviceArena* a, const void* queries, int q_dtype,
   if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->mut[a->mut_last].ev, 0));
   const size_t qstride = static_cast<size_t>(a->dim) * elem_size(q_dtype);
   BatchPlan bp;
-  const bool batched = !a->no_batch && batch_plan(a, q_count - warmup, &bp) &&
-                       reserve_batch(a, bp, has_ring_pass(bp, std::max(warmup, q_count - warmup)));
+  const int timed = q_count - warmup;
+  const bool batched = !a->no_batch && (timed > 1 || a->batch_min == 1) && batch_plan(a, &bp) &&
+                       batch_pays(a, bp, timed, topk) &&
+                       reserve_batch(a, bp, has_ring_pass(bp, std::max(warmup, timed)));
   a->screen_ms = 0.0f;
   std::vector<int> redo;  // queries for the single-query kernel
   if (batched) {
@@ -1157,7 +1189,7 @@ int route_impl(MlaDeviceArena* a, const void* queries, int q_dtype,
     const size_t n_q = static_cast<size_t>(q_count);
     const bool flags = n_q <= kMaxDoneFlags && !grm::blocking_sync() && a->ticks_per_ms > 0.0 &&
                        !(elapsed_ms && grm::event_timing());
-    const int timed_passes = (q_count - warmup + bp.qp_max - 1) / bp.qp_max;
+    const int timed_passes = (timed + bp.qp_max - 1) / bp.qp_max;
     unsigned* d_done = nullptr;
     if (flags) {
       GRM_CHECK_RC(grm::begin_flags(&a->done_flags, kMaxDoneFlags, &a->route_seq));
@@ -2151,7 +2183,7 @@ extern "C" int grm_mla_hip_probe_screen(MlaDeviceArena* a, const void* queries_h
   }
   if (query_dtype != kF32 && query_dtype != kBF16) return grm::fail(-1, "query dtype must be F32 or BF16");
   BatchPlan p;
-  if (!batch_plan(a, std::numeric_limits<int>::max(), &p)) {
+  if (!batch_plan(a, &p)) {
     return grm::fail(-1, "bank has no batched screen (rows too long or too many)");
   }
   if (query_count <= 0 || query_count > p.qp_max) return grm::fail(-1, "query_count out of range");

@@ -45,15 +45,19 @@ def test_row_lengths(hip_lib, dim, dtype):
         assert stats["fallbacks"] <= 2
 
 
-# column tiles and passes; one tile up to several tiles per sub-stream
+# Column tiles and passes; one tile up to several tiles per sub-stream.  The
+# results compared are to come from the screen and the merge: a tile keeps
+# two entries per query, so one or two tiles certify up to two results; at
+# 2,000 rows and k = 16 a tenth of the queries have three in one tile.
 @pytest.mark.parametrize("nq,k", [(4, 1), (32, 3), (33, 16), (64, 8), (65, 5), (128, 2), (130, 7)])
 @pytest.mark.parametrize("n", [20, 32, 33, 2000, 70_001])
 def test_query_counts(hip_lib, nq, k, n):
     rows = wl.mla_rows(n, 96, seed=n)
     qs = wl.mla_queries(nq, 96, seed=n + 1)
     with MlaNodeBank(rows) as bank:
-        check(bank, rows, qs, k)
-        assert bank.route_stats()["batched"] == nq
+        check(bank, rows, qs, k if n >= 2000 else min(k, 2))
+        stats = bank.route_stats()
+        assert stats["batched"] == nq and stats["fallbacks"] <= nq // 4
 
 
 # The ring screen's runs: none, one or several tiles each, with k that a lane
@@ -67,6 +71,20 @@ def test_ring_runs(hip_lib, n, k):
         check(bank, rows, qs, k, query_dtype="bf16")
         stats = bank.route_stats()
         assert stats["batched"] == 200 and stats["fallbacks"] <= 20
+
+
+# Calls that the screen would send back to the single-query kernel take that
+# at once: too few entries for k, or most queries with three in one tile
+@pytest.mark.parametrize("n,k,nq,batched", [
+    (20, 3, 64, False), (300, 16, 64, False), (1000, 16, 3, False), (1000, 16, 8, True),
+    (2000, 16, 3, True), (1000, 3, 2, False), (1000, 3, 3, True), (9000, 3, 2, True)])
+def test_which_calls_are_batched(hip_lib, n, k, nq, batched):
+    rows, qs = wl.mla_rows(n, 96, seed=n), wl.mla_queries(nq, 96, seed=n + 1)
+    with MlaNodeBank(rows) as bank:
+        check(bank, rows, qs, k)
+        stats = bank.route_stats()
+    assert stats["batched"] == (nq if batched else 0)
+    assert stats["single"] == (stats["fallbacks"] if batched else nq)
 
 
 def test_churn_warmup_and_bf16_queries(hip_lib):
