@@ -145,8 +145,10 @@ int wait_tagged(const Cand* entries, size_t n, unsigned seq, hipEvent_t ev) {
 
 constexpr size_t kStampHead = 2;  // start tick, route number
 
+size_t stamps_bytes(size_t max) { return (kStampHead + max) * sizeof(unsigned long long); }
+
 int reserve_stamps(MappedBuf* buf, size_t max) {
-  const size_t bytes = (kStampHead + max) * sizeof(unsigned long long);
+  const size_t bytes = stamps_bytes(max);
   if (buf->bytes < bytes) {
     GRM_CHECK_RC(reserve_mapped_bytes(buf, bytes));
     memset(buf->host, 0, bytes);

@@ -354,11 +354,12 @@ int wait_flags(const MappedBuf& buf, unsigned seq, size_t n, hipEvent_t ev);
 int wait_tagged(const Cand* entries, size_t n, unsigned seq, hipEvent_t ev);
 
 // Device-clock timing of a flagged route (RouteStamps).  reserve_stamps
-// puts a buffer in place for `max` flags: two start words, then one end
-// tick per flag; route_stamps gives the device pointers, with the end
-// ticks from flag `first` on.  stamps_elapsed, once wait_flags has seen
-// flags [0, n) hold seq, gives the route's device time in ms: the latest
-// end tick of the timed flags [first, n) less the start tick, at
+// puts a buffer in place for `max` flags (stamps_bytes, zeroed): two start
+// words, then one end tick per flag; route_stamps gives the device
+// pointers, with the end ticks from flag `first` on.  stamps_elapsed, once
+// wait_flags has seen flags [0, n) hold seq, gives the route's device time
+// in ms: the latest end tick of the timed flags [first, n) less the start
+// tick, at
 // `ticks_per_ms`.  As with list entries, the host may see a flag before
 // the stores ahead of it: a start stamp of another route, or a timed end
 // tick below the start tick (an earlier route's, or of a block that ended
@@ -367,6 +368,7 @@ int wait_tagged(const Cand* entries, size_t n, unsigned seq, hipEvent_t ev);
 // after it.
 // wall_ticks_per_ms: the constant clock's rate on `device` (0 when the
 // device does not report it; such routes keep stream events).
+size_t stamps_bytes(size_t max);
 int reserve_stamps(MappedBuf* buf, size_t max);
 RouteStamps route_stamps(const MappedBuf& buf, size_t first);
 int stamps_elapsed(const MappedBuf& buf, unsigned seq, size_t first, size_t n, hipEvent_t ev,

@@ -466,13 +466,16 @@ struct MlaDeviceArena {
   const float* route_norms = nullptr;  // set around a filtered route: norms it reads
   bool no_batch = false;               // set around a filtered route: single-query path only
   grm::MappedCands blocks_out;  // per-query, per-block top-k (host mapped)
-  // per-(query, block) completion flags (host mapped) and the number the
-  // last flag-waiting route stored there
-  grm::MappedBuf done_flags;
-  unsigned route_seq = 0;
-  // device-clock stamps of timed single-query routes on the flag path
-  // (host mapped), and the clock's ticks per ms (0: stream events)
+  // What flag-waiting routes report (host mapped, one allocation, see
+  // reserve_marks): a completion flag per (query, block), the number the
+  // last such route stored there, device-clock stamps, and the clock at the
+  // start of each batched pass's screen and merge.  ticks_per_ms: the
+  // clock's rate (0: stream events).
+  grm::MappedBuf marks;
+  grm::MappedBuf done_flags;    // these three lie in marks
   grm::MappedBuf stamps;
+  grm::MappedBuf screen_ticks;
+  unsigned route_seq = 0;
   double ticks_per_ms = 0.0;
   std::vector<Cand> merged;
   void* h_stage = nullptr;
@@ -498,7 +501,6 @@ struct MlaDeviceArena {
   uint32_t* d_entries = nullptr;   // screen result planes
   size_t d_entries_count = 0;
   grm::MappedCands batch_out;
-  grm::MappedBuf screen_ticks;  // device clock at the start of each pass's screen and merge
   // host queries staged for fetch_async (GRM_HIP_QUERY_COPY=dma: the copy
   // engine instead)
   grm::MappedBuf q_map;
@@ -546,11 +548,9 @@ void destroy_arena(MlaDeviceArena* a) {
   if (a->d_entries) (void)hipFree(a->d_entries);
   if (a->d_winv) (void)hipFree(a->d_winv);
   grm::release_mapped(&a->batch_out);
-  grm::release_mapped_bytes(&a->screen_ticks);
+  grm::release_mapped_bytes(&a->marks);
   grm::release_mapped_bytes(&a->q_map);
   grm::release_mapped(&a->blocks_out);
-  grm::release_mapped_bytes(&a->done_flags);
-  grm::release_mapped_bytes(&a->stamps);
   if (a->h_stage) (void)hipHostFree(a->h_stage);
   if (a->ev_start) (void)hipEventDestroy(a->ev_start);
   if (a->ev_stop) (void)hipEventDestroy(a->ev_stop);
@@ -1140,6 +1140,28 @@ bool reserve_batch(MlaDeviceArena* a, const BatchPlan& p, bool ring) {
 
 // Completion flags a route may wait on (one per query and route block).
 constexpr size_t kMaxDoneFlags = 8192;
+// Batched passes of a route that waits on flags, the shortest being 32
+// queries, and of its warm-up.
+constexpr size_t kMaxTickPasses = kMaxDoneFlags / 32 + 1;
+
+// Flags, stamps and ticks in one pinned allocation: one costs 20 to 30 us,
+// and the first routes on a bank pay for each.
+int reserve_marks(MlaDeviceArena* a) {
+  if (a->marks.host) return 0;
+  const size_t flags = kMaxDoneFlags * sizeof(unsigned);
+  const size_t stamps = grm::stamps_bytes(kMaxDoneFlags);
+  const size_t ticks = kMaxTickPasses * 2 * sizeof(unsigned long long);
+  GRM_CHECK_RC(grm::reserve_mapped_bytes(&a->marks, flags + stamps + ticks));
+  memset(a->marks.host, 0, a->marks.bytes);
+  auto part = [&](size_t at, size_t bytes) {
+    return grm::MappedBuf{static_cast<unsigned char*>(a->marks.host) + at,
+                          static_cast<unsigned char*>(a->marks.dev) + at, bytes};
+  };
+  a->done_flags = part(0, flags);
+  a->stamps = part(flags, stamps);
+  a->screen_ticks = part(flags + stamps, ticks);
+  return 0;
+}
 
 int route_impl(MlaDeviceArena* a, const void* queries, int q_dtype,
                bool on_device, int q_count, int dim, int warmup, int topk,
@@ -1192,13 +1214,8 @@ int route_impl(MlaDeviceArena* a, const void* queries, int q_dtype,
     const int timed_passes = (timed + bp.qp_max - 1) / bp.qp_max;
     unsigned* d_done = nullptr;
     if (flags) {
+      GRM_CHECK_RC(reserve_marks(a));
       GRM_CHECK_RC(grm::begin_flags(&a->done_flags, kMaxDoneFlags, &a->route_seq));
-      GRM_CHECK_RC(grm::reserve_stamps(&a->stamps, kMaxDoneFlags));
-      if (a->screen_ticks.bytes < 16 * static_cast<size_t>(timed_passes)) {
-        const size_t bytes = 16 * static_cast<size_t>(timed_passes);
-        GRM_CHECK_RC(grm::reserve_mapped_bytes(&a->screen_ticks, bytes));
-        memset(a->screen_ticks.host, 0, bytes);
-      }
       d_done = static_cast<unsigned*>(a->done_flags.dev);
     } else {
       while (a->screen_ev.size() < 2 * static_cast<size_t>(timed_passes)) {
@@ -1295,10 +1312,10 @@ int route_impl(MlaDeviceArena* a, const void* queries, int q_dtype,
     const bool flags = flaggable && (!elapsed_ms || clocked);
     unsigned* d_done = nullptr;
     if (flags) {
+      GRM_CHECK_RC(reserve_marks(a));
       GRM_CHECK_RC(grm::begin_flags(&a->done_flags, kMaxDoneFlags, &a->route_seq));
       d_done = static_cast<unsigned*>(a->done_flags.dev);
     }
-    if (clocked) GRM_CHECK_RC(grm::reserve_stamps(&a->stamps, kMaxDoneFlags));
     // Uncertified batched queries add their time to the timed segment.
     bool started = false;
     for (size_t j = 0; j < redo.size(); ++j) {

@@ -31,6 +31,8 @@ static int fails(const char* name) {
 }
 #define CALL(name) if (fails(#name)) return 2
 static size_t pinned, device;
+static int pins;
+int fake_pins(void) { return pins; }
 size_t fake_pinned(void) { return pinned; }
 size_t fake_device(void) { return device; }
 static void* take(size_t n, size_t* sum) {
@@ -44,7 +46,7 @@ static int give(void* q, size_t* sum) {
   return 0;
 }
 int hipMalloc(void** p, size_t n) { CALL(hipMalloc); *p = take(n, &device); return 0; }
-int hipHostMalloc(void** p, size_t n, unsigned f) { CALL(hipHostMalloc); *p = take(n, &pinned); return 0; }
+int hipHostMalloc(void** p, size_t n, unsigned f) { CALL(hipHostMalloc); ++pins; *p = take(n, &pinned); return 0; }
 int hipFree(void* p) { return give(p, &device); }
 int hipHostFree(void* p) { return give(p, &pinned); }
 int hipHostGetDevicePointer(void** d, void* h, unsigned f) { *d = h; return 0; }
@@ -297,4 +299,20 @@ with MlaNodeBank(np.ones((200, 32), np.float32)) as bank:  # 4 blocks
             assert {us} is None
         else:
             assert abs(ms * 1e3 - {us}) < 1e-3
+""")
+
+
+# Pinned allocations are most of a first call's cost on a new bank: the
+# query's, the results' and one for flags, stamps and ticks
+@pytest.mark.parametrize("nq,timed", [(1, False), (1, True), (8, False), (8, True)])
+def test_pinned_allocations_of_a_first_route(runtime, nq, timed):
+    run(runtime, f"""
+with MlaNodeBank(np.ones((20_000, 64), np.float32)) as bank:
+    hip.fake_ticks(*(ctypes.c_uint64(2000),) * 4)
+    before = hip.fake_pins()
+    try:
+        bank.route(np.ones(({nq}, 64), np.float32), 3, timed={timed})
+    except RuntimeError as e:  # the merge kernel does not run here
+        assert {nq} > 1 and "completion flags" in str(e)
+    assert hip.fake_pins() - before == 3
 """)
