@@ -48,11 +48,12 @@ def sources() -> list[Path]:
     return sorted(CSRC.glob("*.hip"))
 
 
-# Per-source flags.  mla_route.hip: MFMA accumulators in VGPRs (the ring
+# Per-source flags.  The MLA screens: MFMA accumulators in VGPRs (the ring
 # screen keeps its query fragments in AGPRs and reduces the accumulators
 # with VALU instructions, which then need no AGPR-to-VGPR copies).
 SOURCE_FLAGS = {
     "mla_route.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "mla_screen_probe.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 
 

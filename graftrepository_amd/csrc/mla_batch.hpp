@@ -1,5 +1,4 @@
-// mla_batch.hpp -- batched MLA route on the matrix cores (included by
-// mla_route.hip only).
+// mla_batch.hpp -- batched MLA route on the matrix cores: its kernels.
 //
 // Q queries against a bank, law as the single-query route
 // (cpp/grm_runtime.cpp:3518-3545):
@@ -38,6 +37,7 @@
 #pragma once
 
 #include "grm_common.hpp"
+#include "mla_values.hpp"
 
 namespace grm {
 namespace mla {
@@ -421,7 +421,7 @@ __device__ __forceinline__ void wait_vmcnt_lds() {
 // The slot weights the screens multiply by: 1/norm_f (v_rcp_f32), 0 for
 // an all-zero row, -0 for a slot that never ranks (NaN norm: tombstone,
 // unused slot, non-finite row) and for a norm that overflowed.
-__global__ void mla_batch_weights_kernel(const float* __restrict__ norms, uint64_t n,
+static __global__ void mla_batch_weights_kernel(const float* __restrict__ norms, uint64_t n,
                                          float* __restrict__ winv) {
   const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -673,7 +673,7 @@ static_assert(kRingSegs == 4, "a lane's lists of one kind are one 16-byte store"
 // values rounded to bf16 (nearest even; bf16 queries are copied), zero past
 // dim; inv_qn[j] = 1 / ||q_j|| rounded to fp32.  Rows j >= qc are zero with
 // inv_qn NaN (nothing is kept for them).  grid = QP blocks.
-__global__ __launch_bounds__(kWave) void mla_batch_qprep_kernel(
+static __global__ __launch_bounds__(kWave) void mla_batch_qprep_kernel(
     const void* __restrict__ query, int q_dtype, int qc, uint32_t dim, int stride,
     uint16_t* __restrict__ qpad, float* __restrict__ inv_qn, RouteStamps stamps, unsigned seq) {
   route_start_stamp(stamps, seq);
@@ -1125,7 +1125,7 @@ __global__ __launch_bounds__(kMergeThreads) void mla_batch_merge_kernel(
 // out_values[qi*n + slot], and the query's bound B, out_bounds[qi] (+inf
 // where it is not established, screen_in_range).  grid = queries
 // of the pass, one wavefront each.
-__global__ __launch_bounds__(kWave) void mla_batch_probe_finish_kernel(
+static __global__ __launch_bounds__(kWave) void mla_batch_probe_finish_kernel(
     const uint32_t* __restrict__ planes, uint64_t cap, uint32_t n, const float* __restrict__ inv_qn,
     const void* __restrict__ query, int q_dtype, size_t qstride, uint32_t len, ScreenBound sb,
     const unsigned* __restrict__ norm_range, float* __restrict__ out_values,

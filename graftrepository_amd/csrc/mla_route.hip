@@ -29,6 +29,8 @@
 // bound on the screen's rounding error and rescores the shortlist with the
 // exact law; queries without a certificate are routed again here.
 #include "grm_common.hpp"
+#include "mla_screen.hpp"
+#include "mla_values.hpp"
 #include "slot_tables.hpp"
 #include "grm_hip_router.h"
 
@@ -43,8 +45,6 @@
 
 namespace grm {
 namespace mla {
-
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kMaxDim = 4096;
 constexpr int kRouteWaves = 16;          // most waves per block of the single-query kernel
@@ -107,52 +107,6 @@ __device__ inline void stage_query(double* qd, const void* __restrict__ query,
   } else {
     stage_values(qd, static_cast<const float*>(query), dim, dim_pad);
   }
-}
-
-// q[0, N) in order through `use(value, index)`, read from LDS kAhead values
-// ahead of their use: a lone wave on its SIMD would otherwise wait for LDS
-// (over 100 cycles) at every chunk of its serial fp64 chain.
-template <int N, int kAhead, typename F>
-__device__ __forceinline__ void stream_lds(const double* __restrict__ q, F use) {
-  static_assert(N % kAhead == 0, "whole stages");
-  double cur[kAhead], nxt[kAhead];
-#pragma unroll
-  for (int e = 0; e < kAhead; ++e) cur[e] = q[e];
-#pragma unroll
-  for (int s = 0; s < N / kAhead; ++s) {
-    if (s + 1 < N / kAhead) {
-#pragma unroll
-      for (int e = 0; e < kAhead; ++e) nxt[e] = q[(s + 1) * kAhead + e];
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int e = 0; e < kAhead; ++e) use(cur[e], s * kAhead + e);
-#pragma unroll
-    for (int e = 0; e < kAhead; ++e) cur[e] = nxt[e];
-  }
-}
-
-// Value i of a chunk (fp32 or bf16) as a double.
-template <int DT>
-__device__ __forceinline__ double chunk_value(u32x4 v, int i) {
-  const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
-  if constexpr (DT == kF32) {
-    return static_cast<double>(__uint_as_float(w4[i]));
-  } else {
-    const uint32_t w = w4[i >> 1];
-    return static_cast<double>(__uint_as_float((i & 1) ? (w & 0xffff0000u) : (w << 16)));
-  }
-}
-
-// The law's query norm from the staged query (zeros past dim add nothing):
-// one serial fp64 chain over d (cpp/grm_runtime.cpp:4310-4314).  n is a
-// multiple of 4.
-__device__ inline double staged_norm(const double* __restrict__ qd, uint32_t n) {
-  double acc = 0.0;
-  uint32_t d = 0;
-  for (; d + 64 <= n; d += 64) stream_lds<64, 16>(qd + d, [&](double q, int) { acc = fma(q, q, acc); });
-  for (; d < n; d += 4) stream_lds<4, 4>(qd + d, [&](double q, int) { acc = fma(q, q, acc); });
-  return sqrt(acc);
 }
 
 // One query against every slot; each block writes its k best entries to
@@ -421,13 +375,16 @@ __global__ void mla_evict_kernel(const uint64_t* __restrict__ slots,
 }  // namespace mla
 }  // namespace grm
 
-#include "mla_batch.hpp"
-
 using grm::Cand;
 using grm::kBF16;
 using grm::kF16;
 using grm::kF32;
 using grm::kNoId;
+using grm::mla::BatchPlan;
+using grm::mla::PassMarks;
+using grm::mla::PassQueries;
+using grm::mla::PassShape;
+using grm::mla::ScreenLaunch;
 using grm::mla::u32x4;
 
 // ------------------------------------------------------------------ host side
@@ -849,30 +806,10 @@ void write_cands(const Cand* c, int topk, uint64_t* out_ids, float* out_scores) 
   }
 }
 
-// Batched-route plan.
-struct BatchPlan {
-  int ks = 0;          // K-steps of 16 dims that cover a row
-  int p = 0;           // K-steps in flight per wavefront of the stream screen
-  int nb = 0;          // batches of p steps: nb * p >= ks
-  int qp_max = 0;      // queries per pass (32, 64, 128, or 256 on the ring)
-  int qp_stream = 0;   // queries per stream-screen pass
-  uint32_t subs = 0;   // sub-streams of a stream-screen pass
-  int ibits = 0;       // width of the slot code the stream screen writes into its values
-  bool ring = false;   // full passes of a bf16 bank run mla_batch_ring_kernel
-  int ks_ring = 0;     // its K-steps (8, 16 or 18)
-  int ibits_ring = 0;  // its slot code width
-};
-
 // Slot code width of the batched screens.  The code costs the screen bound 2^(ibits-23) relative, so banks
 // whose runs would need more than 16 bits route on the single-query path
 // instead.
 constexpr int kMaxSlotCodeBits = 16;
-
-// LDS of a stream-screen pass of qp queries (of an fp32 bank their bf16
-// parts and remainders).
-size_t stream_lds(const MlaDeviceArena* a, const BatchPlan& p, int qp) {
-  return static_cast<size_t>(qp) * (16 * p.nb * p.p + 8) * (a->dtype == kF32 ? 4 : 2);
-}
 
 // Whether a segment of `queries` has a pass for the ring screen.
 bool has_ring_pass(const BatchPlan& p, int queries) {
@@ -936,7 +873,7 @@ bool batch_plan(const MlaDeviceArena* a, BatchPlan* p) {
   }
   p->nb = best / p->p;
   int qp = grm::mla::kStreamMaxCols;
-  while (qp >= 32 && stream_lds(a, *p, qp) > a->lds_max) qp /= 2;
+  while (qp >= 32 && grm::mla::stream_screen_lds(a->dtype, *p, qp) > a->lds_max) qp /= 2;
   if (qp < 32) return false;
   p->qp_stream = qp;
   // the merge holds kMergePer sub-streams (screen wavefronts) per thread
@@ -964,12 +901,6 @@ bool batch_plan(const MlaDeviceArena* a, BatchPlan* p) {
 
 // One pass of qc queries: on the ring screen when the plan has it and the
 // pass holds more than 128 queries (padded to 256).
-struct PassShape {
-  bool ring;
-  int qp;          // columns
-  uint32_t subs;   // sub-streams
-  int ibits;
-};
 PassShape pass_shape(const MlaDeviceArena* a, const BatchPlan& p, int qc) {
   if (qc > grm::mla::kStreamMaxCols) {
     return {true, grm::mla::kRingQueries, a->cus * 2 * grm::mla::kRingSegs, p.ibits_ring};
@@ -990,98 +921,13 @@ int ensure_weights(MlaDeviceArena* a) {
   return 0;
 }
 
-template <int KS, bool kProbe = false>
-int launch_ring(MlaDeviceArena* a, uint32_t n_tiles32, int ibits, uint32_t* planes,
-                unsigned long long* tick) {
-  using RS = grm::mla::RingShape<KS>;
-  auto kern = grm::mla::mla_batch_ring_kernel<KS, kProbe>;
-  GRM_CHECK_RC(ensure_weights(a));
-  GRM_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    static_cast<int>(RS::kLds)));
-  kern<<<a->cus, grm::mla::kRingWaves * grm::kWave, RS::kLds, a->stream>>>(
-      a->d_tiles, a->d_winv, a->capacity, n_tiles32, a->d_qpad, ibits, planes, tick);
-  GRM_HIP_CHECK(hipGetLastError());
-  return 0;
-}
-
-// A pass's queries (device) and what its kernels report on the way.
-struct PassQueries {
-  const void* q;
-  int dtype;
-  int count;
-};
-struct PassMarks {
-  grm::RouteStamps start{nullptr, nullptr};    // the route's first timed kernel
-  unsigned long long* screen_tick = nullptr;   // [screen start, merge start]
-  hipEvent_t* ev = nullptr;                    // events around the screen kernel
-};
-
-template <int DT, int P, int CT, bool kProbe>
-int launch_stream(MlaDeviceArena* a, const BatchPlan& p, const PassQueries& q, uint32_t* planes,
-                  const PassMarks& m) {
-  auto kern = grm::mla::mla_batch_stream_kernel<DT, P, CT, kProbe>;
-  const size_t lds = stream_lds(a, p, 32 * CT);
-  if (lds > 65536) {
-    GRM_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      static_cast<int>(lds)));
-  }
-  const uint32_t n_tiles32 = static_cast<uint32_t>((a->high_water + 31) / 32);
-  kern<<<a->cus, grm::mla::kBatchWaves * grm::kWave, lds, a->stream>>>(
-      a->d_tiles, a->d_norms, a->capacity, a->chunks, n_tiles32, p.subs,
-      static_cast<uint32_t>(p.nb), static_cast<uint32_t>(p.ks), q.q, q.dtype, q.count, a->dim,
-      a->d_inv_qn, p.ibits, planes, m.start, a->route_seq, m.screen_tick);
-  GRM_HIP_CHECK(hipGetLastError());
-  return 0;
-}
-
-template <int DT, int P, bool kProbe>
-int launch_stream_ct(MlaDeviceArena* a, const BatchPlan& p, int qp, const PassQueries& q,
-                     uint32_t* planes, const PassMarks& m) {
-  if (qp == 32) return launch_stream<DT, P, 1, kProbe>(a, p, q, planes, m);
-  if (qp == 64) return launch_stream<DT, P, 2, kProbe>(a, p, q, planes, m);
-  return launch_stream<DT, P, 4, kProbe>(a, p, q, planes, m);
-}
-
-// The screen of one pass, its queries prepared first where the screen does
-// not do so itself.
-template <bool kProbe>
-int launch_screen(MlaDeviceArena* a, const BatchPlan& p, const PassShape& s, const PassQueries& q,
-                  uint32_t* planes, const PassMarks& m) {
-  if (s.ring) {
-    grm::mla::mla_batch_qprep_kernel<<<s.qp, grm::kWave, 0, a->stream>>>(
-        q.q, q.dtype, q.count, a->dim, 16 * p.ks_ring + 8, a->d_qpad, a->d_inv_qn, m.start,
-        a->route_seq);
-    GRM_HIP_CHECK(hipGetLastError());
-  }
-  if (m.ev) GRM_HIP_CHECK(hipEventRecord(m.ev[0], a->stream));
-  int rc = 0;
-  if (s.ring) {
-    const uint32_t n_tiles32 = static_cast<uint32_t>((a->high_water + 31) / 32);
-    switch (p.ks_ring) {
-      case 8: rc = launch_ring<8, kProbe>(a, n_tiles32, s.ibits, planes, m.screen_tick); break;
-      case 16: rc = launch_ring<16, kProbe>(a, n_tiles32, s.ibits, planes, m.screen_tick); break;
-      default: rc = launch_ring<18, kProbe>(a, n_tiles32, s.ibits, planes, m.screen_tick); break;
-    }
-  } else if (a->dtype == kF32) {
-    switch (p.p) {
-      case 9: rc = launch_stream_ct<kF32, 9, kProbe>(a, p, s.qp, q, planes, m); break;
-      case 8: rc = launch_stream_ct<kF32, 8, kProbe>(a, p, s.qp, q, planes, m); break;
-      case 6: rc = launch_stream_ct<kF32, 6, kProbe>(a, p, s.qp, q, planes, m); break;
-      default: rc = launch_stream_ct<kF32, 4, kProbe>(a, p, s.qp, q, planes, m); break;
-    }
-  } else {
-    switch (p.p) {
-      case 18: rc = launch_stream_ct<kBF16, 18, kProbe>(a, p, s.qp, q, planes, m); break;
-      case 16: rc = launch_stream_ct<kBF16, 16, kProbe>(a, p, s.qp, q, planes, m); break;
-      case 12: rc = launch_stream_ct<kBF16, 12, kProbe>(a, p, s.qp, q, planes, m); break;
-      case 8: rc = launch_stream_ct<kBF16, 8, kProbe>(a, p, s.qp, q, planes, m); break;
-      default: rc = launch_stream_ct<kBF16, 4, kProbe>(a, p, s.qp, q, planes, m); break;
-    }
-  }
-  GRM_CHECK_RC(rc);
-  if (m.ev) GRM_HIP_CHECK(hipEventRecord(m.ev[1], a->stream));
+// The launch of pass s's screen; its result planes at `planes`.
+int screen_launch(MlaDeviceArena* a, const BatchPlan& p, const PassShape& s, const PassQueries& q,
+                  uint32_t* planes, const PassMarks& m, ScreenLaunch* out) {
+  if (s.ring) GRM_CHECK_RC(ensure_weights(a));
+  *out = ScreenLaunch{a->dtype, a->cus, a->stream, a->d_tiles, a->d_norms, a->d_winv, a->capacity,
+                      a->chunks, static_cast<uint32_t>((a->high_water + 31) / 32), a->dim, a->d_qpad,
+                      a->d_inv_qn, p, s, q, planes, m, a->route_seq};
   return 0;
 }
 
@@ -1105,7 +951,9 @@ grm::mla::ScreenBound screen_bound(const MlaDeviceArena* a, const BatchPlan& p, 
 int enqueue_batch_pass(MlaDeviceArena* a, const BatchPlan& p, const PassQueries& q, int topk,
                        Cand* out, unsigned* done, unsigned long long* end_tick, const PassMarks& m) {
   const PassShape s = pass_shape(a, p, q.count);
-  GRM_CHECK_RC(launch_screen<false>(a, p, s, q, a->d_entries, m));
+  ScreenLaunch l;
+  GRM_CHECK_RC(screen_launch(a, p, s, q, a->d_entries, m, &l));
+  GRM_CHECK_RC(grm::mla::launch_screen<false>(l));
   const uint32_t n_tiles32 = static_cast<uint32_t>((a->high_water + 31) / 32);
   auto kern = a->dtype == kF32 ? grm::mla::mla_batch_merge_kernel<kF32>
                                : grm::mla::mla_batch_merge_kernel<kBF16>;
@@ -2227,7 +2075,9 @@ extern "C" int grm_mla_hip_probe_screen(MlaDeviceArena* a, const void* queries_h
   if (a->mut_pending) GRM_HIP_CHECK(hipStreamWaitEvent(a->stream, a->mut[a->mut_last].ev, 0));
   GRM_HIP_CHECK(hipMemcpyAsync(d_q.p, queries_host, qbytes, hipMemcpyHostToDevice, a->stream));
   const PassQueries pq{d_q.p, query_dtype, query_count};
-  GRM_CHECK_RC(launch_screen<true>(a, p, shape, pq, static_cast<uint32_t*>(d_planes.p), PassMarks{}));
+  ScreenLaunch l;
+  GRM_CHECK_RC(screen_launch(a, p, shape, pq, static_cast<uint32_t*>(d_planes.p), PassMarks{}, &l));
+  GRM_CHECK_RC(grm::mla::launch_probe_screen(l));
   const uint32_t len = grm::mla::merge_len(a->dim);
   grm::mla::mla_batch_probe_finish_kernel<<<query_count, grm::kWave, len * sizeof(double), a->stream>>>(
       static_cast<const uint32_t*>(d_planes.p), a->capacity, static_cast<uint32_t>(n), a->d_inv_qn,

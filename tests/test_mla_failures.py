@@ -75,13 +75,14 @@ int hipEventElapsedTime(float* ms, void* a, void* b) { *ms = 1.0f; return 0; }
 int hipFuncSetAttribute(const void* f, int a, int v) { return 0; }
 int hipGetLastError(void) { const int e = last; last = 0; return e; }
 const char* hipGetErrorString(int e) { return "stand-in failure"; }
-static struct { const void* host; const char* name; } kernels[4096];
+static struct { const void* host; const char* name; void* object; } kernels[4096];
 static int n_kernels;
-void** __hipRegisterFatBinary(const void* d) { static void* m[1]; return m; }
+void** __hipRegisterFatBinary(const void* d) { return malloc(sizeof(void*)); }
 void __hipUnregisterFatBinary(void** m) {}
 void __hipRegisterFunction(void** m, const void* host, char* dev, const char* name, unsigned t,
                            void* a, void* b, void* c, void* d, int* e) {
   kernels[n_kernels].host = host;
+  kernels[n_kernels].object = m;
   kernels[n_kernels++].name = strdup(name);
 }
 void __hipRegisterVar(void** m, void* v, char* h, char* d, int e, size_t n, int c, int g) {}
@@ -93,6 +94,12 @@ int __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, void* s) {
 int __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, void** s) {
   *g = pushed.g; *b = pushed.b; *lds = pushed.lds; *s = pushed.s;
   return 0;
+}
+/* a number per code object: that of kernel i, its name at *name; -1 past the last */
+int64_t fake_kernel(int i, const char** name) {
+  if (i >= n_kernels) return -1;
+  *name = kernels[i].name;
+  return (int64_t)kernels[i].object;
 }
 static float* norms;
 static uint64_t* ids;
@@ -315,4 +322,23 @@ with MlaNodeBank(np.ones((20_000, 64), np.float32)) as bank:
     except RuntimeError as e:  # the merge kernel does not run here
         assert {nq} > 1 and "completion flags" in str(e)
     assert hip.fake_pins() - before == 3
+""")
+
+
+# A bank's first route loads the code object its kernels are in: the screens'
+# probe forms, which only tests reach, are not in that one
+def test_probe_forms_have_a_code_object_of_their_own(runtime):
+    run(runtime, r"""
+hip.fake_kernel.restype = ctypes.c_int64
+import graftrepository_amd
+graftrepository_amd.load()
+name, kernels = ctypes.c_char_p(), []
+while (o := hip.fake_kernel(len(kernels), ctypes.byref(name))) != -1:
+    kernels.append((name.value, o))
+def objects(form, *words):
+    return {o for n, o in kernels if form in n and any(w in n for w in words)}
+screens = (b"mla_batch_ring_kernel", b"mla_batch_stream_kernel")
+probe, routes = objects(b"Lb1E", *screens), objects(b"Lb0E", *screens)
+assert len(probe) == len(routes) == 1
+assert routes == objects(b"", b"mla_route_kernel") and probe.isdisjoint(routes)
 """)
