@@ -429,6 +429,7 @@ struct MlaDeviceArena {
   // start of each batched pass's screen and merge.  ticks_per_ms: the
   // clock's rate (0: stream events).
   grm::MappedBuf marks;
+  size_t marks_n = 0;           // flags it has room for
   grm::MappedBuf done_flags;    // these three lie in marks
   grm::MappedBuf stamps;
   grm::MappedBuf screen_ticks;
@@ -988,17 +989,18 @@ bool reserve_batch(MlaDeviceArena* a, const BatchPlan& p, bool ring) {
 
 // Completion flags a route may wait on (one per query and route block).
 constexpr size_t kMaxDoneFlags = 8192;
-// Batched passes of a route that waits on flags, the shortest being 32
-// queries, and of its warm-up.
-constexpr size_t kMaxTickPasses = kMaxDoneFlags / 32 + 1;
 
-// Flags, stamps and ticks in one pinned allocation: one costs 20 to 30 us,
-// and the first routes on a bank pay for each.
-int reserve_marks(MlaDeviceArena* a) {
-  if (a->marks.host) return 0;
-  const size_t flags = kMaxDoneFlags * sizeof(unsigned);
-  const size_t stamps = grm::stamps_bytes(kMaxDoneFlags);
-  const size_t ticks = kMaxTickPasses * 2 * sizeof(unsigned long long);
+// Room for n flags, their stamps, and ticks of as many queries' batched
+// passes (32 queries at least), in one pinned allocation: the first routes
+// on a bank pay for each, and for each page.
+int reserve_marks(MlaDeviceArena* a, size_t n) {
+  if (n <= a->marks_n) return 0;
+  size_t room = 512;
+  while (room < n) room *= 2;
+  const size_t flags = room * sizeof(unsigned);
+  const size_t stamps = grm::stamps_bytes(room);
+  const size_t ticks = (room / 32 + 1) * 2 * sizeof(unsigned long long);
+  a->marks_n = 0;
   GRM_CHECK_RC(grm::reserve_mapped_bytes(&a->marks, flags + stamps + ticks));
   memset(a->marks.host, 0, a->marks.bytes);
   auto part = [&](size_t at, size_t bytes) {
@@ -1008,6 +1010,7 @@ int reserve_marks(MlaDeviceArena* a) {
   a->done_flags = part(0, flags);
   a->stamps = part(flags, stamps);
   a->screen_ticks = part(flags + stamps, ticks);
+  a->marks_n = room;
   return 0;
 }
 
@@ -1062,8 +1065,8 @@ int route_impl(MlaDeviceArena* a, const void* queries, int q_dtype,
     const int timed_passes = (timed + bp.qp_max - 1) / bp.qp_max;
     unsigned* d_done = nullptr;
     if (flags) {
-      GRM_CHECK_RC(reserve_marks(a));
-      GRM_CHECK_RC(grm::begin_flags(&a->done_flags, kMaxDoneFlags, &a->route_seq));
+      GRM_CHECK_RC(reserve_marks(a, n_q));
+      GRM_CHECK_RC(grm::begin_flags(&a->done_flags, n_q, &a->route_seq));
       d_done = static_cast<unsigned*>(a->done_flags.dev);
     } else {
       while (a->screen_ev.size() < 2 * static_cast<size_t>(timed_passes)) {
@@ -1160,8 +1163,8 @@ int route_impl(MlaDeviceArena* a, const void* queries, int q_dtype,
     const bool flags = flaggable && (!elapsed_ms || clocked);
     unsigned* d_done = nullptr;
     if (flags) {
-      GRM_CHECK_RC(reserve_marks(a));
-      GRM_CHECK_RC(grm::begin_flags(&a->done_flags, kMaxDoneFlags, &a->route_seq));
+      GRM_CHECK_RC(reserve_marks(a, n_flags));
+      GRM_CHECK_RC(grm::begin_flags(&a->done_flags, n_flags, &a->route_seq));
       d_done = static_cast<unsigned*>(a->done_flags.dev);
     }
     // Uncertified batched queries add their time to the timed segment.

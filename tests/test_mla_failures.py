@@ -325,6 +325,29 @@ with MlaNodeBank(np.ones((20_000, 64), np.float32)) as bank:
 """)
 
 
+# ... sized for the call, and for a larger one when that comes; without
+# memory for it the call is refused and the next one is as before
+def test_marks_grow_with_the_calls(runtime):
+    run(runtime, r"""
+import os
+os.environ["GRM_HIP_MLA_BATCH_MIN"] = "1000"
+with MlaNodeBank(np.ones((20_000, 64), np.float32)) as bank:
+    hip.fake_ticks(*(ctypes.c_uint64(2000),) * 4)
+    q = np.ones((40, 64), np.float32)
+    before = hip.fake_pinned()
+    bank.route(q[:1], 3)
+    assert hip.fake_pinned() - before < 32_768
+    for nq in (16, 1, 40):  # 157 blocks a query
+        assert abs(bank.route(q[:nq], 3).device_ms - 0.01) < 1e-6
+with MlaNodeBank(np.ones((20_000, 64), np.float32)) as bank:
+    bank.route(q[:1], 3)
+    fail("hipHostMalloc", 3)  # after the query's and the results'
+    refused(bank.route, q, 3)
+    bank.route(q[:1], 3)
+    bank.route(q, 3)
+""")
+
+
 # A bank's first route loads the code object its kernels are in: the screens'
 # probe forms, which only tests reach, are not in that one
 def test_probe_forms_have_a_code_object_of_their_own(runtime):
