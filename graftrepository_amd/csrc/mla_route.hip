@@ -1210,15 +1210,15 @@ int route_impl(MlaDeviceArena* a, const void* queries, int q_dtype,
   return 0;
 }
 
-// The next update's stage, of at least `bytes`, once the kernels of the
-// update before the last have read it.
+// The next update's stage, of at least `bytes` (0: its event alone), once
+// the kernels of the update before the last have read it.
 int next_stage(MlaDeviceArena* a, size_t bytes, MutStage** out) {
   MutStage& m = a->mut[a->mut_last ^ 1];
   if (m.pending) {
     GRM_HIP_CHECK(hipEventSynchronize(m.ev));
     m.pending = false;
   }
-  GRM_CHECK_RC(grm::reserve_mapped_bytes(&m.buf, bytes));
+  if (bytes > 0) GRM_CHECK_RC(grm::reserve_mapped_bytes(&m.buf, bytes));
   *out = &m;
   return 0;
 }
@@ -1861,15 +1861,13 @@ extern "C" int grm_mla_hip_append(MlaDeviceArena* a, const void* rows_host,
     MlaDeviceArena* a;
     const uint64_t* ids;
     uint64_t n = 0;            // ids in the table
-    MutStage* stage = nullptr;
     const uint64_t* slots = nullptr;  // the slots taken, in order (in the stage)
     uint64_t taken = 0;
-    uint64_t high_water = 0;   // before the first was
+    const uint64_t* d_slots = nullptr;  // ... for the device, from when rows may be placed
+    uint64_t high_water = 0;   // before the first was taken
     ~Entered() {
-      if (taken > 0) {
-        (void)launch_evict(a, static_cast<const uint64_t*>(stage->buf.dev), taken);
-        (void)hipStreamSynchronize(a->side);  // the stage is read no more
-      }
+      if (d_slots) (void)launch_evict(a, d_slots, taken);
+      if (taken > 0) (void)hipStreamSynchronize(a->side);  // the stage is read no more
       for (uint64_t i = 0; i < taken; ++i) {
         a->slot_id[slots[i]] = kNoId;
         if (slots[i] < high_water) a->free_slots.insert(slots[i]);
@@ -1892,18 +1890,24 @@ extern "C" int grm_mla_hip_append(MlaDeviceArena* a, const void* rows_host,
   const size_t row_bytes = static_cast<size_t>(a->dim) * elem_size(a->dtype);
   const size_t bytes = count * (2 * sizeof(uint64_t) + row_bytes);
   const bool direct = bytes <= kDirectAppendBytes;
+  // small updates take the two stages in turn; large ones share the bank's
+  // one (and its device copy), once the updates before have read theirs, so
+  // that a bank holds one pinned copy of its largest append
   MutStage* stage = nullptr;
-  GRM_CHECK_RC(next_stage(a, bytes, &stage));
-  if (!direct) {
-    // the device copy is shared by every large append: its last reader is
-    // on the same stream; growing it waits for that
-    if (bytes > a->d_stage_bytes) GRM_CHECK_RC(wait_mutations(a));
-    GRM_CHECK_RC(reserve_device(reinterpret_cast<unsigned char**>(&a->d_stage), &a->d_stage_bytes, bytes));
+  void* h = nullptr;
+  void* d = nullptr;
+  GRM_CHECK_RC(next_stage(a, direct ? bytes : 0, &stage));
+  if (direct) {
+    h = stage->buf.host;
+    d = stage->buf.dev;
+  } else {
+    GRM_CHECK_RC(stage_upload(a, bytes, &h, &d));
   }
-  uint64_t* h_slots = static_cast<uint64_t*>(static_cast<void*>(stage->buf.host));
+  uint64_t* h_slots = static_cast<uint64_t*>(h);
   uint64_t* h_ids = h_slots + count;
   unsigned char* h_rows = reinterpret_cast<unsigned char*>(h_ids + count);
-  entered.stage = stage;
+  const uint64_t* d_slots = static_cast<const uint64_t*>(d);
+  const unsigned char* d_rows = reinterpret_cast<const unsigned char*>(d_slots + 2 * count);
   entered.slots = h_slots;
   entered.high_water = a->high_water;
   for (uint64_t i = 0; i < count; ++i) {
@@ -1926,23 +1930,22 @@ extern "C" int grm_mla_hip_append(MlaDeviceArena* a, const void* rows_host,
     const uint64_t part = std::max<uint64_t>(grm::mla::kPlaceRows,
                                              kAppendPartBytes / row_bytes / grm::mla::kPlaceRows *
                                                  grm::mla::kPlaceRows);
-    const uint64_t* s_slots = static_cast<const uint64_t*>(static_cast<const void*>(stage->buf.dev));
-    const unsigned char* s_rows = reinterpret_cast<const unsigned char*>(s_slots + 2 * count);
+    entered.d_slots = d_slots;
     for (uint64_t r0 = 0; r0 < count; r0 += part) {
       const uint64_t n = std::min<uint64_t>(part, count - r0);
       memcpy(h_rows + r0 * row_bytes, static_cast<const unsigned char*>(rows_host) + r0 * row_bytes,
              n * row_bytes);
-      GRM_CHECK_RC(launch_place(a, s_rows + r0 * row_bytes, n, s_slots + r0, s_slots + count + r0, 0, a->side));
+      GRM_CHECK_RC(launch_place(a, d_rows + r0 * row_bytes, n, d_slots + r0, d_slots + count + r0, 0, a->side));
     }
   } else {
     memcpy(h_rows, rows_host, count * row_bytes);
-    GRM_HIP_CHECK(hipMemcpyAsync(a->d_stage, stage->buf.host, bytes, hipMemcpyHostToDevice, a->side));
-    uint64_t* d_slots = static_cast<uint64_t*>(a->d_stage);
-    uint64_t* d_ids = d_slots + count;
-    GRM_CHECK_RC(launch_place(a, d_ids + count, count, d_slots, d_ids, 0, a->side));
+    GRM_HIP_CHECK(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, a->side));
+    entered.d_slots = d_slots;
+    GRM_CHECK_RC(launch_place(a, d_rows, count, d_slots, d_slots + count, 0, a->side));
   }
   GRM_CHECK_RC(end_update(a, stage));
   entered.n = entered.taken = 0;
+  entered.d_slots = nullptr;
   a->live += count;
   a->epoch += 1;
   if (out_epoch) *out_epoch = a->epoch;

@@ -365,3 +365,24 @@ probe, routes = objects(b"Lb1E", *screens), objects(b"Lb0E", *screens)
 assert len(probe) == len(routes) == 1
 assert routes == objects(b"", b"mla_route_kernel") and probe.isdisjoint(routes)
 """)
+
+
+# large appends share one pinned stage and its device copy
+def test_memory_held_after_large_appends(runtime):
+    run(runtime, r"""
+rows = np.ones((9_000, 288), np.float32)
+ids = np.arange(9_000, dtype=np.uint64) + 1000
+size = 9_000 * (288 * 4 + 16)
+with MlaNodeBank(np.ones((100, 288), np.float32), capacity=CAP) as bank:
+    bank.append(rows[:10], ids[:10] + 20_000)  # the small updates' stages
+    bank.evict(ids[:10] + 20_000)
+    pinned, device = hip.fake_pinned(), hip.fake_device()
+    for _ in range(2):
+        bank.append(rows, ids)
+        bank.append(rows, ids + 50_000)
+        bank.evict(ids)
+        bank.evict(ids + 50_000)
+    assert hip.fake_pinned() - pinned <= size + 2 * 9_000 * 8
+    assert hip.fake_device() - device <= size
+    assert device_ids() == list(range(100))
+""")
