@@ -111,7 +111,11 @@ __device__ __forceinline__ uint32_t bf16_bits_rne(float f) {
 //
 // What bounds it: HBM.  Per tile of 288 fp32 values a wavefront issues 18
 // steps of 24 conversions and 3 CT MFMAs -- 54 MFMAs of 32 cycles at CT = 1
-// against 36 KiB to stream, 15 % of the matrix cores' rate.
+// against 36 KiB to stream, 15 % of the matrix cores' rate.  On small banks
+// (1.5 tiles a wavefront at 100k x 280 fp32, 27.6 us; 2.3 at 150k x 200
+// bf16, 22.2 us) the trips before the first tile and the last reload of the
+// ring, which is never folded, weigh as much: 1.26 and 1.36 x the bank's
+// bytes come from HBM.
 //
 // kProbe (tests of the screen bound only): every coded u goes to
 // planes[q*cap + slot] instead of the lists, and nothing else is written.
@@ -761,7 +765,8 @@ __device__ inline float wave_sort_desc(float v) {
 // while the last wavefront sums the law's norm; then a lane per row runs
 // the fp64 chain from LDS.  With the norm formed first and a lane loading
 // its row itself, 36 chunks at a time, the kernel took 17.2 us for 32 queries
-// x 100k x 280 fp32 and 25.6 for 256 x 1M x 288 bf16; it takes 14.0 and 21.3.
+// x 100k x 280 fp32 and 25.6 for 256 x 1M x 288 bf16; it takes 14.1 and 20.5
+// to 22.9.
 // Writes out[qi*k ..) (host mapped): the law's top-k where certified, else
 // k entries without a node (kNoId: route qi again on the exact path).  With
 // `done` the entries carry the route's tag and done[qi] takes its number

@@ -20,14 +20,16 @@
 //
 // Top-k is fused: each wave keeps a distributed top-k list (grm_common.hpp),
 // blocks merge their waves' lists in LDS and write their k best entries to
-// mapped host memory, where the host merges the per-block lists after the
-// kernel's completion event -- the score vector never leaves registers.
+// mapped host memory, where the host merges the per-block lists once every
+// block has stored its completion flag -- the score vector never leaves
+// registers.
 //
-// Batched queries take the matrix-core path (mla_batch.hpp): an MFMA screen
-// of 32 slots x up to 256 queries per wave keeps a per-lane shortlist, a
-// merge kernel certifies each query's top-k against a proven
-// bound on the screen's rounding error and rescores the shortlist with the
-// exact law; queries without a certificate are routed again here.
+// Batched queries take the matrix-core path (mla_batch.hpp, launched from
+// mla_screen.hpp): an MFMA screen of every 32-slot tile against up to 256
+// queries keeps a per-lane shortlist, a merge kernel certifies each query's
+// top-k against a proven bound on the screen's rounding error and rescores
+// the shortlist with the exact law; queries without a certificate are routed
+// again here.
 #include "grm_common.hpp"
 #include "mla_screen.hpp"
 #include "mla_values.hpp"
@@ -131,10 +133,11 @@ __device__ inline void stage_query(double* qd, const void* __restrict__ query,
 //    bound by HBM (1M x 288 fp32: 170 us = 6.8 TB/s).
 //  * kMaxNW = 8, B = 12..18 (deep): banks of at most 8 tiles per CU, a wave
 //    per tile on every CU.  Bound by latency: one round trip to memory and
-//    the fp64 chain of one row.  10k x 288 fp32 on the device: 8.3 us,
-//    against 24.6 us for 16-wave blocks on 10 CUs; with two, four or eight
-//    waves per block at that size 9.9, 11.4 and 15.5 us.  100k x 288: 20.9
-//    against 31.6 us.
+//    the fp64 chain of one row.  10k x 288 fp32 on the device's clock
+//    (RouteStamps): 7.6 to 8.3 us, against 24.6 us for 16-wave blocks on 10
+//    CUs; with two, four or eight waves per block at that size 9.9, 11.4
+//    and 15.5 us.  100k x 288: 20.0 to 20.9 against 31.6 us.  (A kernel
+//    trace, which holds the dispatch too, reads 12.3 and 25.6 us.)
 template <int DT, int B, int kMaxNW>
 __global__ __launch_bounds__(kMaxNW * kWave) void mla_route_kernel(
     const u32x4* __restrict__ tiles, const float* __restrict__ norms,
@@ -238,7 +241,8 @@ __global__ __launch_bounds__(kMaxNW * kWave) void mla_route_kernel(
 // chains from there while the others write the tiles.  (A thread per row,
 // loading value by value, took a trip to memory per value: 68 us for 1000
 // rows of 288, where these blocks take 8 to 15 us per 450 rows straight
-// from host memory.)  Rows longer than kPlaceCols go slice by slice, the chains'
+// from host memory.  A full batch of 65,536 rows from device memory takes
+// them 102 us against 86, beside the 2 ms its upload takes.)  Rows longer than kPlaceCols go slice by slice, the chains'
 // sums carried along; values past dim are zeros, which leave a sum as it is.
 constexpr int kPlaceRows = 16;
 constexpr int kPlaceCols = 320;  // values per slice
@@ -807,9 +811,9 @@ void write_cands(const Cand* c, int topk, uint64_t* out_ids, float* out_scores) 
   }
 }
 
-// Slot code width of the batched screens.  The code costs the screen bound 2^(ibits-23) relative, so banks
-// whose runs would need more than 16 bits route on the single-query path
-// instead.
+// Slot code width of the batched screens.  The code costs the screen bound
+// 2^(ibits-23) relative, so banks whose runs would need more than 16 bits
+// route on the single-query path instead.
 constexpr int kMaxSlotCodeBits = 16;
 
 // Whether a segment of `queries` has a pass for the ring screen.
@@ -1476,9 +1480,9 @@ int enqueue_latent_query(MlaDeviceArena* a, const void* d_latent, int dtype, uin
 // routing different banks on one GPU take turns and each gets its own
 // answer.  Queries run one after another on the bank's stream, so one
 // query's lists fit the array: up to kScratchCands entries (grid blocks x
-// topk; 1024 blocks x 16 at most with the default grid cap).  Each block
-// writes all k of its entries before the merge reads them, so nothing in
-// the array has to start at zero.
+// topk; the grid has a block per compute unit at most, 256 x 16 here).
+// Each block writes all k of its entries before the merge reads them, so
+// nothing in the array has to start at zero.
 constexpr int kScratchDevices = 64;
 
 std::mutex g_scratch_mu;

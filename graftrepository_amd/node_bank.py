@@ -201,7 +201,7 @@ class MlaNodeBank(_Bank):
 
     def probe_screen(self, queries, *, query_dtype: str = "bf16"):
         """Test entry: the batched route's screened score of every (query,
-        slot) pair of a small bf16 bank and each query's screen bound B.
+        slot) pair of a small bank and each query's screen bound B.
         Returns (values [Q, slots] f32, bounds [Q] f64, slot node ids)."""
         self._need_open()
         qd = _dtype_code(query_dtype)
